@@ -45,11 +45,69 @@ __device__ inline uint32_t f2ord(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-template <typename T>
-__device__ inline T wave_sum(T v) {
+/* Sums over the lanes of a wave in the order of a butterfly over lane distances
+ * 32, 16, 8, 4, 2, 1.  The exchanges run on the vector ALU: rows of 32 and 16 lanes
+ * change places with v_permlane32_swap / v_permlane16_swap, distances 8 and below
+ * stay inside a row of 16 (DPP).  Through ds_bpermute, each of the 6 steps of each of
+ * a pass's 29 sums was an LDS round trip that the next step waited for, at the end of
+ * every chunk: without them one 2 k-point scan takes 419 us instead of 509, the batch
+ * of 512 scans 5.09 ms instead of 5.73, a reference testcase of 2 k points 426 us
+ * instead of 472, all with the same bits. */
+__device__ inline double join_f64(uint32_t lo, uint32_t hi) {
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+/* lane i: rows of 32 (16) lanes: a's halves (row pairs) added in the lower (even)
+ * rows, b's in the upper (odd) ones */
+__device__ inline double fold32(double a, double b) {
+    const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+    return join_f64(lo[0], hi[0]) + join_f64(lo[1], hi[1]);
+}
+__device__ inline double fold16(double a, double b) {
+    const uint64_t x = (uint64_t)__double_as_longlong(a), y = (uint64_t)__double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(x >> 32), (uint32_t)(y >> 32), false, false);
+    return join_f64(lo[0], hi[0]) + join_f64(lo[1], hi[1]);
+}
+template <int CTRL>
+__device__ inline double add_dpp(double v) {
+    const uint64_t x = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)x, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(x >> 32), CTRL, 0xf, 0xf, true);
+    return v + join_f64(lo, hi);
+}
+/* the last four steps, within each row of 16 lanes: distance 8 and 4 as rotations of
+ * the row (by then lanes 8, then 4 apart hold the same value), 2 and 1 as quad
+ * permutations */
+__device__ inline double row_sum(double v) {
+    v = add_dpp<0x128>(v);  /* row_ror:8 */
+    v = add_dpp<0x124>(v);  /* row_ror:4 */
+    v = add_dpp<0x4e>(v);   /* quad_perm [2, 3, 0, 1] */
+    return add_dpp<0xb1>(v); /* quad_perm [1, 0, 3, 2] */
+}
+__device__ inline double wave_sum(double v) {
+    v = fold32(v, v);
+    return row_sum(fold16(v, v));
+}
+
+/* The wave sums of N <= 32 values per lane into out[0..N): the first two steps fold
+ * two values into one register each, so that eight registers remain, register j of
+ * row r holding value 8 r + j. */
+template <int N>
+__device__ inline void wave_sums(const double* v, double* out) {
+    static_assert(N <= 32, "one register per value of a quarter wave");
+    double q[8];
 #pragma unroll
-    for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
+    for (int j = 0; j < 8; j++) {
+        const auto val = [&](int k) { return k < N ? v[k] : 0.0; };
+        q[j] = row_sum(fold16(fold32(val(j), val(j + 16)), fold32(val(j + 8), val(j + 24))));
+    }
+    const int lane = threadIdx.x % WAVE, j = lane % 16, k = 8 * (lane / 16) + j;
+    double s = q[0];
+#pragma unroll
+    for (int i = 1; i < 8; i++) s = j == i ? q[i] : s;
+    if (j < 8 && k < N) out[k] = s;
 }
 
 static inline int grid_for(int64_t n, int block) { return (int)((n + block - 1) / block); }
@@ -1565,12 +1623,8 @@ __device__ inline int chunk_accumulate(const NdtGridDev& g, const float4* __rest
 template <int BLOCK>
 __device__ inline void block_reduce_acc(double* vals /* NRED per thread, registers */, double (*lds)[NRED],
                                         double* out) {
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-#pragma unroll
-    for (int k = 0; k < NRED; k++) {
-        double v = wave_sum(vals[k]);
-        if (lane == 0) lds[wave][k] = v;
-    }
+    const int wave = threadIdx.x / WAVE;
+    wave_sums<NRED>(vals, lds[wave]);
     __syncthreads();
     if (threadIdx.x < NRED) {
         double s = 0.0;
@@ -2773,11 +2827,9 @@ __global__ __launch_bounds__(256) void k_deriv_compat(CompatGridDev g, const flo
             }
         }
     }
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    for (int k = 0; k < NRED_COMPAT; k++) {
-        double v = wave_sum(acc[k]);
-        if (lane == 0) lds[wave][k] = v;
-    }
+    const int wave = threadIdx.x / WAVE;
+    wave_sums<32>(acc, lds[wave]);
+    wave_sums<NRED_COMPAT - 32>(acc + 32, lds[wave] + 32);
     __syncthreads();
     if (threadIdx.x < NRED_COMPAT) {
         double s = 0.0;
