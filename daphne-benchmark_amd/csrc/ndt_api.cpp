@@ -413,70 +413,93 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         g->fdev.origin_cell[k] = g->origin_cell[k];
     }
     g->fdev.resolution = res;
-    /* compact the valid voxels */
-    DevBuf vrank, sc3;
-    BUF_TRY(vrank, sizeof(uint32_t) * (nvox + 1));
-    BUF_TRY(sc3, scan_scratch_bytes(nvox) + 512);
-    uint32_t* vtotal = (uint32_t*)((char*)sc3.p + ((scan_scratch_bytes(nvox) + 255) & ~(size_t)255));
-    LAUNCH_TRY(exclusive_scan_u32(g->all_valid.as<uint32_t>(), vrank.as<uint32_t>(), nvox, vtotal, sc3.p, c->stream));
-    uint32_t h_nvalid = 0;
-    HIP_TRY(hipMemcpyAsync(&h_nvalid, vtotal, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    const int64_t nv = h_nvalid;
     g->info.map_points = m;
     g->info.voxels = nvox;
-    g->info.valid_voxels = nv;
-    BUF_TRY(g->mean_c, sizeof(double) * 3 * (nv + 1));
-    BUF_TRY(g->icov_c, sizeof(double) * 6 * (nv + 1));
-    BUF_TRY(g->icov_f, sizeof(float4) * 2 * (nv + 1));
-    DevBuf vkey_c;
-    BUF_TRY(vkey_c, sizeof(uint64_t) * (nv + 1));
-    LAUNCH_TRY(launch_compact_voxels(g->all_valid.as<uint32_t>(), vrank.as<uint32_t>(), nvox, g->all_mean.as<double>(),
-                                     g->all_icov.as<double>(), g->all_key.as<uint64_t>(), g->mean_c.as<double>(),
-                                     g->icov_c.as<double>(), g->icov_f.as<float4>(), vkey_c.as<uint64_t>(), c->stream));
-    /* dilation: candidate lists of every query cell */
-    const int64_t ne = 27 * nv;
-    int64_t nq = 0;
-    if (ne > 0) {
-        BUF_TRY(keys, sizeof(uint64_t) * ne);
-        BUF_TRY(vals, sizeof(uint32_t) * ne);
-        BUF_TRY(keys_t, sizeof(uint64_t) * ne);
-        BUF_TRY(vals_t, sizeof(uint32_t) * ne);
-        BUF_TRY(scratch, radix_sort_scratch_bytes(ne));
-        LAUNCH_TRY(launch_dilate_emit(vkey_c.as<uint64_t>(), nv, g->bits, keys.as<uint64_t>(), vals.as<uint32_t>(), c->stream));
-        LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(),
-                                    ne, B + 5, scratch.p, c->stream));
-        e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, flags, ranks, starts, sc2, &nq);
-        if (e) return e;
-    }
-    int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nq, 1)));
-    int64_t cap = 1ll << log2cap;
-    BUF_TRY(g->slots, sizeof(HashSlot) * cap);
-    LAUNCH_TRY(launch_hash_clear(g->slots.as<HashSlot>(), cap, c->stream));
-    BUF_TRY(g->cand_head, sizeof(float4) * (ne + 1));
-    BUF_TRY(g->cand_s32, 2 * sizeof(float4) * (ne + 1));
-    BUF_TRY(g->vs64, VS64_STRIDE * sizeof(double2) * (nv + 1));
-    LAUNCH_TRY(launch_voxel_s64(g->mean_c.as<double>(), g->icov_c.as<double>(), nv, g->vs64.as<double2>(), c->stream));
-    /* dense query-cell index when the map's cell box is at most 2^28 cells (2 GiB);
-     * the environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
+    /* dense query-cell index when the map's cell box is at most 2^28 cells; the
+     * environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
      * index, so that tests run that path on maps of every size */
     const double box = (double)g->dims[0] * (double)g->dims[1] * (double)g->dims[2];
     const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
     const bool dense = box <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
+    int64_t nv = 0, ne = 0, nq = 0;
+    int32_t tiles[2] = {0, 0};
     if (dense) {
-        const size_t cells = (size_t)g->dims[0] * (size_t)g->dims[1] * (size_t)g->dims[2];
-        BUF_TRY(g->dense, sizeof(uint2) * cells);
-        HIP_TRY(hipMemsetAsync(g->dense.p, 0, sizeof(uint2) * cells, c->stream));
-        if (nq > 0)
-            LAUNCH_TRY(launch_dense_fill(keys.as<uint64_t>(), starts.as<uint32_t>(), nq, ne, g->bits, g->dims,
-                                         g->dense.as<uint2>(), c->stream));
+        tiles[0] = (g->dims[0] + 3) / 4;
+        tiles[1] = (g->dims[1] + 3) / 4;
+        const int64_t ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
+        BUF_TRY(g->dense, sizeof(uint32_t) * (size_t)(ncells + 1));
+        BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)ncells);
+        BUF_TRY(c->bk_vid, sizeof(uint32_t) * (size_t)ncells);
+        BUF_TRY(scratch, cells_scratch_bytes(ncells));
+        uint64_t* totals = nullptr;
+        LAUNCH_TRY(launch_cells_index(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), nvox, g->bits, tiles, ncells,
+                                      c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_vid.as<uint32_t>(),
+                                      scratch.p, &totals, c->stream));
+        HIP_TRY(hipMemcpyAsync(c->hsmall, totals, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        const uint64_t* h = (const uint64_t*)c->hsmall;
+        nv = (int64_t)(h[0] >> 32);
+        ne = 27 * nv;
+        nq = (int64_t)h[1];
+        if (ne > 0xfffffffell) return fail(NDT_ERR_NOMEM, "more candidates than the index numbers");
     }
-    if (nq > 0) {
-        LAUNCH_TRY(launch_hash_insert(keys.as<uint64_t>(), starts.as<uint32_t>(), nq, ne, 5, g->slots.as<HashSlot>(),
-                                      log2cap, c->stream));
-        LAUNCH_TRY(launch_cand_fill(keys.as<uint64_t>(), vals.as<uint32_t>(), ne, g->mean_c.as<double>(),
-                                    g->icov_c.as<double>(), g->bits, g->origin_cell, (double)g->params.resolution,
-                                    g->cand_head.as<float4>(), g->cand_s32.as<float4>(), c->stream));
+    DevBuf vkey_c;
+    if (!dense) {
+        /* compact the valid voxels */
+        DevBuf vrank, sc3;
+        BUF_TRY(vrank, sizeof(uint32_t) * (nvox + 1));
+        BUF_TRY(sc3, scan_scratch_bytes(nvox) + 512);
+        uint32_t* vtotal = (uint32_t*)((char*)sc3.p + ((scan_scratch_bytes(nvox) + 255) & ~(size_t)255));
+        LAUNCH_TRY(exclusive_scan_u32(g->all_valid.as<uint32_t>(), vrank.as<uint32_t>(), nvox, vtotal, sc3.p, c->stream));
+        uint32_t h_nvalid = 0;
+        HIP_TRY(hipMemcpyAsync(&h_nvalid, vtotal, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        nv = h_nvalid;
+        BUF_TRY(g->mean_c, sizeof(double) * 3 * (nv + 1));
+        BUF_TRY(g->icov_c, sizeof(double) * 6 * (nv + 1));
+        BUF_TRY(vkey_c, sizeof(uint64_t) * (nv + 1));
+        LAUNCH_TRY(launch_compact_voxels(g->all_valid.as<uint32_t>(), vrank.as<uint32_t>(), nvox, g->all_mean.as<double>(),
+                                         g->all_icov.as<double>(), g->all_key.as<uint64_t>(), g->mean_c.as<double>(),
+                                         g->icov_c.as<double>(), vkey_c.as<uint64_t>(), c->stream));
+        /* dilation: candidate lists of every query cell */
+        ne = 27 * nv;
+        if (ne > 0) {
+            BUF_TRY(keys, sizeof(uint64_t) * ne);
+            BUF_TRY(vals, sizeof(uint32_t) * ne);
+            BUF_TRY(keys_t, sizeof(uint64_t) * ne);
+            BUF_TRY(vals_t, sizeof(uint32_t) * ne);
+            BUF_TRY(scratch, radix_sort_scratch_bytes(ne));
+            LAUNCH_TRY(launch_dilate_emit(vkey_c.as<uint64_t>(), nv, g->bits, keys.as<uint64_t>(), vals.as<uint32_t>(),
+                                          c->stream));
+            LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(),
+                                        vals_t.as<uint32_t>(), ne, B + 5, scratch.p, c->stream));
+            e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, flags, ranks, starts, sc2, &nq);
+            if (e) return e;
+        }
+    }
+    g->info.valid_voxels = nv;
+    const int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nq, 1)));
+    const int64_t cap = 1ll << log2cap;
+    BUF_TRY(g->cand_head, sizeof(float4) * (ne + 1));
+    BUF_TRY(g->cand_s32, 2 * sizeof(float4) * (ne + 1));
+    BUF_TRY(g->vs64, VS64_STRIDE * sizeof(double2) * (nv + 1));
+    if (dense) {
+        LAUNCH_TRY(launch_cells_fill(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), g->all_mean.as<double>(),
+                                     g->all_icov.as<double>(), nvox, g->bits, g->origin_cell, res, tiles,
+                                     c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_vid.as<uint32_t>(),
+                                     g->cand_head.as<float4>(), g->cand_s32.as<float4>(), g->vs64.as<double2>(),
+                                     c->stream));
+    } else {
+        BUF_TRY(g->slots, sizeof(HashSlot) * cap);
+        LAUNCH_TRY(launch_hash_clear(g->slots.as<HashSlot>(), cap, c->stream));
+        LAUNCH_TRY(launch_voxel_s64(g->mean_c.as<double>(), g->icov_c.as<double>(), nv, g->vs64.as<double2>(), c->stream));
+        if (nq > 0) {
+            LAUNCH_TRY(launch_hash_insert(keys.as<uint64_t>(), starts.as<uint32_t>(), nq, ne, 5, g->slots.as<HashSlot>(),
+                                          log2cap, c->stream));
+            LAUNCH_TRY(launch_cand_fill(keys.as<uint64_t>(), vals.as<uint32_t>(), ne, g->mean_c.as<double>(),
+                                        g->icov_c.as<double>(), g->bits, g->origin_cell, (double)g->params.resolution,
+                                        g->cand_head.as<float4>(), g->cand_s32.as<float4>(), c->stream));
+        }
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
     g->info.query_cells = nq;
@@ -484,8 +507,9 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     g->info.hash_capacity = cap;
     g->info.dense_cells = dense ? (int64_t)box : 0;
     NdtGridDev& d = g->dev;
-    d.dense = dense ? g->dense.as<uint2>() : nullptr;
+    d.dense = dense ? g->dense.as<uint32_t>() : nullptr;
     for (int k = 0; k < 3; k++) d.dims[k] = g->dims[k];
+    for (int k = 0; k < 2; k++) d.tiles[k] = tiles[k];
     d.slots = g->slots.as<HashSlot>();
     d.head = g->cand_head.as<float4>();
     d.s32 = g->cand_s32.as<float4>();

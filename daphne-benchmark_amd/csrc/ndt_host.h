@@ -157,7 +157,8 @@ struct ndt_ctx {
     /* grid-build temporaries, and the compat callback's grid and scan, kept for
      * reuse: freeing device memory synchronises the device, which would serialise
      * contexts that work concurrently (one per host thread) */
-    DevBuf bk_keys, bk_vals, bk_keys_t, bk_vals_t, bk_scratch, bk_flags, bk_ranks, bk_starts, bk_sc2, bk_mm;
+    DevBuf bk_keys, bk_vals, bk_keys_t, bk_vals_t, bk_scratch, bk_flags, bk_ranks, bk_starts, bk_sc2, bk_mm,
+        bk_mask, bk_vid;
     DevBuf compat_scan;
     ndt_grid* compat_grid = nullptr;
     /* pinned staging buffer for host-to-device uploads; pin_pending while a copy
@@ -183,7 +184,7 @@ struct ndt_grid {
     ndt_grid_info info;
     /* ndt */
     ndt::NdtGridDev dev;
-    DevBuf slots, dense, cand_head, cand_s32, vs64, icov_f, mean_c, icov_c;
+    DevBuf slots, dense, cand_head, cand_s32, vs64, mean_c, icov_c;
     int32_t dims[3] = {0, 0, 0};
     /* map points sorted by voxel + occupied-voxel hash (fitness score) */
     ndt::FitGridDev fdev;

@@ -239,9 +239,18 @@ NDT_HD uint64_t hash_slot(uint64_t key, int log2cap) {
 /* double2 entries per voxel in vs64 (80 bytes; padding records to 128 bytes, one
  * cache line each, made the alignment launch 1 % slower) */
 constexpr int VS64_STRIDE = 5;
+/* Cells of a dense index in order of tiles of 4 x 4 x 2 cells, tx x ty tiles per layer:
+ * the index of cell (c0, c1, c2) of the box (at most 2^28 cells, whole tiles below
+ * 2^31). */
+NDT_HD int32_t cell_index(int32_t c0, int32_t c1, int32_t c2, int32_t tx, int32_t ty) {
+    return ((((c2 >> 1) * ty + (c1 >> 2)) * tx + (c0 >> 2)) << 5) | ((c2 & 1) << 4) | ((c1 & 3) << 2) | (c0 & 3);
+}
+
 struct NdtGridDev {
-    const uint2* dense;      /* query cell -> (begin, count), dense over the map's cell box, or null */
+    const uint32_t* dense;   /* query cell (cell_index) -> begin of its candidate run, which ends
+                                where the next cell's begins; over the map's cell box, or null */
     int32_t dims[3];         /* cells per axis of the dense index */
+    int32_t tiles[2];        /* tiles per axis x, y of the dense index */
     const HashSlot* slots;   /* query cell -> candidate range (when dense is null) */
     const float4* head;      /* candidates: relative mean, voxel id */
     const float4* s32;       /* candidates: float32 statistics (2 per entry) */
@@ -456,7 +465,7 @@ int launch_voxel_stats_ndt(const float4* pts, const uint32_t* sorted_idx, const 
                            int32_t* count, uint32_t* valid, uint64_t* vkey, hipStream_t stream);
 int launch_compact_voxels(const uint32_t* valid, const uint32_t* rank, int64_t nvox, const double* mean,
                           const double* icov, const uint64_t* vkey, double* mean_out, double* icov_out,
-                          float4* icov_f, uint64_t* vkey_out, hipStream_t stream);
+                          uint64_t* vkey_out, hipStream_t stream);
 int launch_dilate_emit(const uint64_t* vkey, int64_t nvalid, const int* bits, uint64_t* keys, uint32_t* vals,
                        hipStream_t stream);
 int launch_hash_insert(const uint64_t* sorted_keys, const uint32_t* starts, int64_t nq, int64_t nentries,
@@ -472,8 +481,19 @@ int launch_voxel_stats_compat(const float4* pts, const uint32_t* sorted_idx, con
                               double* mean, double* icov, int32_t* count, uint64_t* vkey, hipStream_t stream);
 
 /* ndt alignment: init states from guesses, then the cooperative persistent kernel */
-int launch_dense_fill(const uint64_t* sorted_keys, const uint32_t* starts, int64_t nq, int64_t nentries,
-                      const int* bits, const int32_t* dims, uint2* dense, hipStream_t stream);
+/* dense query-cell index of the nvox voxels (those with valid[v] take part): run starts
+ * begin[0..ncells] and, where a cell holds a valid voxel, its number vid[cell]; mask,
+ * begin and vid hold ncells entries (begin one more).  *totals is device memory in
+ * scratch: candidates and, in the upper half, valid voxels; then query cells. */
+size_t cells_scratch_bytes(int64_t ncells);
+int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
+                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
+                       uint64_t** totals, hipStream_t stream);
+/* the candidate entries and float64 statistics behind that index */
+int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double* mean, const double* icov, int64_t nvox,
+                      const int* bits, const int64_t* origin_cell, double res, const int32_t* tiles, const uint32_t* mask,
+                      const uint32_t* begin, const uint32_t* vid, float4* head, float4* s32, double2* vs64,
+                      hipStream_t stream);
 int launch_gather_points(const float4* pts, const uint32_t* idx, int64_t n, float4* out, hipStream_t stream);
 int launch_fitness(FitGridDev fg, const float4* pts, const int64_t* offsets, const int32_t* counts, int32_t S,
                    const double* poses, double max_d2, int shells, int nblk, double* partials, hipStream_t stream);

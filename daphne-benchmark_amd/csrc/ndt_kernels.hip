@@ -633,8 +633,7 @@ int launch_voxel_stats_ndt(const float4* pts, const uint32_t* sorted_idx, const 
 __global__ void k_compact_voxels(const uint32_t* __restrict__ valid, const uint32_t* __restrict__ rank, int64_t nvox,
                                  const double* __restrict__ mean, const double* __restrict__ icov,
                                  const uint64_t* __restrict__ vkey, double* __restrict__ mean_out,
-                                 double* __restrict__ icov_out, float4* __restrict__ icov_f,
-                                 uint64_t* __restrict__ vkey_out) {
+                                 double* __restrict__ icov_out, uint64_t* __restrict__ vkey_out) {
     int64_t v = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (v >= nvox || !valid[v]) return;
     int64_t r = rank[v];
@@ -642,16 +641,14 @@ __global__ void k_compact_voxels(const uint32_t* __restrict__ valid, const uint3
     const double* C = icov + 9 * v;
     double u[6] = {C[0], C[1], C[2], C[4], C[5], C[8]};
     for (int k = 0; k < 6; k++) icov_out[6 * r + k] = u[k];
-    icov_f[2 * r] = make_float4((float)u[0], (float)u[1], (float)u[2], (float)u[3]);
-    icov_f[2 * r + 1] = make_float4((float)u[4], (float)u[5], 0.0f, 0.0f);
     vkey_out[r] = vkey[v];
 }
 
 int launch_compact_voxels(const uint32_t* valid, const uint32_t* rank, int64_t nvox, const double* mean,
-                          const double* icov, const uint64_t* vkey, double* mean_out, double* icov_out, float4* icov_f,
+                          const double* icov, const uint64_t* vkey, double* mean_out, double* icov_out,
                           uint64_t* vkey_out, hipStream_t stream) {
     hipLaunchKernelGGL(k_compact_voxels, dim3(grid_for(nvox, 256)), dim3(256), 0, stream, valid, rank, nvox, mean,
-                       icov, vkey, mean_out, icov_out, icov_f, vkey_out);
+                       icov, vkey, mean_out, icov_out, vkey_out);
     return (int)hipGetLastError();
 }
 
@@ -722,30 +719,6 @@ __global__ void k_hash_insert(const uint64_t* __restrict__ skeys, const uint32_t
         }
         h = (h + 1) & mask;
     }
-}
-
-/* Dense query-cell index: entry (c2 * D1 + c1) * D0 + c0 = (begin, count) of the
- * candidate run of query cell (c0, c1, c2); cells without candidates stay (0, 0). */
-__global__ void k_dense_fill(const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ starts, int64_t nq,
-                             int64_t nentries, Bits3 B, int32_t d0, int32_t d1, uint2* __restrict__ dense) {
-    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (q >= nq) return;
-    const uint32_t b = starts[q];
-    const uint32_t e = (q + 1 < nq) ? starts[q + 1] : (uint32_t)nentries;
-    const uint64_t key = skeys[b] >> 5;
-    const int64_t c0 = (int64_t)(key & ((1ull << B.b[0]) - 1));
-    const int64_t c1 = (int64_t)((key >> B.b[0]) & ((1ull << B.b[1]) - 1));
-    const int64_t c2 = (int64_t)(key >> (B.b[0] + B.b[1]));
-    dense[(c2 * d1 + c1) * d0 + c0] = make_uint2(b, e - b);
-}
-
-int launch_dense_fill(const uint64_t* sorted_keys, const uint32_t* starts, int64_t nq, int64_t nentries,
-                      const int* bits, const int32_t* dims, uint2* dense, hipStream_t stream) {
-    Bits3 B;
-    for (int k = 0; k < 3; k++) B.b[k] = bits[k];
-    hipLaunchKernelGGL(k_dense_fill, dim3(grid_for(nq, 256)), dim3(256), 0, stream, sorted_keys, starts, nq, nentries, B,
-                       dims[0], dims[1], dense);
-    return (int)hipGetLastError();
 }
 
 int launch_hash_insert(const uint64_t* sorted_keys, const uint32_t* starts, int64_t nq, int64_t nentries, int shift,
@@ -830,6 +803,223 @@ __global__ void k_voxel_s64(const double* __restrict__ mean, const double* __res
 int launch_voxel_s64(const double* mean, const double* icov, int64_t nvalid, double2* vs64, hipStream_t stream) {
     if (nvalid <= 0) return 0;
     hipLaunchKernelGGL(k_voxel_s64, dim3(grid_for(nvalid, 256)), dim3(256), 0, stream, mean, icov, nvalid, vs64);
+    return (int)hipGetLastError();
+}
+
+/* ------------------------------------------------------------------ dense query-cell index
+ * Built from the cells, without sorting the 27 entries per valid voxel: every valid
+ * voxel sets its probe's bit in the 27 cells that see it, one scan over the cells
+ * turns the bit counts into run starts and numbers the valid voxels, and every
+ * voxel then writes its 27 entries at the places its bits give.
+ *
+ * Sorting the entries (four radix passes and a scan over 27 entries per valid voxel)
+ * was latency and launches, 25 of them: without it a map and its first pass take 1.05 ms
+ * instead of 1.31 (100 k points) and 4.29 instead of 4.91 (1 M).  Boxes too large for
+ * a word per cell keep the sorted entries and their hash.
+ *
+ * Cells, and with them candidate runs and voxel numbers, are ordered in tiles of
+ * 4 x 4 x 2 cells (cell_index): a tile's 32 run starts are one 128-byte line, and what
+ * the align kernels gather for 64 neighbouring points lies together (137 M requests to
+ * L2 for the batch of 512 scans, 155 M with rows of cells; the same time). */
+
+__device__ inline void cell_of_key(uint64_t key, const Bits3& B, int32_t* c) {
+    c[0] = (int32_t)(key & ((1ull << B.b[0]) - 1));
+    c[1] = (int32_t)((key >> B.b[0]) & ((1ull << B.b[1]) - 1));
+    c[2] = (int32_t)(key >> (B.b[0] + B.b[1]));
+}
+
+/* thread (voxel, dz, dy): the three probes of a row.  Bit o of a cell's mask is probe
+ * o = 9 (dz + 1) + 3 (dy + 1) + (dx + 1): the cell at (dx, dy, dz) from it holds a
+ * valid voxel. */
+__global__ void k_cell_masks(const uint64_t* __restrict__ vkey, const uint32_t* __restrict__ valid, int64_t nvox, Bits3 B,
+                             int32_t tx, int32_t ty, uint32_t* __restrict__ mask) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t v = i / 9;
+    if (v >= nvox || !valid[v]) return;
+    const int row = (int)(i - 9 * v), dz = row / 3 - 1, dy = row % 3 - 1;
+    int32_t c[3];
+    cell_of_key(vkey[v], B, c);
+    for (int dx = -1; dx <= 1; dx++)
+        atomicOr(&mask[cell_index(c[0] - dx, c[1] - dy, c[2] - dz, tx, ty)], 1u << (3 * row + dx + 1));
+}
+
+/* What a cell adds to the scan: its candidates, and in the upper half 1 when it holds
+ * a valid voxel itself (probe 13). */
+__device__ inline uint64_t cell_sum(uint32_t mask) {
+    return (uint64_t)__popc(mask) | ((uint64_t)((mask >> 13) & 1u) << 32);
+}
+
+/* exclusive block scan of one 64-bit value per thread; returns the block total */
+__device__ inline uint64_t block_exclusive_scan64(uint64_t v, uint64_t* excl, uint64_t* lds_waves) {
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    uint64_t incl = v;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+        const uint64_t t = (uint64_t)__shfl_up((long long)incl, off, WAVE);
+        if (lane >= off) incl += t;
+    }
+    if (lane == WAVE - 1) lds_waves[wave] = incl;
+    __syncthreads();
+    uint64_t before = 0, total = 0;
+    for (int w = 0; w < (int)(blockDim.x / WAVE); w++) {
+        const uint64_t c = lds_waves[w];
+        if (w < wave) before += c;
+        total += c;
+    }
+    __syncthreads();
+    *excl = before + incl - v;
+    return total;
+}
+
+/* a thread's 16 cells, a workgroup's 4096: the masks end with whole tiles, and the
+ * cells past the last one count as empty */
+constexpr int CELL_ITEMS = 16;
+constexpr int CELL_TILE = 256 * CELL_ITEMS;
+__device__ inline void load_masks(const uint32_t* __restrict__ mask, int64_t ncells, int64_t base, uint32_t* m) {
+#pragma unroll
+    for (int k = 0; k < CELL_ITEMS; k += 4) {
+        const uint4 q = base + k < ncells ? *(const uint4*)(mask + base + k) : make_uint4(0u, 0u, 0u, 0u);
+        m[k] = q.x;
+        m[k + 1] = q.y;
+        m[k + 2] = q.z;
+        m[k + 3] = q.w;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_cells_reduce(const uint32_t* __restrict__ mask, int64_t ncells,
+                                                      uint64_t* __restrict__ bsum, uint64_t* __restrict__ totals) {
+    __shared__ uint64_t lw[256 / WAVE];
+    uint32_t m[CELL_ITEMS];
+    load_masks(mask, ncells, blockIdx.x * (int64_t)CELL_TILE + threadIdx.x * CELL_ITEMS, m);
+    uint64_t s = 0, used = 0, ex;
+#pragma unroll
+    for (int k = 0; k < CELL_ITEMS; k++) {
+        s += cell_sum(m[k]);
+        used += m[k] ? 1u : 0u;
+    }
+    const uint64_t total = block_exclusive_scan64(s, &ex, lw);
+    const uint64_t nq = block_exclusive_scan64(used, &ex, lw);
+    if (threadIdx.x == 0) {
+        bsum[blockIdx.x] = total;
+        if (nq) atomicAdd((unsigned long long*)&totals[1], (unsigned long long)nq);
+    }
+}
+
+/* totals[0] = candidates, and valid voxels in the upper half; totals[1] = query cells */
+__global__ __launch_bounds__(1024) void k_cells_top(uint64_t* __restrict__ bsum, int64_t nb, uint64_t* __restrict__ totals) {
+    __shared__ uint64_t lw[1024 / WAVE];
+    const int64_t per = (nb + blockDim.x - 1) / blockDim.x;
+    const int64_t b = threadIdx.x * per;
+    uint64_t s = 0, run;
+    for (int64_t i = b; i < b + per && i < nb; i++) s += bsum[i];
+    const uint64_t tot = block_exclusive_scan64(s, &run, lw);
+    for (int64_t i = b; i < b + per && i < nb; i++) {
+        const uint64_t v = bsum[i];
+        bsum[i] = run;
+        run += v;
+    }
+    if (threadIdx.x == 0) totals[0] = tot;
+}
+
+/* begin[cell] (begin[ncells] = all candidates), and the number of the valid voxel in
+ * each cell that holds one */
+__global__ __launch_bounds__(256) void k_cells_down(const uint32_t* __restrict__ mask, int64_t ncells,
+                                                    const uint64_t* __restrict__ bsum, uint32_t* __restrict__ begin,
+                                                    uint32_t* __restrict__ vid) {
+    __shared__ uint64_t lw[256 / WAVE];
+    uint32_t m[CELL_ITEMS];
+    const int64_t base = blockIdx.x * (int64_t)CELL_TILE + threadIdx.x * CELL_ITEMS;
+    load_masks(mask, ncells, base, m);
+    uint64_t s = 0, run;
+#pragma unroll
+    for (int k = 0; k < CELL_ITEMS; k++) s += cell_sum(m[k]);
+    block_exclusive_scan64(s, &run, lw);
+    run += bsum[blockIdx.x];
+#pragma unroll
+    for (int k = 0; k < CELL_ITEMS; k += 4) {
+        uint32_t at[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            at[j] = (uint32_t)run;
+            if ((m[k + j] >> 13) & 1u) vid[base + k + j] = (uint32_t)(run >> 32);
+            run += cell_sum(m[k + j]);
+        }
+        if (base + k < ncells) *(uint4*)(begin + base + k) = make_uint4(at[0], at[1], at[2], at[3]);
+        /* the masks end with a group of four cells */
+        if (base + k + 4 == ncells) begin[ncells] = (uint32_t)run;
+    }
+}
+
+/* thread (voxel, probe): the voxel's entry in the run of the query cell that sees it
+ * at this probe (mean relative to the cell's lower corner in float32, values in
+ * [-res, 2 res), kept to about 1e-7 m at any map extent, with the voxel's number; and
+ * the float32 inverse covariance); probe 13 also writes the float64 statistics. */
+__global__ void k_cells_fill(const uint64_t* __restrict__ vkey, const uint32_t* __restrict__ valid,
+                             const double* __restrict__ mean, const double* __restrict__ icov, int64_t nvox, Bits3 B,
+                             int64_t o0, int64_t o1, int64_t o2, double res, int32_t tx, int32_t ty,
+                             const uint32_t* __restrict__ mask, const uint32_t* __restrict__ begin,
+                             const uint32_t* __restrict__ vid, float4* __restrict__ head, float4* __restrict__ s32,
+                             double2* __restrict__ vs64) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t v = i / 27;
+    if (v >= nvox || !valid[v]) return;
+    const int o = (int)(i - 27 * v);
+    int32_t c[3];
+    cell_of_key(vkey[v], B, c);
+    const uint32_t id = vid[cell_index(c[0], c[1], c[2], tx, ty)];
+    const int32_t q0 = c[0] - (o % 3 - 1), q1 = c[1] - (o / 3 % 3 - 1), q2 = c[2] - (o / 9 - 1);
+    const int32_t qi = cell_index(q0, q1, q2, tx, ty);
+    const uint32_t at = begin[qi] + (uint32_t)__popc(mask[qi] & ((1u << o) - 1u));
+    const double m0 = mean[3 * v], m1 = mean[3 * v + 1], m2 = mean[3 * v + 2];
+    const double* C = icov + 9 * v;
+    const double c00 = C[0], c01 = C[1], c02 = C[2], c11 = C[4], c12 = C[5], c22 = C[8];
+    head[at] = make_float4((float)(m0 - (double)(q0 + o0) * res), (float)(m1 - (double)(q1 + o1) * res),
+                           (float)(m2 - (double)(q2 + o2) * res), __uint_as_float(id));
+    s32[2 * (int64_t)at] = make_float4((float)c00, (float)c01, (float)c02, (float)c11);
+    s32[2 * (int64_t)at + 1] = make_float4((float)c12, (float)c22, 0.0f, 0.0f);
+    if (o == 13) {
+        double2* w = vs64 + VS64_STRIDE * (int64_t)id;
+        w[0] = make_double2(m0, m1);
+        w[1] = make_double2(m2, c00);
+        w[2] = make_double2(c01, c02);
+        w[3] = make_double2(c11, c12);
+        w[4] = make_double2(c22, 0.0);
+    }
+}
+
+size_t cells_scratch_bytes(int64_t ncells) {
+    return sizeof(uint64_t) * (size_t)((ncells + CELL_TILE - 1) / CELL_TILE + 2);
+}
+
+int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
+                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
+                       uint64_t** totals, hipStream_t stream) {
+    Bits3 B;
+    for (int k = 0; k < 3; k++) B.b[k] = bits[k];
+    const int64_t nb = (ncells + CELL_TILE - 1) / CELL_TILE;
+    uint64_t* tot = (uint64_t*)scratch;
+    uint64_t* bsum = tot + 2;
+    hipError_t e = hipMemsetAsync(mask, 0, sizeof(uint32_t) * (size_t)ncells, stream);
+    if (e == hipSuccess) e = hipMemsetAsync(tot, 0, 2 * sizeof(uint64_t), stream);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(k_cell_masks, dim3(grid_for(9 * nvox, 256)), dim3(256), 0, stream, vkey, valid, nvox, B, tiles[0],
+                       tiles[1], mask);
+    hipLaunchKernelGGL(k_cells_reduce, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, tot);
+    hipLaunchKernelGGL(k_cells_top, dim3(1), dim3(1024), 0, stream, bsum, nb, tot);
+    hipLaunchKernelGGL(k_cells_down, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, begin, vid);
+    *totals = tot;
+    return (int)hipGetLastError();
+}
+
+int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double* mean, const double* icov, int64_t nvox,
+                      const int* bits, const int64_t* origin_cell, double res, const int32_t* tiles, const uint32_t* mask,
+                      const uint32_t* begin, const uint32_t* vid, float4* head, float4* s32, double2* vs64,
+                      hipStream_t stream) {
+    Bits3 B;
+    for (int k = 0; k < 3; k++) B.b[k] = bits[k];
+    hipLaunchKernelGGL(k_cells_fill, dim3(grid_for(27 * nvox, 256)), dim3(256), 0, stream, vkey, valid, mean, icov, nvox, B,
+                       origin_cell[0], origin_cell[1], origin_cell[2], res, tiles[0], tiles[1], mask, begin, vid, head,
+                       s32, vs64);
     return (int)hipGetLastError();
 }
 
@@ -1110,6 +1300,16 @@ __device__ inline double cell_quot(const NdtGridDev& g, const double x) {
     return g.res_pow2 ? x * g.inv_resolution_d : x / g.resolution_d;
 }
 
+/* (begin, count) of the candidate run of a query cell of the dense index: two
+ * neighbouring words, one 8-byte load. */
+__device__ inline uint2 cell_run(const NdtGridDev& g, int32_t c0, int32_t c1, int32_t c2) {
+    struct __attribute__((aligned(4))) Run {
+        uint32_t begin, end;
+    };
+    const Run r = *(const Run*)(g.dense + cell_index(c0, c1, c2, g.tiles[0], g.tiles[1]));
+    return make_uint2(r.begin, r.end - r.begin);
+}
+
 /* Transform, cell and index lookup; false when the point has no candidates. */
 __device__ inline bool point_lookup(const NdtGridDev& g, const float4 p, const double* R, const double* t,
                                     PointLook& L) {
@@ -1127,7 +1327,7 @@ __device__ inline bool point_lookup(const NdtGridDev& g, const float4 p, const d
     if (g.dense) {
         /* direct index: neighbouring points read neighbouring entries */
         if (c0 < 0 || c1 < 0 || c2 < 0 || c0 >= g.dims[0] || c1 >= g.dims[1] || c2 >= g.dims[2]) return false;
-        const uint2 e = g.dense[(c2 * g.dims[1] + c1) * g.dims[0] + c0];
+        const uint2 e = cell_run(g, (int32_t)c0, (int32_t)c1, (int32_t)c2);
         begin = e.x;
         count = e.y;
         if (!count) return false;
@@ -1178,7 +1378,7 @@ __device__ inline void lookup_issue(const NdtGridDev& g, const float4 p, const b
     const int i0 = ok ? (int)c0 : 0, i1 = ok ? (int)c1 : 0, i2 = ok ? (int)c2 : 0;
     /* the load is unconditional (entry 0 stands in for points without a cell), so
      * that its wait is counted exactly where the entry is used */
-    const uint2 v = g.dense[(i2 * g.dims[1] + i1) * g.dims[0] + i0];
+    const uint2 v = cell_run(g, i0, i1, i2);
     e = ok ? v : make_uint2(0u, 0u);
 }
 

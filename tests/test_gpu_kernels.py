@@ -1,4 +1,6 @@
 """Kernels at the sizes where their tiles, waves and remainders can go wrong."""
+import os
+
 import numpy as np
 import pytest
 
@@ -27,3 +29,43 @@ def test_pass_sums_of_part_filled_waves(A, orc, scene, n):
     assert abs(sg - so) <= 1e-10 * abs(so)
     assert np.abs(gg - go).max() <= 1e-10 * np.abs(go).max()
     assert np.abs(Hg - Ho).max() <= 1e-10 * np.abs(Ho).max()
+
+
+def _hashed(A, ctx, mp, prm):
+    os.environ["NDT_FORCE_HASHED_INDEX"] = "1"
+    try:
+        return A.Grid(ctx, mp, prm)
+    finally:
+        del os.environ["NDT_FORCE_HASHED_INDEX"]
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1), (2, 1, 1), (1, 2, 3), (3, 4, 5), (4, 4, 2), (5, 9, 1), (13, 1, 7), (33, 31, 6),
+                                 (64, 65, 4)])
+@pytest.mark.parametrize("res", [1.0, 0.7])
+def test_dense_index_matches_hashed(A, ctx, box, res):
+    """The dense index (cell masks, tiles of 4 x 4 x 2 cells) against the hashed one on
+    boxes of cells that do and do not fill their tiles, the first and last cells
+    included: the same voxels, query cells and candidates, and the same bits from a pass
+    over points in, between and outside the cells (the two differ in the lookup only)."""
+    rng = np.random.default_rng(sum(box))
+    cells = np.stack(np.meshgrid(*[np.arange(b) for b in box], indexing="ij"), -1).reshape(-1, 3)
+    keep = rng.random(len(cells)) < 0.6
+    keep[0] = keep[-1] = True
+    cells = cells[keep] - np.array([3, 5, 1])
+    pts = (cells[:, None, :] + rng.uniform(0.02, 0.98, (len(cells), 9, 3))).reshape(-1, 3) * res
+    pts = np.concatenate([pts, pts[::40] + 0.003])  # and a few voxels of more points
+    mp = np.c_[pts, np.ones(len(pts))].astype(np.float32)
+    prm = A.params(A.NDT_MODE_NDT, resolution=res)
+    dense, hashed = A.Grid(ctx, mp, prm), _hashed(A, ctx, mp, prm)
+    a, b = dense.info(), hashed.info()
+    assert a["dense_cells"] > 0 and b["dense_cells"] == 0
+    for k in ("voxels", "valid_voxels", "query_cells", "candidates", "hash_capacity"):
+        assert a[k] == b[k]
+    lo, hi = pts.min(0) - 2.5 * res, pts.max(0) + 2.5 * res
+    scan = np.c_[rng.uniform(lo, hi, (700, 3)), np.ones(700)].astype(np.float32)
+    p = np.array([0.03, -0.02, 0.01, 0.004, -0.003, 0.01])
+    for point in (A.NDT_POINT_FP64, A.NDT_POINT_FP32):
+        q = A.params(A.NDT_MODE_NDT, resolution=res, point_precision=point)
+        x, y = dense.derivatives(scan, p, prm=q), hashed.derivatives(scan, p, prm=q)
+        assert x[3] == y[3] and x[3] > 0
+        assert x[0] == y[0] and np.array_equal(x[1], y[1]) and np.array_equal(x[2], y[2])
