@@ -136,6 +136,8 @@ extern "C" int ndt_ctx_create(int32_t device, ndt_ctx** out) {
     if ((e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking)) != hipSuccess ||
         (e = hipEventCreate(&c->ev0)) != hipSuccess || (e = hipEventCreate(&c->ev1)) != hipSuccess ||
         (e = hipEventCreate(&c->ev2)) != hipSuccess ||
+        (e = hipEventCreateWithFlags(&c->ev_stage[0], hipEventDisableTiming)) != hipSuccess ||
+        (e = hipEventCreateWithFlags(&c->ev_stage[1], hipEventDisableTiming)) != hipSuccess ||
         (e = hipHostMalloc(&c->hsmall, HSMALL_BYTES, hipHostMallocDefault)) != hipSuccess) {
         delete c;
         return fail(NDT_ERR_HIP, std::string("stream/event creation: ") + hipGetErrorString(e));
@@ -156,6 +158,8 @@ void ndt::ctx_release(ndt_ctx* c) {
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->ev2) (void)hipEventDestroy(c->ev2);
+    for (hipEvent_t ev : c->ev_stage)
+        if (ev) (void)hipEventDestroy(ev);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->pin) (void)hipHostFree(c->pin);
     if (c->hsmall) (void)hipHostFree(c->hsmall);
@@ -275,25 +279,40 @@ static int pinned_reserve(ndt_ctx* c, size_t bytes) {
     return 0;
 }
 
+/* `bytes` of the staging buffer for an upload: behind the parts that copies in flight
+ * still read while there is room, otherwise its front, once they have completed. */
+static int pinned_stage(ndt_ctx* c, size_t bytes, char** p) {
+    if (!c->pin_pending) c->pin_off = 0;
+    const size_t room = (bytes + 255) & ~(size_t)255;
+    if (c->pin_off + room > c->pin_bytes) {
+        if (c->pin_pending) {
+            HIP_TRY(hipStreamSynchronize(c->stream));
+            c->pin_pending = false;
+        }
+        c->pin_off = 0;
+        const int e = pinned_reserve(c, room);
+        if (e) return e;
+    }
+    *p = (char*)c->pin + c->pin_off;
+    c->pin_off += room;
+    return 0;
+}
+
 /* Host-to-device copies (one or two) through the pinned staging buffer: a pageable
  * hipMemcpyAsync is staged by the runtime through buffers shared by every stream,
- * which serialises contexts that upload concurrently.  The staging buffer is
- * refilled only after the previous copies from it have completed. */
+ * which serialises contexts that upload concurrently. */
 static int upload_staged2(ndt_ctx* c, void* d1, const void* s1, size_t b1, void* d2, const void* s2, size_t b2) {
-    if (c->pin_pending) {
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        c->pin_pending = false;
-    }
     const size_t off2 = (b1 + 255) & ~(size_t)255;
-    int e = pinned_reserve(c, off2 + b2);
+    char* p = nullptr;
+    int e = pinned_stage(c, off2 + b2, &p);
     if (e) return e;
-    std::memcpy(c->pin, s1, b1);
-    HIP_TRY(hipMemcpyAsync(d1, c->pin, b1, hipMemcpyHostToDevice, c->stream));
-    if (b2) {
-        std::memcpy((char*)c->pin + off2, s2, b2);
-        HIP_TRY(hipMemcpyAsync(d2, (char*)c->pin + off2, b2, hipMemcpyHostToDevice, c->stream));
-    }
+    std::memcpy(p, s1, b1);
     c->pin_pending = true;
+    HIP_TRY(hipMemcpyAsync(d1, p, b1, hipMemcpyHostToDevice, c->stream));
+    if (b2) {
+        std::memcpy(p + off2, s2, b2);
+        HIP_TRY(hipMemcpyAsync(d2, p + off2, b2, hipMemcpyHostToDevice, c->stream));
+    }
     return 0;
 }
 
@@ -301,40 +320,69 @@ static int upload_staged(ndt_ctx* c, void* dst, const void* src, size_t bytes) {
     return upload_staged2(c, dst, src, bytes, nullptr, nullptr, 0);
 }
 
-/* m points (x, y, z, w floats) to dst through the pinned staging buffer in chunks
- * of 16,384 points: each chunk is copied and checked on the host, then its copy to
- * the device is queued, so the transfer of one chunk overlaps the host work on the
- * next.  Returns NDT_ERR_INVALID at the first chunk holding a point whose x, y or
- * z is not finite (chunks before it may already be on the device). */
-static int upload_points_finite(ndt_ctx* c, void* dst, const float* src, int64_t m) {
-    if (c->pin_pending) {
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        c->pin_pending = false;
-    }
-    int e = pinned_reserve(c, sizeof(float4) * (size_t)m);
-    if (e) return e;
-    constexpr int64_t CHUNK = 16384;
-    for (int64_t p0 = 0; p0 < m; p0 += CHUNK) {
-        const int64_t n = std::min(CHUNK, m - p0);
-        const float* sp = src + 4 * p0;
-        float* hp = (float*)c->pin + 4 * p0;
-        bool finite = true;
-        for (int64_t i = 0; i < 4 * n; i += 4) {
-            const float x = sp[i], y = sp[i + 1], z = sp[i + 2];
-            hp[i] = x;
-            hp[i + 1] = y;
-            hp[i + 2] = z;
-            hp[i + 3] = sp[i + 3];
-            /* v - v is 0 for a finite v and NaN for an infinite or NaN one */
-            finite &= (x - x == 0.0f) & (y - y == 0.0f) & (z - z == 0.0f);
-        }
+/* Points of the concatenated arrays [p0, p1) to the staging buffer; false if `finite` is
+ * asked for and an x, y or z is not (the copy is then of no use). */
+static bool gather_points(float* dst, const float* const* arrays, const int64_t* offsets, int32_t S, int64_t p0,
+                          int64_t p1, bool finite) {
+    typedef float vec4 __attribute__((vector_size(16)));
+    int32_t s = (int32_t)(std::upper_bound(offsets, offsets + S, p0) - offsets) - 1;
+    vec4 sum[4] = {};
+    for (int64_t a = p0; a < p1; s++) {
+        const int64_t e = s + 1 < S ? std::min(p1, offsets[s + 1]) : p1;
+        const float* src = arrays[s] + 4 * (a - offsets[s]);
+        float* d = dst + 4 * (a - p0);
         if (!finite) {
-            c->pin_pending = p0 > 0;
-            return fail(NDT_ERR_INVALID, "compat mode needs finite map points");
+            std::memcpy(d, src, sizeof(vec4) * (size_t)(e - a));
+        } else {
+            for (int64_t i = 0; i < e - a; i++) {
+                vec4 v;
+                std::memcpy(&v, src + 4 * i, sizeof(v));
+                std::memcpy(d + 4 * i, &v, sizeof(v));
+                sum[i & 3] += v - v; /* 0 for a finite coordinate, NaN for an infinite or NaN one */
+            }
         }
-        HIP_TRY(hipMemcpyAsync((char*)dst + sizeof(float4) * p0, hp, sizeof(float4) * n, hipMemcpyHostToDevice,
-                               c->stream));
+        a = e;
+    }
+    for (int k = 0; k < 3; k++)
+        if (!(sum[0][k] + sum[1][k] + sum[2][k] + sum[3][k] == 0.0f)) return false;
+    return true;
+}
+
+/* Uploads of points go through the staging buffer in pieces, at most UPLOAD_RING of them
+ * in it at a time: the copy of one is under way while the next is filled.
+ * Measured per call with pieces of 0.5, 1, 2, 4 and 8 MB: a batch of 28 MB 3.98, 3.69,
+ * 3.61, 3.65 and 3.69 ms, a callback on a 16 MB map 1.23, 1.23, 1.20, 1.23 and 1.30 ms
+ * (1.88 ms with a copy of every 256 KB and a scalar check).  One thread fills them: four
+ * took 1.08 ms for that map when its pages and the CPUs were warm, but up to 5 ms on the
+ * first calls of a new state. */
+constexpr size_t UPLOAD_PIECE = (size_t)2 << 20;
+constexpr int UPLOAD_RING = 6;
+
+/* `head_bytes` (a multiple of 256) and the t points of S arrays behind them to dst.  With
+ * `finite`, NDT_ERR_INVALID if a point's x, y or z is not finite (parts of the upload may
+ * have been made).  The arrays are free when this returns. */
+static int upload_points(ndt_ctx* c, char* dst, const void* head, size_t head_bytes, const float* const* arrays,
+                         const int64_t* offsets, int32_t S, int64_t t, bool finite) {
+    const size_t bytes = sizeof(float4) * (size_t)t;
+    const int64_t step = (int64_t)(UPLOAD_PIECE / sizeof(float4));
+    const int64_t pieces = (t + step - 1) / step, half = UPLOAD_RING / 2;
+    char* stage = nullptr;
+    int err = pinned_stage(c, head_bytes + std::min(bytes, UPLOAD_RING * UPLOAD_PIECE), &stage);
+    if (err) return err;
+    if (head_bytes) std::memcpy(stage, head, head_bytes);
+    for (int64_t k = 0; k < pieces; k++) {
+        const int64_t p0 = k * step, p1 = std::min(t, p0 + step);
+        /* the ring's halves are filled again once the copies from them have completed */
+        if (k >= UPLOAD_RING && k % half == 0) HIP_TRY(hipEventSynchronize(c->ev_stage[k / half & 1]));
+        char* d = stage + head_bytes + UPLOAD_PIECE * (size_t)(k % UPLOAD_RING);
+        if (!gather_points((float*)d, arrays, offsets, S, p0, p1, finite))
+            return fail(NDT_ERR_INVALID, "compat mode needs finite map points");
+        const size_t lead = k == 0 ? head_bytes : 0;
         c->pin_pending = true;
+        HIP_TRY(hipMemcpyAsync(dst + head_bytes - lead + sizeof(float4) * (size_t)p0, d - lead,
+                               lead + sizeof(float4) * (size_t)(p1 - p0), hipMemcpyHostToDevice, c->stream));
+        if (pieces > UPLOAD_RING && (k + 1) % half == 0)
+            HIP_TRY(hipEventRecord(c->ev_stage[k / half & 1], c->stream));
     }
     return 0;
 }
@@ -343,7 +391,8 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     const double res = (double)g->params.resolution;
     BUF_TRY(c->pts, sizeof(float4) * m);
     {
-        const int eu = upload_staged(c, c->pts.p, map, sizeof(float4) * m);
+        const int64_t first = 0;
+        const int eu = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, false);
         if (eu) return eu;
     }
     DevBuf& mm = c->bk_mm;
@@ -538,7 +587,8 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
     /* initCompute, src/CPU/ndt_mapping/kernel.cpp:1302-1373 */
     const float res = g->params.resolution;
     BUF_TRY(c->pts, sizeof(float4) * m);
-    int e = upload_points_finite(c, c->pts.p, map, m);
+    const int64_t first = 0;
+    int e = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, true);
     if (e) return e;
     DevBuf& mm = c->bk_mm;
     BUF_TRY(mm, 64);
@@ -906,76 +956,63 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     return collect_results(c, counts, S, aborted, results, used_alt);
 }
 
-/* Spreads the bits of a 10-bit value to every third bit (Morton interleave). */
-static inline uint32_t spread3(uint32_t v) {
-    v &= 0x3ff;
-    v = (v | (v << 16)) & 0x030000FF;
-    v = (v | (v << 8)) & 0x0300F00F;
-    v = (v | (v << 4)) & 0x030C30C3;
-    v = (v | (v << 2)) & 0x09249249;
-    return v;
-}
-
 /* Copies scans into one device buffer, each scan's points reordered along a Morton
  * curve of 1 m cells of its own (sensor-frame) coordinates: consecutive points,
  * and so the points of one workgroup, then look up neighbouring voxels and hit the
  * same cache lines.  A rigid transform keeps that locality.  The alignment does not
- * depend on the point order beyond floating-point rounding of the sums. */
+ * depend on the point order beyond floating-point rounding of the sums.  The points go
+ * to the device as they are and are ordered there; the work is enqueued on the context's
+ * stream, and the callers' buffers are free when this returns. */
 static int pack_scans(ndt_ctx* c, DevBuf& dst, const float* const* scans, const int64_t* counts, int32_t S,
                       std::vector<int64_t>& offsets, int64_t* total) {
     offsets.assign(S, 0);
-    int64_t t = 0;
+    int64_t t = 0, ntiles = 0;
+    int32_t nsmall = 0;
     for (int32_t s = 0; s < S; s++) {
         if (!scans[s] || counts[s] <= 0) return fail(NDT_ERR_INVALID, "empty or null scan");
         if (counts[s] > 0x7fffffffll) return fail(NDT_ERR_UNSUPPORTED, "scan larger than 2^31 points");
         offsets[s] = t;
         t += counts[s];
+        if (counts[s] <= ORDER_SMALL) nsmall++;
+        else ntiles += (counts[s] + ORDER_TILE - 1) / ORDER_TILE;
     }
+    if (ntiles > 0x7fffffffll) return fail(NDT_ERR_UNSUPPORTED, "scans larger than 2^43 points together");
+    /* the small scans' segments, the larger ones', then their tiles */
+    const size_t seg_bytes = sizeof(OrderSeg) * (size_t)S;
+    const size_t head_bytes = (seg_bytes + sizeof(OrderTile) * (size_t)ntiles + 255) & ~(size_t)255;
+    const size_t words = sizeof(uint32_t) * (size_t)t;
     BUF_TRY(dst, sizeof(float4) * t);
-    std::vector<float> staging((size_t)(4 * t));
-    auto work = [&](int32_t s0, int32_t s1) {
-        /* stable LSD radix sort of the 30-bit Morton keys, three passes of 10 bits */
-        std::vector<uint32_t> key, idx, tmp, cnt(1025);
-        for (int32_t s = s0; s < s1; s++) {
-            const float* src = scans[s];
-            const int64_t n = counts[s];
-            key.resize((size_t)n);
-            idx.resize((size_t)n);
-            tmp.resize((size_t)n);
-            for (int64_t i = 0; i < n; i++) {
-                uint32_t q[3];
-                for (int k = 0; k < 3; k++) {
-                    float v = src[4 * i + k];
-                    double cell = std::isfinite(v) ? std::floor((double)v) + 512.0 : 0.0;
-                    q[k] = (uint32_t)std::min(1023.0, std::max(0.0, cell));
-                }
-                key[(size_t)i] = spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
-                idx[(size_t)i] = (uint32_t)i;
-            }
-            for (int sh = 0; sh < 30; sh += 10) {
-                std::fill(cnt.begin(), cnt.end(), 0u);
-                for (int64_t i = 0; i < n; i++) cnt[((key[idx[(size_t)i]] >> sh) & 1023u) + 1]++;
-                for (int b = 0; b < 1024; b++) cnt[(size_t)b + 1] += cnt[(size_t)b];
-                for (int64_t i = 0; i < n; i++) tmp[cnt[(key[idx[(size_t)i]] >> sh) & 1023u]++] = idx[(size_t)i];
-                idx.swap(tmp);
-            }
-            float* d = staging.data() + 4 * offsets[s];
-            for (int64_t i = 0; i < n; i++) std::memcpy(d + 4 * i, src + 4 * (size_t)idx[(size_t)i], 16);
+    BUF_TRY(c->raw, head_bytes + sizeof(float4) * (size_t)t);
+    if (ntiles > 0) BUF_TRY(c->order, 2 * words + sizeof(uint32_t) * ORDER_HIST_WORDS * (size_t)ntiles);
+    std::vector<char> head(head_bytes);
+    OrderSeg* segs = (OrderSeg*)head.data();
+    OrderTile* tiles = (OrderTile*)(head.data() + seg_bytes);
+    int32_t small = 0, large = nsmall, tile = 0;
+    for (int32_t s = 0; s < S; s++) {
+        OrderSeg sg{offsets[s], (int32_t)counts[s], 0, 0, 0};
+        if (counts[s] <= ORDER_SMALL) {
+            segs[small++] = sg;
+            continue;
         }
-    };
-    /* scans are independent: reorder them on up to 16 host threads */
-    const int32_t nthreads = (int32_t)std::max(1u, std::min(16u, std::min(std::thread::hardware_concurrency(),
-                                                                           (unsigned)((S + 3) / 4))));
-    if (nthreads <= 1 || t < (1 << 16)) {
-        work(0, S);
-    } else {
-        std::vector<std::thread> pool;
-        for (int32_t k = 0; k < nthreads; k++)
-            pool.emplace_back(work, (int32_t)((int64_t)S * k / nthreads), (int32_t)((int64_t)S * (k + 1) / nthreads));
-        for (auto& th : pool) th.join();
+        sg.tile0 = tile;
+        for (int64_t p = 0; p < counts[s]; p += ORDER_TILE)
+            tiles[tile++] = {offsets[s] + p, (int32_t)std::min<int64_t>(ORDER_TILE, counts[s] - p), large - nsmall};
+        sg.ntiles = tile - sg.tile0;
+        segs[large++] = sg;
     }
-    HIP_TRY(hipMemcpyAsync(dst.p, staging.data(), sizeof(float4) * t, hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    int e = upload_points(c, c->raw.as<char>(), head.data(), head_bytes, scans, offsets.data(), S, t, false);
+    if (e) return e;
+    const OrderSeg* d_segs = c->raw.as<OrderSeg>();
+    const OrderTile* d_tiles = (const OrderTile*)(c->raw.as<char>() + seg_bytes);
+    const float4* raw = (const float4*)(c->raw.as<char>() + head_bytes);
+    if (ntiles > 0) {
+        /* the passes' second key and index arrays lie in dst: the last pass, which
+         * writes the points there, reads the first ones */
+        uint32_t *w = c->order.as<uint32_t>(), *w2 = dst.as<uint32_t>();
+        LAUNCH_TRY(launch_order_large(raw, d_segs + nsmall, S - nsmall, d_tiles, (int)ntiles, w, w2, w + t, w2 + t,
+                                      w + 2 * t, dst.as<float4>(), c->stream));
+    }
+    if (nsmall > 0) LAUNCH_TRY(launch_order_small(raw, d_segs, nsmall, dst.as<float4>(), c->stream));
     *total = t;
     return 0;
 }

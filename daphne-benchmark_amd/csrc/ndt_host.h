@@ -146,6 +146,7 @@ struct ndt_ctx {
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipEvent_t ev2 = nullptr; /* between the two graphs of a captured learned step */
+    hipEvent_t ev_stage[2] = {nullptr, nullptr}; /* copies out of the staging buffer's halves */
     int cus = 0;
     /* device address of the allocation-free entry point's workspace on this
      * context's device (looked up at creation), or null with the lookup's error */
@@ -153,6 +154,7 @@ struct ndt_ctx {
     int scratch_err = 0;
     char name[256] = {0};
     /* workspaces */
+    DevBuf raw, order; /* scans as uploaded, and the work space of ordering them */
     DevBuf pts, desc, states, sync, partials, out, guesses, small, partials2, queue, items, done;
     /* grid-build temporaries, and the compat callback's grid and scan, kept for
      * reuse: freeing device memory synchronises the device, which would serialise
@@ -165,6 +167,7 @@ struct ndt_ctx {
      * from it may still be in flight on the stream */
     void* pin = nullptr;
     size_t pin_bytes = 0;
+    size_t pin_off = 0; /* end of the part that copies in flight may read */
     bool pin_pending = false;
     /* small pinned buffer for scalars read back by host-side control (bounding
      * box, run counts, a compat pass's sums); each use ends with a stream

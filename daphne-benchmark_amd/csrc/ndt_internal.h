@@ -438,6 +438,27 @@ struct ScanOut {
  * (defined in ndt_kernels.hip; every launcher enqueues on `stream` and returns a
  * hipError_t value) */
 
+/* Scan points in the order of their Morton curve (see k_order_small): scans of up to
+ * ORDER_SMALL points one workgroup each, larger ones in tiles of ORDER_TILE points. */
+constexpr int ORDER_SMALL = 8192, ORDER_TILE = 4096;
+constexpr int ORDER_HIST_WORDS = 1024; /* histogram words per tile */
+struct OrderSeg {
+    int64_t offset; /* first point of the scan */
+    int32_t n;
+    int32_t tile0, ntiles; /* larger scans: its tiles */
+    int32_t pad;
+};
+struct OrderTile {
+    int64_t start; /* first point */
+    int32_t n;
+    int32_t seg; /* index of the scan among the larger ones */
+};
+int launch_order_small(const float4* raw, const OrderSeg* segs, int nsegs, float4* out, hipStream_t stream);
+/* key_a/b, idx_a/b: a word per point of the batch each; hist: ORDER_HIST_WORDS per tile */
+int launch_order_large(const float4* raw, const OrderSeg* segs, int nsegs, const OrderTile* tiles, int ntiles,
+                       uint32_t* key_a, uint32_t* key_b, uint32_t* idx_a, uint32_t* idx_b, uint32_t* hist, float4* out,
+                       hipStream_t stream);
+
 int launch_bbox(const float4* pts, int64_t n, uint32_t* minmax_bits /* 6 */, hipStream_t stream);
 int launch_keys_ndt(const float4* pts, int64_t n, double resolution, const int64_t* origin_cell,
                     const int* bits, uint64_t* keys, uint32_t* vals, hipStream_t stream);

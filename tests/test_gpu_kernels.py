@@ -69,3 +69,46 @@ def test_dense_index_matches_hashed(A, ctx, box, res):
         x, y = dense.derivatives(scan, p, prm=q), hashed.derivatives(scan, p, prm=q)
         assert x[3] == y[3] and x[3] > 0
         assert x[0] == y[0] and np.array_equal(x[1], y[1]) and np.array_equal(x[2], y[2])
+
+
+def _curve_order(scan):
+    """The order of a scan's points: stable, along the Morton curve of 1 m cells."""
+    key = np.zeros(len(scan), np.uint32)
+    for k in range(3):
+        v = scan[:, k].astype(np.float64)
+        q = np.where(np.isfinite(v), np.clip(np.floor(np.where(np.isfinite(v), v, 0.0)) + 512, 0, 1023), 0)
+        for b in range(10):
+            key |= ((q.astype(np.uint32) >> b) & 1) << (3 * b + k)
+    return np.argsort(key, kind="stable")
+
+
+@pytest.mark.parametrize("counts", [(1,), (63, 64, 65), (1023, 1, 1025), (8192,), (8193,), (2047, 20481, 12288, 700), (2200000,)])
+def test_scan_order(A, ctx, scene, counts):
+    """Scans of one workgroup (up to 8,192 points) and of several tiles (4,096 points),
+    alone and mixed, with ties, far-off and non-finite points, and more points than the
+    staging buffer's halves hold: a scan gives the same bits as the same points in curve
+    order, and other bits than in the reverse of it where the order can be told."""
+    sc, mp, grid, _ = scene
+    rng = np.random.default_rng(sum(counts))
+    raw, guesses = [], []
+    for k, n in enumerate(counts):
+        scan, _, guess = A.make_scan(sc, mp, A.scan_cfg(min(n, 20000)), 90 + k)
+        scan = np.tile(scan, (-(-n // len(scan)), 1))[:n]
+        scan = np.ascontiguousarray(scan[rng.permutation(n)])
+        scan[n // 2:, :3] += rng.uniform(-0.01, 0.01, (n - n // 2, 3)).astype(np.float32)
+        for j, bad in enumerate((np.nan, np.inf, -np.inf, 3e38, -700.0)):
+            if n > 60:
+                scan[rng.integers(n), j % 3] = bad
+        raw.append(scan)
+        guesses.append(guess)
+    prm = A.params(A.NDT_MODE_NDT, max_iterations=2, points_per_wg=256)
+
+    def bits(scans):
+        return [(r["final_f64"].tobytes(), r["score"], r["iterations"], r["passes"])
+                for r in grid.align_batch(scans, guesses, prm)]
+    got = bits(raw)
+    ordered = [s[_curve_order(s)] for s in raw]
+    assert got == bits(ordered)
+    if max(counts) >= 1023:
+        # reversed input: ties come out the other way round, so the sums round otherwise
+        assert got != bits([np.ascontiguousarray(s[::-1]) for s in ordered])
