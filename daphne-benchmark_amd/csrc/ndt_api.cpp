@@ -219,37 +219,17 @@ static inline float ord2f(uint32_t u) {
     return f;
 }
 
-/* runs of equal keys in a sorted array: flags -> ranks -> starts; returns count */
-static int sorted_runs(ndt_ctx* c, const uint64_t* keys, int64_t n, int shift, uint64_t limit, DevBuf& flags,
-                       DevBuf& ranks, DevBuf& starts, DevBuf& scratch, int64_t* nruns) {
-    BUF_TRY(flags, sizeof(uint32_t) * (n + 1));
-    BUF_TRY(ranks, sizeof(uint32_t) * (n + 1));
-    BUF_TRY(scratch, scan_scratch_bytes(n) + 512);
-    LAUNCH_TRY(launch_run_heads(keys, n, shift, limit, flags.as<uint32_t>(), c->stream));
-    uint32_t* total = (uint32_t*)((char*)scratch.p + ((scan_scratch_bytes(n) + 255) & ~(size_t)255));
-    LAUNCH_TRY(exclusive_scan_u32(flags.as<uint32_t>(), ranks.as<uint32_t>(), n, total, scratch.p, c->stream));
-    HIP_TRY(hipMemcpyAsync(c->hsmall, total, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+/* runs of equal keys in a sorted array: their starts and number, and the number of keys
+ * below the limit */
+static int sorted_runs(ndt_ctx* c, const uint64_t* keys, int64_t n, int shift, uint64_t limit, DevBuf& starts,
+                       DevBuf& scratch, int64_t* nruns, int64_t* below) {
+    BUF_TRY(starts, sizeof(uint32_t) * (n + 1));
+    BUF_TRY(scratch, runs_scratch_bytes(n));
+    LAUNCH_TRY(launch_runs(keys, n, shift, limit, starts.as<uint32_t>(), scratch.as<uint32_t>(), c->stream));
+    HIP_TRY(hipMemcpyAsync(c->hsmall, scratch.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    const uint32_t h_total = *(const uint32_t*)c->hsmall;
-    BUF_TRY(starts, sizeof(uint32_t) * (h_total + 1));
-    LAUNCH_TRY(launch_run_starts(flags.as<uint32_t>(), ranks.as<uint32_t>(), n, starts.as<uint32_t>(), c->stream));
-    *nruns = h_total;
-    return 0;
-}
-
-/* count of sorted keys below limit (non-sentinel prefix) */
-static int count_below(ndt_ctx* c, const uint64_t* keys, int64_t n, uint64_t limit, int64_t* out) {
-    /* binary search on the host over a few device reads */
-    int64_t lo = 0, hi = n;
-    while (lo < hi) {
-        int64_t mid = (lo + hi) / 2;
-        uint64_t k = 0;
-        HIP_TRY(hipMemcpyAsync(&k, keys + mid, sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (k < limit) lo = mid + 1;
-        else hi = mid;
-    }
-    *out = lo;
+    *nruns = ((const uint32_t*)c->hsmall)[0];
+    *below = ((const uint32_t*)c->hsmall)[1];
     return 0;
 }
 
@@ -387,22 +367,32 @@ static int upload_points(ndt_ctx* c, char* dst, const void* head, size_t head_by
     return 0;
 }
 
+/* bounding box of the m points in c->pts, as ordered words (minima, maxima) */
+static int map_bounds(ndt_ctx* c, int64_t m, uint32_t mm[6]) {
+    BUF_TRY(c->bk_mm, 64);
+    uint32_t* hs = (uint32_t*)c->hsmall;
+    const uint32_t init[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
+    std::memcpy(hs, init, sizeof(init));
+    HIP_TRY(hipMemcpyAsync(c->bk_mm.p, hs, sizeof(init), hipMemcpyHostToDevice, c->stream));
+    LAUNCH_TRY(launch_bbox(c->pts.as<float4>(), m, c->bk_mm.as<uint32_t>(), c->stream));
+    HIP_TRY(hipMemcpyAsync(hs + 16, c->bk_mm.p, sizeof(init), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    std::memcpy(mm, hs + 16, sizeof(init));
+    return 0;
+}
+
 static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) {
     const double res = (double)g->params.resolution;
+    int e = 0;
     BUF_TRY(c->pts, sizeof(float4) * m);
     {
         const int64_t first = 0;
-        const int eu = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, false);
-        if (eu) return eu;
+        e = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, false);
+        if (e) return e;
     }
-    DevBuf& mm = c->bk_mm;
-    BUF_TRY(mm, 64);
-    uint32_t init[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
-    HIP_TRY(hipMemcpyAsync(mm.p, init, sizeof(init), hipMemcpyHostToDevice, c->stream));
-    LAUNCH_TRY(launch_bbox(c->pts.as<float4>(), m, mm.as<uint32_t>(), c->stream));
     uint32_t h_mm[6];
-    HIP_TRY(hipMemcpyAsync(h_mm, mm.p, sizeof(h_mm), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    e = map_bounds(c, m, h_mm);
+    if (e) return e;
     if (h_mm[0] == 0xFFFFFFFFu) return fail(NDT_ERR_INVALID, "map has no finite points");
     int64_t lo_cell[3], hi_cell[3];
     for (int k = 0; k < 3; k++) {
@@ -415,40 +405,35 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     const int B = g->bits[0] + g->bits[1] + g->bits[2];
     if (B + 5 > 62) return fail(NDT_ERR_UNSUPPORTED, "map extent too large for the cell key");
     DevBuf &keys = c->bk_keys, &vals = c->bk_vals, &keys_t = c->bk_keys_t, &vals_t = c->bk_vals_t;
-    DevBuf &scratch = c->bk_scratch, &flags = c->bk_flags, &ranks = c->bk_ranks, &starts = c->bk_starts;
-    DevBuf& sc2 = c->bk_sc2;
+    DevBuf &scratch = c->bk_scratch, &starts = c->bk_starts, &sc2 = c->bk_sc2;
     BUF_TRY(keys, sizeof(uint64_t) * m);
     BUF_TRY(vals, sizeof(uint32_t) * m);
     BUF_TRY(keys_t, sizeof(uint64_t) * m);
     BUF_TRY(vals_t, sizeof(uint32_t) * m);
     BUF_TRY(scratch, radix_sort_scratch_bytes(m));
-    LAUNCH_TRY(launch_keys_ndt(c->pts.as<float4>(), m, res, g->origin_cell, g->bits, keys.as<uint64_t>(),
-                               vals.as<uint32_t>(), c->stream));
+    const uint64_t limit = (1ull << B) - 1; /* the key of points without a cell */
+    LAUNCH_TRY(launch_keys_ndt(c->pts.as<float4>(), m, res, g->origin_cell, g->bits,
+                               (radix_sort_from_tmp(B) ? keys_t : keys).as<uint64_t>(), c->stream));
     LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
-                                B + 1, scratch.p, c->stream));
-    const uint64_t limit = 1ull << B;
+                                B, true, scratch.p, c->stream));
     int64_t nvox = 0, nvalid_pts = 0;
-    int e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, flags, ranks, starts, sc2, &nvox);
-    if (e) return e;
-    e = count_below(c, keys.as<uint64_t>(), m, limit, &nvalid_pts);
+    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, starts, sc2, &nvox, &nvalid_pts);
     if (e) return e;
     if (nvox == 0) return fail(NDT_ERR_INVALID, "map has no finite points");
-    BUF_TRY(g->all_mean, sizeof(double) * 3 * nvox);
-    BUF_TRY(g->all_icov, sizeof(double) * 9 * nvox);
-    BUF_TRY(g->all_cov, sizeof(double) * 9 * nvox);
-    BUF_TRY(g->all_count, sizeof(int32_t) * nvox);
-    BUF_TRY(g->all_valid, sizeof(uint32_t) * (nvox + 1));
-    BUF_TRY(g->all_key, sizeof(uint64_t) * nvox);
-    LAUNCH_TRY(launch_voxel_stats_ndt(c->pts.as<float4>(), vals.as<uint32_t>(), keys.as<uint64_t>(), starts.as<uint32_t>(),
-                                      nvox, nvalid_pts, g->params.min_points, g->params.min_eig_ratio, g->bits,
-                                      g->all_mean.as<double>(), g->all_icov.as<double>(), g->all_cov.as<double>(),
-                                      g->all_count.as<int32_t>(), g->all_valid.as<uint32_t>(), g->all_key.as<uint64_t>(),
-                                      c->stream));
-    /* map points sorted by voxel and a hash of the occupied voxels, for nearest-point
-     * queries (fitness score) */
+    /* map points sorted by voxel: for the statistics, and with a hash of the occupied
+     * voxels for nearest-point queries (fitness score) */
     BUF_TRY(g->fit_pts, sizeof(float4) * (size_t)std::max<int64_t>(nvalid_pts, 1));
     LAUNCH_TRY(launch_gather_points(c->pts.as<float4>(), vals.as<uint32_t>(), nvalid_pts, g->fit_pts.as<float4>(),
                                     c->stream));
+    BUF_TRY(g->all_mean, sizeof(double) * 3 * nvox);
+    BUF_TRY(g->all_icov, sizeof(double) * 9 * nvox);
+    BUF_TRY(g->all_count, sizeof(int32_t) * nvox);
+    BUF_TRY(g->all_valid, sizeof(uint32_t) * (nvox + 1));
+    BUF_TRY(g->all_key, sizeof(uint64_t) * nvox);
+    LAUNCH_TRY(launch_voxel_stats_ndt(g->fit_pts.as<float4>(), keys.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts,
+                                      g->params.min_points, g->params.min_eig_ratio, g->all_mean.as<double>(),
+                                      g->all_icov.as<double>(), g->all_count.as<int32_t>(), g->all_valid.as<uint32_t>(),
+                                      g->all_key.as<uint64_t>(), c->stream));
     const int flog2 = std::max(4, ceil_log2(2 * nvox));
     BUF_TRY(g->fit_slots, sizeof(HashSlot) << flog2);
     LAUNCH_TRY(launch_hash_clear(g->fit_slots.as<HashSlot>(), 1ll << flog2, c->stream));
@@ -518,11 +503,13 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
             BUF_TRY(keys_t, sizeof(uint64_t) * ne);
             BUF_TRY(vals_t, sizeof(uint32_t) * ne);
             BUF_TRY(scratch, radix_sort_scratch_bytes(ne));
-            LAUNCH_TRY(launch_dilate_emit(vkey_c.as<uint64_t>(), nv, g->bits, keys.as<uint64_t>(), vals.as<uint32_t>(),
-                                          c->stream));
+            const bool from_tmp = radix_sort_from_tmp(B + 5);
+            LAUNCH_TRY(launch_dilate_emit(vkey_c.as<uint64_t>(), nv, g->bits, (from_tmp ? keys_t : keys).as<uint64_t>(),
+                                          (from_tmp ? vals_t : vals).as<uint32_t>(), c->stream));
             LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(),
-                                        vals_t.as<uint32_t>(), ne, B + 5, scratch.p, c->stream));
-            e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, flags, ranks, starts, sc2, &nq);
+                                        vals_t.as<uint32_t>(), ne, B + 5, false, scratch.p, c->stream));
+            int64_t all = 0;
+            e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, starts, sc2, &nq, &all);
             if (e) return e;
         }
     }
@@ -590,17 +577,9 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
     const int64_t first = 0;
     int e = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, true);
     if (e) return e;
-    DevBuf& mm = c->bk_mm;
-    BUF_TRY(mm, 64);
-    uint32_t* hs = (uint32_t*)c->hsmall;
-    const uint32_t init[6] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u, 0u};
-    std::memcpy(hs, init, sizeof(init));
-    HIP_TRY(hipMemcpyAsync(mm.p, hs, sizeof(init), hipMemcpyHostToDevice, c->stream));
-    LAUNCH_TRY(launch_bbox(c->pts.as<float4>(), m, mm.as<uint32_t>(), c->stream));
-    HIP_TRY(hipMemcpyAsync(hs + 16, mm.p, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
     uint32_t h_mm[6];
-    std::memcpy(h_mm, hs + 16, sizeof(h_mm));
+    e = map_bounds(c, m, h_mm);
+    if (e) return e;
     CompatGridDev& d = g->cdev;
     int64_t ncells = 1;
     for (int k = 0; k < 3; k++) {
@@ -621,19 +600,19 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
         g->info.max_corner[k] = d.maxv[k];
     }
     DevBuf &keys = c->bk_keys, &vals = c->bk_vals, &keys_t = c->bk_keys_t, &vals_t = c->bk_vals_t;
-    DevBuf &scratch = c->bk_scratch, &flags = c->bk_flags, &ranks = c->bk_ranks, &starts = c->bk_starts;
-    DevBuf& sc2 = c->bk_sc2;
+    DevBuf &scratch = c->bk_scratch, &starts = c->bk_starts, &sc2 = c->bk_sc2;
     BUF_TRY(keys, sizeof(uint64_t) * m);
     BUF_TRY(vals, sizeof(uint32_t) * m);
     BUF_TRY(keys_t, sizeof(uint64_t) * m);
     BUF_TRY(vals_t, sizeof(uint32_t) * m);
     BUF_TRY(scratch, radix_sort_scratch_bytes(m));
-    LAUNCH_TRY(launch_keys_compat(c->pts.as<float4>(), m, d.minv, d.dims, res, keys.as<uint64_t>(), vals.as<uint32_t>(),
-                                  c->stream));
+    const int nbits = std::max(1, ceil_log2(ncells + 1));
+    LAUNCH_TRY(launch_keys_compat(c->pts.as<float4>(), m, d.minv, d.dims, res,
+                                  (radix_sort_from_tmp(nbits) ? keys_t : keys).as<uint64_t>(), c->stream));
     LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
-                                std::max(1, ceil_log2(ncells + 1)), scratch.p, c->stream));
-    int64_t nvox = 0;
-    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, (uint64_t)ncells, flags, ranks, starts, sc2, &nvox);
+                                nbits, true, scratch.p, c->stream));
+    int64_t nvox = 0, inside = 0;
+    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, (uint64_t)ncells, starts, sc2, &nvox, &inside);
     if (e) return e;
     BUF_TRY(g->all_mean, sizeof(double) * 3 * nvox);
     BUF_TRY(g->all_icov, sizeof(double) * 9 * nvox);

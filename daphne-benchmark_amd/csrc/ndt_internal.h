@@ -461,28 +461,28 @@ int launch_order_large(const float4* raw, const OrderSeg* segs, int nsegs, const
 
 int launch_bbox(const float4* pts, int64_t n, uint32_t* minmax_bits /* 6 */, hipStream_t stream);
 int launch_keys_ndt(const float4* pts, int64_t n, double resolution, const int64_t* origin_cell,
-                    const int* bits, uint64_t* keys, uint32_t* vals, hipStream_t stream);
+                    const int* bits, uint64_t* keys, hipStream_t stream);
 int launch_keys_compat(const float4* pts, int64_t n, const float* minv, const int* dims, float resolution,
-                       uint64_t* keys, uint32_t* vals, hipStream_t stream);
-/* stable LSD radix sort of (key, value) pairs on the low `nbits` bits; the result
- * ends in (keys, vals); tmp buffers hold n entries each; scratch from
- * radix_sort_scratch_bytes */
+                       uint64_t* keys, hipStream_t stream);
+/* stable LSD radix sort of (key, value) pairs on the low `nbits` bits.  The pairs are in
+ * (keys_tmp, vals_tmp) where radix_sort_from_tmp(nbits), otherwise in (keys, vals), and
+ * end in (keys, vals); with iota the values are the keys' indices and not read.  The tmp
+ * buffers hold n entries each; scratch from radix_sort_scratch_bytes */
 size_t radix_sort_scratch_bytes(int64_t n);
+bool radix_sort_from_tmp(int nbits);
 int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_t* vals_tmp, int64_t n,
-                     int nbits, void* scratch, hipStream_t stream);
+                     int nbits, bool iota, void* scratch, hipStream_t stream);
 size_t scan_scratch_bytes(int64_t n);
 /* exclusive prefix sum of n uint32 values; total (sum) written to *total_dev */
 int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_dev, void* scratch,
                        hipStream_t stream);
-/* flags[i] = 1 where a run of equal (key >> shift) starts; keys >= limit are excluded */
-int launch_run_heads(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* flags,
-                     hipStream_t stream);
-/* starts[rank] = i for each head i (rank = exclusive scan of flags) */
-int launch_run_starts(const uint32_t* flags, const uint32_t* ranks, int64_t n, uint32_t* starts,
-                      hipStream_t stream);
-int launch_voxel_stats_ndt(const float4* pts, const uint32_t* sorted_idx, const uint64_t* sorted_keys,
-                           const uint32_t* seg_start, int64_t nseg, int64_t nvalid_pts, int min_points,
-                           double min_eig_ratio, const int* bits, double* mean, double* icov, double* cov,
+/* starts[r] = where run r of equal (key >> shift) starts among the n sorted keys, keys >=
+ * limit left out; scratch[0] = number of runs, scratch[1] = number of keys below the limit */
+size_t runs_scratch_bytes(int64_t n);
+int launch_runs(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* starts, uint32_t* scratch,
+                hipStream_t stream);
+int launch_voxel_stats_ndt(const float4* pts, const uint64_t* sorted_keys, const uint32_t* seg_start, int64_t nseg,
+                           int64_t nvalid_pts, int min_points, double min_eig_ratio, double* mean, double* icov,
                            int32_t* count, uint32_t* valid, uint64_t* vkey, hipStream_t stream);
 int launch_compact_voxels(const uint32_t* valid, const uint32_t* rank, int64_t nvox, const double* mean,
                           const double* icov, const uint64_t* vkey, double* mean_out, double* icov_out,

@@ -18,7 +18,9 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_cooperative_groups.h>
 
+#include <algorithm>
 #include <mutex>
+#include <utility>
 
 #include "ndt_internal.h"
 
@@ -183,13 +185,14 @@ struct KeyLayout {
     int b[3];
 };
 
+/* keys of points without a cell: all bits set, which no cell's key has (a map's cells
+ * leave the last one of an axis free) */
 __global__ void k_keys_ndt(const float4* __restrict__ pts, int64_t n, double res, KeyLayout L,
-                           uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
+                           uint64_t* __restrict__ keys) {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4 p = pts[i];
-    const uint64_t sentinel = 1ull << (L.b[0] + L.b[1] + L.b[2]);
-    uint64_t key = sentinel;
+    uint64_t key = (1ull << (L.b[0] + L.b[1] + L.b[2])) - 1;
     if (isfinite(p.x) && isfinite(p.y) && isfinite(p.z)) {
         int64_t c[3] = {(int64_t)floor((double)p.x / res) - L.o[0], (int64_t)floor((double)p.y / res) - L.o[1],
                         (int64_t)floor((double)p.z / res) - L.o[2]};
@@ -198,17 +201,16 @@ __global__ void k_keys_ndt(const float4* __restrict__ pts, int64_t n, double res
         if (ok) key = ((uint64_t)c[2] << (L.b[0] + L.b[1])) | ((uint64_t)c[1] << L.b[0]) | (uint64_t)c[0];
     }
     keys[i] = key;
-    vals[i] = (uint32_t)i;
 }
 
 int launch_keys_ndt(const float4* pts, int64_t n, double resolution, const int64_t* origin_cell, const int* bits,
-                    uint64_t* keys, uint32_t* vals, hipStream_t stream) {
+                    uint64_t* keys, hipStream_t stream) {
     KeyLayout L;
     for (int k = 0; k < 3; k++) {
         L.o[k] = origin_cell[k];
         L.b[k] = bits[k];
     }
-    hipLaunchKernelGGL(k_keys_ndt, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, resolution, L, keys, vals);
+    hipLaunchKernelGGL(k_keys_ndt, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, resolution, L, keys);
     return (int)hipGetLastError();
 }
 
@@ -226,97 +228,23 @@ __device__ inline int compat_linearize(const float* minv, const int* dims, float
     return ix + dims[0] * (iy + dims[1] * iz);
 }
 
-__global__ void k_keys_compat(const float4* __restrict__ pts, int64_t n, CompatLayout L, uint64_t* __restrict__ keys,
-                              uint32_t* __restrict__ vals) {
+__global__ void k_keys_compat(const float4* __restrict__ pts, int64_t n, CompatLayout L, uint64_t* __restrict__ keys) {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4 p = pts[i];
     keys[i] = (uint64_t)(uint32_t)compat_linearize(L.minv, L.dims, L.res, p.x, p.y, p.z);
-    vals[i] = (uint32_t)i;
 }
 
 int launch_keys_compat(const float4* pts, int64_t n, const float* minv, const int* dims, float resolution,
-                       uint64_t* keys, uint32_t* vals, hipStream_t stream) {
+                       uint64_t* keys, hipStream_t stream) {
     CompatLayout L;
     for (int k = 0; k < 3; k++) {
         L.minv[k] = minv[k];
         L.dims[k] = dims[k];
     }
     L.res = resolution;
-    hipLaunchKernelGGL(k_keys_compat, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, L, keys, vals);
+    hipLaunchKernelGGL(k_keys_compat, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, L, keys);
     return (int)hipGetLastError();
-}
-
-/* ------------------------------------------------------------------ radix sort
- * Stable LSD radix sort, 8-bit digits.  Per pass: per-tile digit histograms
- * (digit-major), one exclusive scan, and a stable scatter in which each tile
- * ranks its keys round by round with wave ballots. */
-
-constexpr int RS_BLOCK = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_BLOCK * RS_ITEMS;
-
-__global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const uint64_t* __restrict__ keys, int64_t n, int shift,
-                                                      uint32_t* __restrict__ hist, int nblocks) {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
-    __syncthreads();
-    int64_t base = (int64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; r++) {
-        int64_t idx = base + r * RS_BLOCK + threadIdx.x;
-        if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[(int64_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
-}
-
-__global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                         uint64_t* __restrict__ kout, uint32_t* __restrict__ vout,
-                                                         int64_t n, int shift, const uint32_t* __restrict__ offs,
-                                                         int nblocks) {
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[RS_BLOCK / WAVE][256];
-    const int tid = threadIdx.x;
-    const int wave = tid / WAVE, lane = tid % WAVE;
-    base[tid] = offs[(int64_t)tid * nblocks + blockIdx.x];
-    run[tid] = 0;
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    int64_t tbase = (int64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; r++) {
-        int64_t idx = tbase + r * RS_BLOCK + tid;
-        bool valid = idx < n;
-        uint64_t key = valid ? kin[idx] : 0;
-        uint32_t val = valid ? vin[idx] : 0;
-        uint32_t d = valid ? (uint32_t)((key >> shift) & 255u) : 256u;
-        uint64_t peers = __ballot(1);
-#pragma unroll
-        for (int b = 0; b < 9; b++) {
-            uint64_t m = __ballot((d >> b) & 1u);
-            peers &= ((d >> b) & 1u) ? m : ~m;
-        }
-        uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
-        for (int w = 0; w < RS_BLOCK / WAVE; w++) wcnt[w][tid] = 0;
-        __syncthreads();
-        if (valid && rank == 0) wcnt[wave][d] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        {
-            uint32_t acc = run[tid];
-            for (int w = 0; w < RS_BLOCK / WAVE; w++) {
-                uint32_t c = wcnt[w][tid];
-                wcnt[w][tid] = acc;
-                acc += c;
-            }
-            run[tid] = acc;
-        }
-        __syncthreads();
-        if (valid) {
-            uint32_t pos = base[d] + wcnt[wave][d] + rank;
-            kout[pos] = key;
-            vout[pos] = val;
-        }
-        __syncthreads();
-    }
 }
 
 /* ------------------------------------------------------------------ scan */
@@ -442,35 +370,161 @@ int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* t
     return (int)hipGetLastError();
 }
 
-size_t radix_sort_scratch_bytes(int64_t n) {
-    int64_t nb = (n + RS_TILE - 1) / RS_TILE;
-    int64_t h = 256 * nb;
-    return (size_t)h * sizeof(uint32_t) + scan_scratch_bytes(h) + 256;
+/* ------------------------------------------------------------------ radix sort
+ * Stable LSD radix sort of (key, value) pairs.  The digits are as wide as the fewest
+ * passes of up to RS_BITS bits need (map keys of 18 to 22 bits: two passes).  Three
+ * launches a pass: digit histograms of the tiles (digit-major), a scan of each digit's
+ * tile counts by a wave, and the scatter, in which a wave ranks its contiguous part of
+ * the tile 64 keys at a time by ballots over its own counters in LDS, so that no wave
+ * waits for another inside the tile.  Launches and their latency bound it up to a few
+ * 100 k pairs, the scatter's 24 bytes a pair above.  Against 8-bit digits ranked by the
+ * whole workgroup (three passes of up to five launches): 100 k points 92 -> 42 us, 1 M
+ * points 175 -> 100 us; loading those maps, with the run starts and the number of points
+ * in cells from the device instead of a search on the host, 0.81 -> 0.39 and 3.8 -> 3.0
+ * ms. */
+constexpr int RS_BITS = 11, RS_BLOCK = 256, RS_WAVES = RS_BLOCK / WAVE;
+
+static int rs_passes(int nbits) { return (std::max(1, nbits) + RS_BITS - 1) / RS_BITS; }
+/* tiles of 1024 keys while four times larger ones would leave most of the 256 compute
+ * units idle; larger tiles have fewer digit counters to clear, write and scan per key
+ * (a pass with tiles of 1024 and of 4096 keys: 100 k keys 16 and 31 us, 1 M keys 70 and
+ * 49 us) */
+constexpr int64_t RS_SMALL = 262144;
+static int rs_tile(int64_t n) { return n <= RS_SMALL ? 1024 : 4096; }
+
+/* lanes of the wave with the same digit (of `bits` bits) as this one, valid lanes only */
+__device__ inline uint64_t digit_peers(uint32_t d, int bits, bool valid) {
+    uint64_t peers = __ballot(valid);
+    for (int b = 0; b < bits; b++) {
+        const uint64_t m = __ballot((d >> b) & 1u);
+        peers &= ((d >> b) & 1u) ? m : ~m;
+    }
+    return peers;
 }
 
-int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits,
-                     void* scratch, hipStream_t stream) {
-    if (n <= 1 || nbits <= 0) return 0;
-    int nb = (int)((n + RS_TILE - 1) / RS_TILE);
-    int64_t h = 256ll * nb;
-    uint32_t* hist = (uint32_t*)scratch;
-    void* sc = (void*)(((uintptr_t)(hist + h) + 255) & ~(uintptr_t)255);
-    uint64_t *ki = keys, *ko = keys_tmp;
-    uint32_t *vi = vals, *vo = vals_tmp;
-    int passes = (nbits + 7) / 8;
-    for (int p = 0; p < passes; p++) {
-        int shift = 8 * p;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_BLOCK), 0, stream, ki, n, shift, hist, nb);
-        int e = exclusive_scan_u32(hist, hist, h, nullptr, sc, stream);
-        if (e) return e;
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_BLOCK), 0, stream, ki, vi, ko, vo, n, shift, hist, nb);
-        uint64_t* tk = ki; ki = ko; ko = tk;
-        uint32_t* tv = vi; vi = vo; vo = tv;
+/* this lane's place for digit d: the wave's next place for it plus the lower lanes'
+ * share; the counter moves on by all of them */
+__device__ inline uint32_t take_place(uint32_t* next, uint32_t d, int bits, bool valid) {
+    const uint64_t peers = digit_peers(d, bits, valid);
+    const int lane = threadIdx.x % WAVE;
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
+    uint32_t at = 0;
+    if (valid) at = next[d] + rank;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (valid && (peers >> lane) == 1ull) next[d] = at + 1; /* the last of them */
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return at;
+}
+
+__global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const uint64_t* __restrict__ keys, int64_t n, int tile, int shift,
+                                                      int bits, uint32_t* __restrict__ hist) {
+    __shared__ uint32_t h[1 << RS_BITS];
+    const int digits = 1 << bits, nb = gridDim.x;
+    for (int d = threadIdx.x; d < digits; d += RS_BLOCK) h[d] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * tile;
+    for (int r = threadIdx.x; r < tile; r += RS_BLOCK)
+        if (base + r < n) atomicAdd(&h[(uint32_t)(keys[base + r] >> shift) & (digits - 1)], 1u);
+    __syncthreads();
+    for (int d = threadIdx.x; d < digits; d += RS_BLOCK) hist[(int64_t)d * nb + blockIdx.x] = h[d];
+}
+
+/* a wave per digit: exclusive scan of its tile counts, and their total */
+__global__ __launch_bounds__(RS_BLOCK) void k_rs_offsets(uint32_t* __restrict__ hist, int digits, int nb,
+                                                         uint32_t* __restrict__ totals) {
+    const int d = blockIdx.x * RS_WAVES + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    if (d >= digits) return;
+    uint32_t* h = hist + (int64_t)d * nb;
+    uint32_t run = 0;
+    for (int i0 = 0; i0 < nb; i0 += WAVE) {
+        const uint32_t v = i0 + lane < nb ? h[i0 + lane] : 0u;
+        uint32_t incl = v;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            const uint32_t t = __shfl_up(incl, off, WAVE);
+            if (lane >= off) incl += t;
+        }
+        if (i0 + lane < nb) h[i0 + lane] = run + incl - v;
+        run += __shfl(incl, WAVE - 1, WAVE);
     }
-    if (ki != keys) {
-        hipError_t e = hipMemcpyAsync(keys, ki, sizeof(uint64_t) * n, hipMemcpyDeviceToDevice, stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(vals, vi, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, stream);
-        if (e != hipSuccess) return (int)e;
+    if (lane == 0) totals[d] = run;
+}
+
+/* vin == null: the values are the keys' indices */
+__global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                         uint64_t* __restrict__ kout, uint32_t* __restrict__ vout,
+                                                         int64_t n, int tile, int shift, int bits,
+                                                         const uint32_t* __restrict__ hist,
+                                                         const uint32_t* __restrict__ totals) {
+    __shared__ uint32_t next[RS_WAVES][1 << RS_BITS];
+    __shared__ uint32_t lw[RS_WAVES];
+    const int digits = 1 << bits, nb = gridDim.x;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    for (int w = 0; w < RS_WAVES; w++)
+        for (int d = tid; d < digits; d += RS_BLOCK) next[w][d] = 0;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * tile;
+    const int part = tile / RS_WAVES, m = (int)min((int64_t)tile, n - base);
+    const int b = wave * part, e = min(m, b + part);
+    for (int i = b + lane; i < e; i += WAVE)
+        atomicAdd(&next[wave][(uint32_t)(kin[base + i] >> shift) & (digits - 1)], 1u);
+    /* first place of every digit: thread t takes the digits t * per and on */
+    const int per = (digits + RS_BLOCK - 1) / RS_BLOCK;
+    uint32_t sum = 0, place;
+    for (int d = tid * per; d < min(digits, (tid + 1) * per); d++) sum += totals[d];
+    block_exclusive_scan(sum, &place, lw);
+    for (int d = tid * per; d < min(digits, (tid + 1) * per); d++) {
+        uint32_t run = place + hist[(int64_t)d * nb + blockIdx.x];
+        place += totals[d];
+        for (int w = 0; w < RS_WAVES; w++) {
+            const uint32_t c = next[w][d];
+            next[w][d] = run;
+            run += c;
+        }
+    }
+    __syncthreads();
+    for (int i0 = b; i0 < e; i0 += WAVE) {
+        const bool valid = i0 + lane < e;
+        const int64_t i = base + min(i0 + lane, m - 1);
+        const uint64_t k = kin[i];
+        const uint32_t v = vin ? vin[i] : (uint32_t)i;
+        const uint32_t at = take_place(next[wave], (uint32_t)(k >> shift) & (digits - 1), bits, valid);
+        if (valid) {
+            kout[at] = k;
+            vout[at] = v;
+        }
+    }
+}
+
+size_t radix_sort_scratch_bytes(int64_t n) {
+    const int64_t nb = (n + rs_tile(n) - 1) / rs_tile(n);
+    return sizeof(uint32_t) * (size_t)((nb + 1) << RS_BITS);
+}
+
+bool radix_sort_from_tmp(int nbits) { return rs_passes(nbits) & 1; }
+
+int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_t* vals_tmp, int64_t n, int nbits,
+                     bool iota, void* scratch, hipStream_t stream) {
+    if (n <= 0) return 0;
+    const int passes = rs_passes(nbits), tile = rs_tile(n);
+    const int bits = (std::max(1, nbits) + passes - 1) / passes, digits = 1 << bits;
+    const int nb = (int)((n + tile - 1) / tile);
+    uint32_t *totals = (uint32_t*)scratch, *hist = totals + (1 << RS_BITS);
+    uint64_t *ki = passes & 1 ? keys_tmp : keys, *ko = passes & 1 ? keys : keys_tmp;
+    uint32_t *vi = passes & 1 ? vals_tmp : vals, *vo = passes & 1 ? vals : vals_tmp;
+    for (int pass = 0; pass < passes; pass++) {
+        const int shift = pass * bits;
+        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(RS_BLOCK), 0, stream, ki, n, tile, shift, bits, hist);
+        hipLaunchKernelGGL(k_rs_offsets, dim3((digits + RS_WAVES - 1) / RS_WAVES), dim3(RS_BLOCK), 0, stream, hist, digits,
+                           nb, totals);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(RS_BLOCK), 0, stream, ki, pass == 0 && iota ? nullptr : vi, ko, vo,
+                           n, tile, shift, bits, hist, totals);
+        std::swap(ki, ko);
+        std::swap(vi, vo);
     }
     return (int)hipGetLastError();
 }
@@ -508,35 +562,6 @@ __device__ inline uint32_t curve_key(const float4 p) {
         q[k] = (uint32_t)fmin(1023.0, fmax(0.0, cell));
     }
     return spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
-}
-
-/* lanes of the wave with the same digit as this one (valid lanes only) */
-__device__ inline uint64_t digit_peers(uint32_t d, bool valid) {
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < ORDER_BITS; b++) {
-        const uint64_t m = __ballot((d >> b) & 1u);
-        peers &= ((d >> b) & 1u) ? m : ~m;
-    }
-    return peers;
-}
-
-/* this lane's place for digit d: the wave's next place for it plus the lower lanes'
- * share; the counter moves on by all of them */
-__device__ inline uint32_t take_place(uint32_t* next, uint32_t d, bool valid) {
-    const uint64_t peers = digit_peers(d, valid);
-    const int lane = threadIdx.x % WAVE;
-    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
-    uint32_t at = 0;
-    if (valid) at = next[d] + rank;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (valid && (peers >> lane) == 1ull) next[d] = at + 1; /* the last of them */
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    return at;
 }
 
 constexpr int ORDER_SMALL_WAVES = 16;
@@ -578,7 +603,7 @@ __global__ __launch_bounds__(1024) void k_order_small(const float4* __restrict__
             const bool valid = i0 + lane < e;
             const uint32_t v = valid ? src[i0 + lane] : 0u;
             const uint32_t d = valid ? (key[v] >> shift) & (ORDER_DIGITS - 1) : 0u;
-            const uint32_t at = take_place(next[wave], d, valid);
+            const uint32_t at = take_place(next[wave], d, ORDER_BITS, valid);
             if (valid) dst[at] = (uint16_t)v;
         }
         __syncthreads();
@@ -655,7 +680,7 @@ __global__ __launch_bounds__(256) void k_order_scatter(const float4* __restrict_
         const int64_t i = tl.start + min(i0 + lane, tl.n - 1);
         const uint32_t k = key_in[i];
         const uint32_t v = pass == 0 ? (uint32_t)(i - base) : idx_in[i];
-        const uint32_t at = take_place(next[wave], (k >> shift) & (ORDER_DIGITS - 1), valid);
+        const uint32_t at = take_place(next[wave], (k >> shift) & (ORDER_DIGITS - 1), ORDER_BITS, valid);
         if (valid) {
             if (pass == ORDER_PASSES - 1) {
                 out[base + at] = raw[base + v];
@@ -688,31 +713,83 @@ int launch_order_large(const float4* raw, const OrderSeg* segs, int nsegs, const
 
 /* ------------------------------------------------------------------ runs */
 
-__global__ void k_run_heads(const uint64_t* __restrict__ keys, int64_t n, int shift, uint64_t limit,
-                            uint32_t* __restrict__ flags) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t k = keys[i];
-    uint32_t f = 0;
-    if (k < limit) f = (i == 0) || ((keys[i - 1] >> shift) != (k >> shift));
-    flags[i] = f;
+/* Where runs of equal (key >> shift) start among the sorted keys below the limit, in three
+ * launches: run heads per tile, a scan of the tiles, and the starts.  A wave looks at 64
+ * keys at a time. */
+constexpr int RUN_TILE = SC_TILE, RUN_PART = RUN_TILE / (SC_BLOCK / WAVE);
+
+__device__ inline bool run_head(const uint64_t* keys, int64_t i, int shift, uint64_t limit) {
+    const uint64_t k = keys[i];
+    return k < limit && (i == 0 || (keys[i - 1] >> shift) != (k >> shift));
 }
 
-int launch_run_heads(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* flags,
-                     hipStream_t stream) {
-    hipLaunchKernelGGL(k_run_heads, dim3(grid_for(n, 256)), dim3(256), 0, stream, keys, n, shift, limit, flags);
-    return (int)hipGetLastError();
+__global__ __launch_bounds__(SC_BLOCK) void k_runs_count(const uint64_t* __restrict__ keys, int64_t n, int shift,
+                                                         uint64_t limit, uint32_t* __restrict__ bsum,
+                                                         uint32_t* __restrict__ below) {
+    __shared__ uint32_t cnt[SC_BLOCK / WAVE];
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int64_t base = (int64_t)blockIdx.x * RUN_TILE + wave * RUN_PART + lane;
+    uint32_t c = 0;
+    for (int r = 0; r < RUN_PART; r += WAVE) {
+        const int64_t i = base + r;
+        bool head = false;
+        if (i < n) {
+            head = run_head(keys, i, shift, limit);
+            /* keys below the limit: they are sorted, so one thread sees the end */
+            const bool in = keys[i] < limit;
+            if (!in && (i == 0 || keys[i - 1] < limit)) *below = (uint32_t)i;
+            if (in && i == n - 1) *below = (uint32_t)n;
+        }
+        c += (uint32_t)__popcll(__ballot(head));
+    }
+    if (lane == 0) cnt[wave] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t s = 0;
+        for (int w = 0; w < SC_BLOCK / WAVE; w++) s += cnt[w];
+        bsum[blockIdx.x] = s;
+    }
 }
 
-__global__ void k_run_starts(const uint32_t* __restrict__ flags, const uint32_t* __restrict__ ranks, int64_t n,
-                             uint32_t* __restrict__ starts) {
-    int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (flags[i]) starts[ranks[i]] = (uint32_t)i;
+__global__ __launch_bounds__(SC_BLOCK) void k_runs_write(const uint64_t* __restrict__ keys, int64_t n, int shift,
+                                                         uint64_t limit, const uint32_t* __restrict__ bsum,
+                                                         uint32_t* __restrict__ starts) {
+    __shared__ uint32_t cnt[SC_BLOCK / WAVE];
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int64_t base = (int64_t)blockIdx.x * RUN_TILE + wave * RUN_PART + lane;
+    uint32_t c = 0, heads = 0; /* bit r: this lane's key of round r is a head */
+    for (int r = 0; r < RUN_PART / WAVE; r++) {
+        const int64_t i = base + r * WAVE;
+        const bool head = i < n && run_head(keys, i, shift, limit);
+        heads |= (uint32_t)head << r;
+        c += (uint32_t)__popcll(__ballot(head));
+    }
+    if (lane == 0) cnt[wave] = c;
+    __syncthreads();
+    uint32_t at = bsum[blockIdx.x];
+    for (int w = 0; w < wave; w++) at += cnt[w];
+    for (int r = 0; r < RUN_PART / WAVE; r++) {
+        const bool head = (heads >> r) & 1u;
+        const uint64_t m = __ballot(head);
+        if (head)
+            starts[at + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                (uint32_t)(base + r * WAVE);
+        at += (uint32_t)__popcll(m);
+    }
 }
 
-int launch_run_starts(const uint32_t* flags, const uint32_t* ranks, int64_t n, uint32_t* starts, hipStream_t stream) {
-    hipLaunchKernelGGL(k_run_starts, dim3(grid_for(n, 256)), dim3(256), 0, stream, flags, ranks, n, starts);
+size_t runs_scratch_bytes(int64_t n) {
+    return sizeof(uint32_t) * (size_t)(2 + (n + RUN_TILE - 1) / RUN_TILE);
+}
+
+int launch_runs(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* starts, uint32_t* scratch,
+                hipStream_t stream) {
+    const int64_t nb = (n + RUN_TILE - 1) / RUN_TILE;
+    uint32_t* bsum = scratch + 2;
+    hipLaunchKernelGGL(k_runs_count, dim3((unsigned)nb), dim3(SC_BLOCK), 0, stream, keys, n, shift, limit, bsum,
+                       scratch + 1);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, bsum, nb, scratch);
+    hipLaunchKernelGGL(k_runs_write, dim3((unsigned)nb), dim3(SC_BLOCK), 0, stream, keys, n, shift, limit, bsum, starts);
     return (int)hipGetLastError();
 }
 
@@ -771,11 +848,11 @@ __device__ void sym3_eig(const double* Ain, double* ev, double* V) {
     }
 }
 
-__global__ void k_voxel_stats_ndt(const float4* __restrict__ pts, const uint32_t* __restrict__ sidx,
-                                  const uint64_t* __restrict__ skeys, const uint32_t* __restrict__ seg_start,
-                                  int64_t nseg, int64_t nvalid_pts, int min_points, double eig_ratio,
-                                  double* __restrict__ mean_out, double* __restrict__ icov_out,
-                                  double* __restrict__ cov_out, int32_t* __restrict__ count,
+/* pts: the map's points in the order of their voxels */
+__global__ void k_voxel_stats_ndt(const float4* __restrict__ pts, const uint64_t* __restrict__ skeys,
+                                  const uint32_t* __restrict__ seg_start, int64_t nseg, int64_t nvalid_pts,
+                                  int min_points, double eig_ratio, double* __restrict__ mean_out,
+                                  double* __restrict__ icov_out, int32_t* __restrict__ count,
                                   uint32_t* __restrict__ valid, uint64_t* __restrict__ vkey) {
     int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (s >= nseg) return;
@@ -783,22 +860,24 @@ __global__ void k_voxel_stats_ndt(const float4* __restrict__ pts, const uint32_t
     int64_t e = (s + 1 < nseg) ? (int64_t)seg_start[s + 1] : nvalid_pts;
     int64_t n = e - b;
     double sum[3] = {0, 0, 0};
+#pragma unroll 4
     for (int64_t k = b; k < e; k++) {
-        float4 p = pts[sidx[k]];
+        float4 p = pts[k];
         sum[0] += p.x;
         sum[1] += p.y;
         sum[2] += p.z;
     }
     double mean[3] = {sum[0] / (double)n, sum[1] / (double)n, sum[2] / (double)n};
     double C[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
     for (int64_t k = b; k < e; k++) {
-        float4 p = pts[sidx[k]];
+        float4 p = pts[k];
         double d[3] = {p.x - mean[0], p.y - mean[1], p.z - mean[2]};
         for (int r = 0; r < 3; r++)
             for (int c = 0; c < 3; c++) C[r * 3 + c] += d[r] * d[c];
     }
     uint32_t ok = 0;
-    double icov[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, cov[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    double icov[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (n >= min_points && n >= 2) {
         for (int k = 0; k < 9; k++) C[k] /= (double)(n - 1);
         double ev[3], V[9];
@@ -809,35 +888,25 @@ __global__ void k_voxel_stats_ndt(const float4* __restrict__ pts, const uint32_t
                 if (ev[k] < lo) ev[k] = lo;
             for (int r = 0; r < 3; r++)
                 for (int c = 0; c < 3; c++) {
-                    double a = 0, bb = 0;
-                    for (int k = 0; k < 3; k++) {
-                        a += V[r * 3 + k] * ev[k] * V[c * 3 + k];
-                        bb += V[r * 3 + k] * (1.0 / ev[k]) * V[c * 3 + k];
-                    }
-                    cov[r * 3 + c] = a;
-                    icov[r * 3 + c] = bb;
+                    double a = 0;
+                    for (int k = 0; k < 3; k++) a += V[r * 3 + k] * (1.0 / ev[k]) * V[c * 3 + k];
+                    icov[r * 3 + c] = a;
                 }
             ok = 1;
         }
     }
     for (int c = 0; c < 3; c++) mean_out[3 * s + c] = mean[c];
-    for (int k = 0; k < 9; k++) {
-        icov_out[9 * s + k] = icov[k];
-        cov_out[9 * s + k] = cov[k];
-    }
+    for (int k = 0; k < 9; k++) icov_out[9 * s + k] = icov[k];
     count[s] = (int32_t)n;
     valid[s] = ok;
     vkey[s] = skeys[b];
 }
 
-int launch_voxel_stats_ndt(const float4* pts, const uint32_t* sorted_idx, const uint64_t* sorted_keys,
-                           const uint32_t* seg_start, int64_t nseg, int64_t nvalid_pts, int min_points,
-                           double min_eig_ratio, const int* bits, double* mean, double* icov, double* cov,
+int launch_voxel_stats_ndt(const float4* pts, const uint64_t* sorted_keys, const uint32_t* seg_start, int64_t nseg,
+                           int64_t nvalid_pts, int min_points, double min_eig_ratio, double* mean, double* icov,
                            int32_t* count, uint32_t* valid, uint64_t* vkey, hipStream_t stream) {
-    (void)bits;
-    hipLaunchKernelGGL(k_voxel_stats_ndt, dim3(grid_for(nseg, 128)), dim3(128), 0, stream, pts, sorted_idx,
-                       sorted_keys, seg_start, nseg, nvalid_pts, min_points, min_eig_ratio, mean, icov, cov, count,
-                       valid, vkey);
+    hipLaunchKernelGGL(k_voxel_stats_ndt, dim3(grid_for(nseg, 128)), dim3(128), 0, stream, pts, sorted_keys, seg_start,
+                       nseg, nvalid_pts, min_points, min_eig_ratio, mean, icov, count, valid, vkey);
     return (int)hipGetLastError();
 }
 

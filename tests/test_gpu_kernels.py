@@ -112,3 +112,29 @@ def test_scan_order(A, ctx, scene, counts):
     if max(counts) >= 1023:
         # reversed input: ties come out the other way round, so the sums round otherwise
         assert got != bits([np.ascontiguousarray(s[::-1]) for s in ordered])
+
+
+@pytest.mark.parametrize("n,extent", [(1, 1.0), (63, 3.0), (1023, 9.0), (1024, 9.0), (1025, 9.0), (4097, 30.0), (262144, 60.0),
+                                      (262145, 60.0), (300001, 2e6)])
+def test_map_sort(A, ctx, n, extent):
+    """Maps whose cell keys take one to four sorting passes (extents of 1 m to 2,000 km),
+    of sizes around the tiles of both widths, a tenth of the points without a cell: every
+    voxel's cell and count exactly, its mean as a sequential float64 sum in input order
+    (the device adds in the same order: only the division may round differently)."""
+    rng = np.random.default_rng(n)
+    pts = rng.uniform(0, extent, (n, 3)).astype(np.float32)
+    pts[:, 2] = rng.uniform(-1, 1, n) * min(extent, 3.0)
+    if n > 20:
+        pts[rng.integers(n, size=n // 10), rng.integers(3, size=n // 10)] = np.nan
+        pts[rng.integers(n, size=3), 0] = np.inf
+    grid = A.Grid(ctx, np.c_[pts, np.ones(n, np.float32)], A.params(A.NDT_MODE_NDT))
+    v = grid.voxels()
+    ok = np.isfinite(pts).all(1)
+    cell = np.floor(pts[ok].astype(np.float64)).astype(np.int64)
+    keys, inv, cnt = np.unique(cell[:, ::-1], axis=0, return_inverse=True, return_counts=True)
+    inv = inv.reshape(-1)
+    assert np.array_equal(v["key"], keys[:, ::-1]) and np.array_equal(v["n"], cnt)
+    for k in range(3):
+        s = np.zeros(len(keys))
+        np.add.at(s, inv, pts[ok, k].astype(np.float64))
+        assert np.abs(v["mean"][:, k] - s / cnt).max() <= 2.0 ** -52 * extent
