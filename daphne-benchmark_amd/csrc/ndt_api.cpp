@@ -420,22 +420,41 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, starts, sc2, &nvox, &nvalid_pts);
     if (e) return e;
     if (nvox == 0) return fail(NDT_ERR_INVALID, "map has no finite points");
+    /* dense query-cell index when the map's cell box is at most 2^28 cells; the
+     * environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
+     * index, so that tests run that path on maps of every size */
+    const double box = (double)g->dims[0] * (double)g->dims[1] * (double)g->dims[2];
+    const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
+    const bool dense = box <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
+    int32_t tiles[2] = {0, 0};
+    int64_t ncells = 0;
+    if (dense) {
+        tiles[0] = (g->dims[0] + 3) / 4;
+        tiles[1] = (g->dims[1] + 3) / 4;
+        ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
+    }
+    const int flog2 = std::max(4, ceil_log2(2 * nvox));
+    {
+        DevLayout l;
+        l.add(g->fit_pts, sizeof(float4) * (size_t)std::max<int64_t>(nvalid_pts, 1));
+        l.add(g->all_mean, sizeof(double) * 3 * nvox);
+        l.add(g->all_icov, sizeof(double) * 9 * nvox);
+        l.add(g->all_count, sizeof(int32_t) * nvox);
+        l.add(g->all_valid, sizeof(uint32_t) * (nvox + 1));
+        l.add(g->all_key, sizeof(uint64_t) * nvox);
+        l.add(g->fit_slots, sizeof(HashSlot) << flog2);
+        if (dense) l.add(g->dense, sizeof(uint32_t) * (size_t)(ncells + 1));
+        e = l.place(g->voxel_mem);
+        if (e) return e;
+    }
     /* map points sorted by voxel: for the statistics, and with a hash of the occupied
      * voxels for nearest-point queries (fitness score) */
-    BUF_TRY(g->fit_pts, sizeof(float4) * (size_t)std::max<int64_t>(nvalid_pts, 1));
     LAUNCH_TRY(launch_gather_points(c->pts.as<float4>(), vals.as<uint32_t>(), nvalid_pts, g->fit_pts.as<float4>(),
                                     c->stream));
-    BUF_TRY(g->all_mean, sizeof(double) * 3 * nvox);
-    BUF_TRY(g->all_icov, sizeof(double) * 9 * nvox);
-    BUF_TRY(g->all_count, sizeof(int32_t) * nvox);
-    BUF_TRY(g->all_valid, sizeof(uint32_t) * (nvox + 1));
-    BUF_TRY(g->all_key, sizeof(uint64_t) * nvox);
     LAUNCH_TRY(launch_voxel_stats_ndt(g->fit_pts.as<float4>(), keys.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts,
                                       g->params.min_points, g->params.min_eig_ratio, g->all_mean.as<double>(),
                                       g->all_icov.as<double>(), g->all_count.as<int32_t>(), g->all_valid.as<uint32_t>(),
                                       g->all_key.as<uint64_t>(), c->stream));
-    const int flog2 = std::max(4, ceil_log2(2 * nvox));
-    BUF_TRY(g->fit_slots, sizeof(HashSlot) << flog2);
     LAUNCH_TRY(launch_hash_clear(g->fit_slots.as<HashSlot>(), 1ll << flog2, c->stream));
     LAUNCH_TRY(launch_hash_insert(keys.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts, 0,
                                   g->fit_slots.as<HashSlot>(), flog2, c->stream));
@@ -449,19 +468,8 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     g->fdev.resolution = res;
     g->info.map_points = m;
     g->info.voxels = nvox;
-    /* dense query-cell index when the map's cell box is at most 2^28 cells; the
-     * environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
-     * index, so that tests run that path on maps of every size */
-    const double box = (double)g->dims[0] * (double)g->dims[1] * (double)g->dims[2];
-    const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
-    const bool dense = box <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
     int64_t nv = 0, ne = 0, nq = 0;
-    int32_t tiles[2] = {0, 0};
     if (dense) {
-        tiles[0] = (g->dims[0] + 3) / 4;
-        tiles[1] = (g->dims[1] + 3) / 4;
-        const int64_t ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
-        BUF_TRY(g->dense, sizeof(uint32_t) * (size_t)(ncells + 1));
         BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)ncells);
         BUF_TRY(c->bk_vid, sizeof(uint32_t) * (size_t)ncells);
         BUF_TRY(scratch, cells_scratch_bytes(ncells));
@@ -516,9 +524,15 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     g->info.valid_voxels = nv;
     const int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nq, 1)));
     const int64_t cap = 1ll << log2cap;
-    BUF_TRY(g->cand_head, sizeof(float4) * (ne + 1));
-    BUF_TRY(g->cand_s32, 2 * sizeof(float4) * (ne + 1));
-    BUF_TRY(g->vs64, VS64_STRIDE * sizeof(double2) * (nv + 1));
+    {
+        DevLayout l;
+        l.add(g->cand_head, sizeof(float4) * (ne + 1));
+        l.add(g->cand_s32, 2 * sizeof(float4) * (ne + 1));
+        l.add(g->vs64, VS64_STRIDE * sizeof(double2) * (nv + 1));
+        if (!dense) l.add(g->slots, sizeof(HashSlot) * cap);
+        e = l.place(g->cand_mem);
+        if (e) return e;
+    }
     if (dense) {
         LAUNCH_TRY(launch_cells_fill(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), g->all_mean.as<double>(),
                                      g->all_icov.as<double>(), nvox, g->bits, g->origin_cell, res, tiles,
@@ -526,7 +540,6 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
                                      g->cand_head.as<float4>(), g->cand_s32.as<float4>(), g->vs64.as<double2>(),
                                      c->stream));
     } else {
-        BUF_TRY(g->slots, sizeof(HashSlot) * cap);
         LAUNCH_TRY(launch_hash_clear(g->slots.as<HashSlot>(), cap, c->stream));
         LAUNCH_TRY(launch_voxel_s64(g->mean_c.as<double>(), g->icov_c.as<double>(), nv, g->vs64.as<double2>(), c->stream));
         if (nq > 0) {
@@ -614,17 +627,22 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
     int64_t nvox = 0, inside = 0;
     e = sorted_runs(c, keys.as<uint64_t>(), m, 0, (uint64_t)ncells, starts, sc2, &nvox, &inside);
     if (e) return e;
-    BUF_TRY(g->all_mean, sizeof(double) * 3 * nvox);
-    BUF_TRY(g->all_icov, sizeof(double) * 9 * nvox);
-    BUF_TRY(g->all_count, sizeof(int32_t) * nvox);
-    BUF_TRY(g->all_key, sizeof(uint64_t) * nvox);
+    const int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nvox, 1)));
+    const int64_t cap = 1ll << log2cap;
+    {
+        DevLayout l;
+        l.add(g->all_mean, sizeof(double) * 3 * nvox);
+        l.add(g->all_icov, sizeof(double) * 9 * nvox);
+        l.add(g->all_count, sizeof(int32_t) * nvox);
+        l.add(g->all_key, sizeof(uint64_t) * nvox);
+        l.add(g->slots, sizeof(HashSlot) * cap);
+        e = l.place(g->voxel_mem);
+        if (e) return e;
+    }
     LAUNCH_TRY(launch_voxel_stats_compat(c->pts.as<float4>(), vals.as<uint32_t>(), keys.as<uint64_t>(),
                                          starts.as<uint32_t>(), nvox, m, (double)(size_t)ncells, g->all_mean.as<double>(),
                                          g->all_icov.as<double>(), g->all_count.as<int32_t>(), g->all_key.as<uint64_t>(),
                                          c->stream));
-    int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nvox, 1)));
-    int64_t cap = 1ll << log2cap;
-    BUF_TRY(g->slots, sizeof(HashSlot) * cap);
     LAUNCH_TRY(launch_hash_clear(g->slots.as<HashSlot>(), cap, c->stream));
     LAUNCH_TRY(launch_hash_insert_ids(g->all_key.as<uint64_t>(), nvox, g->slots.as<HashSlot>(), log2cap, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
