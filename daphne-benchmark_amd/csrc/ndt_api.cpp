@@ -433,6 +433,9 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         tiles[1] = (g->dims[1] + 3) / 4;
         ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
     }
+    /* nearest-point queries: the first point of every cell of the box where that takes no
+     * more memory than the hash of the occupied voxels (32 to 64 bytes each) */
+    const bool rows = dense && box <= 16.0 * (double)nvox;
     const int flog2 = std::max(4, ceil_log2(2 * nvox));
     {
         DevLayout l;
@@ -442,7 +445,8 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         l.add(g->all_count, sizeof(int32_t) * nvox);
         l.add(g->all_valid, sizeof(uint32_t) * (nvox + 1));
         l.add(g->all_key, sizeof(uint64_t) * nvox);
-        l.add(g->fit_slots, sizeof(HashSlot) << flog2);
+        if (rows) l.add(g->fit_begin, sizeof(uint32_t) * ((size_t)box + 1));
+        else l.add(g->fit_slots, sizeof(HashSlot) << flog2);
         if (dense) l.add(g->dense, sizeof(uint32_t) * (size_t)(ncells + 1));
         e = l.place(g->voxel_mem);
         if (e) return e;
@@ -455,14 +459,21 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
                                       g->params.min_points, g->params.min_eig_ratio, g->all_mean.as<double>(),
                                       g->all_icov.as<double>(), g->all_count.as<int32_t>(), g->all_valid.as<uint32_t>(),
                                       g->all_key.as<uint64_t>(), c->stream));
-    LAUNCH_TRY(launch_hash_clear(g->fit_slots.as<HashSlot>(), 1ll << flog2, c->stream));
-    LAUNCH_TRY(launch_hash_insert(keys.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts, 0,
-                                  g->fit_slots.as<HashSlot>(), flog2, c->stream));
+    if (rows) {
+        LAUNCH_TRY(launch_fit_rows(g->all_key.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts, g->bits,
+                                   g->dims, g->fit_begin.as<uint32_t>(), c->stream));
+    } else {
+        LAUNCH_TRY(launch_hash_clear(g->fit_slots.as<HashSlot>(), 1ll << flog2, c->stream));
+        LAUNCH_TRY(launch_hash_insert(keys.as<uint64_t>(), starts.as<uint32_t>(), nvox, nvalid_pts, 0,
+                                      g->fit_slots.as<HashSlot>(), flog2, c->stream));
+    }
+    g->fdev.begin = g->fit_begin.as<uint32_t>();
     g->fdev.slots = g->fit_slots.as<HashSlot>();
     g->fdev.pts = g->fit_pts.as<float4>();
     g->fdev.log2cap = flog2;
     for (int k = 0; k < 3; k++) {
         g->fdev.bits[k] = g->bits[k];
+        g->fdev.dims[k] = g->dims[k];
         g->fdev.origin_cell[k] = g->origin_cell[k];
     }
     g->fdev.resolution = res;

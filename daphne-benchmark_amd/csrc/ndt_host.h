@@ -103,8 +103,12 @@ struct DevLayout {
         offsets[n++] = bytes;
         bytes += (want + 255) & ~(size_t)255;
     }
+    /* The runtime keeps freed memory for requests of the same size: from 1 MB on, sizes are
+     * multiples of 4 MB, so that maps of about the same size find each other's (three maps
+     * of 100 k points in turn: 0.43 ms each against 0.74). */
     int place(DevBuf& buf) {
-        const int e = buf.ensure(bytes);
+        const size_t unit = (size_t)4 << 20;
+        const int e = buf.ensure(bytes < (unit >> 2) ? bytes : (bytes + unit - 1) / unit * unit);
         for (int k = 0; k < n; k++) views[k]->p = e ? nullptr : buf.as<char>() + offsets[k];
         return e;
     }
@@ -216,9 +220,10 @@ struct ndt_grid {
     ndt::DevView slots, dense, cand_head, cand_s32, vs64;
     DevBuf mean_c, icov_c; /* hashed index */
     int32_t dims[3] = {0, 0, 0};
-    /* map points sorted by voxel + occupied-voxel hash (fitness score) */
+    /* map points sorted by voxel and where each cell's start, or an occupied-voxel hash
+     * (fitness score) */
     ndt::FitGridDev fdev;
-    ndt::DevView fit_pts, fit_slots;
+    ndt::DevView fit_pts, fit_begin, fit_slots;
     /* all occupied voxels (diagnostics) */
     ndt::DevView all_mean, all_icov, all_count, all_valid, all_key;
     /* compat */

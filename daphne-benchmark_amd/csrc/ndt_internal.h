@@ -269,6 +269,8 @@ struct NdtGridDev {
 /* Device view of the map points of an ndt grid, sorted by voxel, for nearest-point
  * queries (fitness score). */
 struct FitGridDev {
+    const uint32_t* begin;   /* first sorted point of every cell of the map's box (x first, one more), or null: */
+    int32_t dims[3];         /* the box */
     const HashSlot* slots;   /* occupied voxel -> range of sorted points */
     const float4* pts;       /* map points sorted by voxel key */
     int log2cap;
@@ -516,6 +518,8 @@ int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double*
                       const uint32_t* begin, const uint32_t* vid, float4* head, float4* s32, double2* vs64,
                       hipStream_t stream);
 int launch_gather_points(const float4* pts, const uint32_t* idx, int64_t n, float4* out, hipStream_t stream);
+int launch_fit_rows(const uint64_t* vkey, const uint32_t* starts, int64_t nvox, int64_t npts, const int* bits,
+                    const int32_t* dims, uint32_t* begin, hipStream_t stream);
 int launch_fitness(FitGridDev fg, const float4* pts, const int64_t* offsets, const int32_t* counts, int32_t S,
                    const double* poses, double max_d2, int shells, int nblk, double* partials, hipStream_t stream);
 int launch_init_queue(const ScanDesc* scans, int32_t S, uint64_t total_chunks, WorkQueue* q, uint64_t* items,

@@ -138,3 +138,38 @@ def test_map_sort(A, ctx, n, extent):
         s = np.zeros(len(keys))
         np.add.at(s, inv, pts[ok, k].astype(np.float64))
         assert np.abs(v["mean"][:, k] - s / cnt).max() <= 2.0 ** -52 * extent
+
+
+@pytest.mark.parametrize("box", [(1, 1, 1), (3, 2, 1), (9, 7, 4), (40, 33, 5)])
+@pytest.mark.parametrize("res", [1.0, 0.7])
+def test_fitness_rows_match_hashed(A, orc, ctx, box, res):
+    """Nearest map points by runs of cells against the hashed search and the oracle's
+    brute force: scan points on the map, on cell faces, several cells outside the box
+    (more than one shell), beyond the search's reach and not finite, with and without a
+    range limit.  The two searches take the minimum of the same distances: same bits."""
+    rng = np.random.default_rng(sum(box))
+    cells = np.stack(np.meshgrid(*[np.arange(b) for b in box], indexing="ij"), -1).reshape(-1, 3) - np.array([2, 1, 3])
+    cells = cells[rng.random(len(cells)) < 0.5] if len(cells) > 8 else cells
+    pts = (cells[:, None, :] + rng.uniform(0.001, 0.999, (len(cells), 4, 3))).reshape(-1, 3) * res
+    mp = np.c_[pts, np.ones(len(pts))].astype(np.float32)
+    prm = A.params(A.NDT_MODE_NDT, resolution=res)
+    rows, hashed = A.Grid(ctx, mp, prm), _hashed(A, ctx, mp, prm)
+    lo, hi = pts.min(0), pts.max(0)
+    near = rng.uniform(lo - 0.5, hi + 0.5, (300, 3))
+    face = np.round(rng.uniform(lo, hi, (64, 3)) / res) * res
+    out = rng.uniform(lo - 5 * res, hi + 5 * res, (60, 3))
+    far = np.array([[1e4, 0, 0], [0, 0, -40 * res + lo[2]], [0, 3e9, 0]])
+    scan = np.r_[pts[:100] + 0.01, near, face, out, far]
+    finite = np.c_[scan, np.ones(len(scan))].astype(np.float32)
+    dirty = finite.copy()
+    dirty[::50, 1] = np.nan
+    sc = A.Scans(ctx, [finite, dirty, finite[:1]])
+    poses = np.stack([np.eye(4)] * 3)
+    poses[1, :3, 3] = 0.01, -0.02, 0.03
+    for limit in (0.0, 0.3, 2.5):
+        a, na = sc.fitness(rows, poses, limit)
+        b, nb = sc.fitness(hashed, poses, limit)
+        assert np.array_equal(na, nb) and np.array_equal(a, b)
+        if limit:
+            want, n = orc.fitness_score(mp, finite, poses[0], limit)
+            assert na[0] == n and (n == 0 or abs(a[0] - want) <= 1e-12 * want)
