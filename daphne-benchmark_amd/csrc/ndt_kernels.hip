@@ -2115,69 +2115,87 @@ __device__ inline void block_reduce_acc(double* vals /* NRED per thread, registe
 }
 
 /* ------------------------------------------------------------------ the Newton / line-search controller
- * Runs on one thread of the workgroup that completes a scan's pass.  Consumes the
- * 28 sums of the pass just evaluated at st.x_t and either chooses the next pose
- * to evaluate or finishes the scan.  Same semantics as computeTransformation /
- * computeStepLengthMT (src/CPU/ndt_mapping/kernel.cpp:1015-1144, :1175-1272) in
- * their textbook form (line search live, translation updated, true convergence). */
+ * Runs on the first wave of the workgroup that completes a scan's pass: every lane
+ * makes the same decisions on the same state in LDS (scalars are stored by all of them,
+ * with the same value), vectors are handled by a lane per entry.  Consumes the 28 sums of
+ * the pass just evaluated at st.x_t and either chooses the next pose to evaluate or
+ * finishes the scan.  Same semantics as computeTransformation / computeStepLengthMT
+ * (src/CPU/ndt_mapping/kernel.cpp:1015-1144, :1175-1272) in their textbook form (line
+ * search live, translation updated, true convergence).
+ * Between two passes of a scan this is on its critical path, a chain of dependent float64
+ * operations that no other work hides.  On a lone scan of 2 k points (17 passes of 22 us)
+ * it took 7.3 us a pass on one lane, 5.5 with the system at a lane per entry and rolled
+ * loops, and 4.1 as it is; the pass parameters after it 1.7 us, and 1.2 since the launch's
+ * parameters are read from LDS. */
 
-/* Gaussian elimination with partial pivoting (rows of A and b swapped together),
- * unrolled so that the system stays in registers.  Same arithmetic as the
- * reference's solve (kernel.cpp:293-343) apart from the right-hand-side swap,
- * which the reference omits. */
-__device__ inline void solve6_pivot(double* result, const double* Ain, const double* bin) {
-    double A[6][6], b[6];
+__device__ inline double lane_value(double v, int lane) {
+    const uint64_t b = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+    return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+/* orders the wave's LDS accesses for the compiler (the hardware keeps them in order) */
+__device__ inline void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+/* ((((v0 + v1) + v2) + v3) + v4) + v5 of the first six lanes, on every lane */
+__device__ inline double sum_lanes6(double v) {
+    double s = lane_value(v, 0);
 #pragma unroll
-    for (int i = 0; i < 6; i++) {
-        b[i] = bin[i];
+    for (int k = 1; k < 6; k++) s = s + lane_value(v, k);
+    return s;
+}
+
+/* The Newton step: solves H x = -grad by Gaussian elimination with partial pivoting (rows
+ * of H and the right-hand side swapped together), with the arithmetic of the reference's
+ * solve (kernel.cpp:293-343) apart from the right-hand-side swap, which the reference
+ * omits.  All lanes of a wave call it: lane i < 6 holds row i, so that a column's
+ * quotients are made at once and a row's entries follow each other without waiting; the
+ * pivot row comes through lane reads.  The back substitution is the same on all lanes. */
+__device__ inline void wave_solve6(double* x, const double* hess /* upper triangle */, const double* grad) {
+    const int lane = threadIdx.x % WAVE, i = min(lane, 5);
+    double row[7];
 #pragma unroll
-        for (int k = 0; k < 6; k++) A[i][k] = Ain[i * 6 + k];
-    }
+    for (int k = 0; k < 6; k++) row[k] = hess[i <= k ? tri_index(i, k) : tri_index(k, i)];
+    row[6] = -grad[i];
 #pragma unroll
     for (int j = 0; j < 6; j++) {
-        double mx = fabs(A[j][j]);
+        double mx = fabs(lane_value(row[j], j));
         int mi = j;
 #pragma unroll
-        for (int i = j + 1; i < 6; i++) {
-            double v = fabs(A[i][j]);
+        for (int r = j + 1; r < 6; r++) {
+            const double v = fabs(lane_value(row[j], r));
             if (v > mx) {
-                mi = i;
+                mi = r;
                 mx = v;
             }
         }
+        if (mi != j) {
+            const int from = (lane == j ? mi : lane == mi ? j : lane) * 4;
 #pragma unroll
-        for (int i = j + 1; i < 6; i++) {
-            const bool sw = (mi == i);
-#pragma unroll
-            for (int k = 0; k < 6; k++) {
-                double t = A[i][k];
-                A[i][k] = sw ? A[j][k] : t;
-                A[j][k] = sw ? t : A[j][k];
-            }
-            double t = b[i];
-            b[i] = sw ? b[j] : t;
-            b[j] = sw ? t : b[j];
+            for (int k = j; k < 7; k++) row[k] = bperm_f64(from, row[k]);
         }
-        if (mx == 0.0) A[j][j] = 0.001;
+        if (mx == 0.0 && lane == j) row[j] = 0.001;
+        if (j < 5) {
+            const double pivot = row[j] / lane_value(row[j], j);
 #pragma unroll
-        for (int i = j + 1; i < 6; i++) {
-            double pivot = A[i][j] / A[j][j];
-#pragma unroll
-            for (int k = 0; k < 6; k++) A[i][k] = A[i][k] - pivot * A[j][k];
-            b[i] = b[i] - pivot * b[j];
+            for (int k = j + 1; k < 7; k++) {
+                const double next = row[k] - pivot * lane_value(row[k], j);
+                if (lane > j) row[k] = next;
+            }
         }
     }
-    double r[6];
-    r[5] = b[5] / A[5][5];
 #pragma unroll
-    for (int i = 4; i >= 0; i--) {
+    for (int q = 5; q >= 0; q--) {
         double sum = 0.0;
 #pragma unroll
-        for (int j = i + 1; j < 6; j++) sum = sum + A[i][j] * r[j];
-        r[i] = (b[i] - sum) / A[i][i];
+        for (int j = q + 1; j < 6; j++) sum = sum + lane_value(row[j], q) * x[j];
+        x[q] = (lane_value(row[6], q) - sum) / lane_value(row[q], q);
     }
-#pragma unroll
-    for (int i = 0; i < 6; i++) result[i] = r[i];
 }
 
 __device__ __attribute__((noinline)) void ctl_finish(ScanState& st, const AlignParams& prm, int converged, ScanOut* out) {
@@ -2189,10 +2207,9 @@ __device__ __attribute__((noinline)) void ctl_finish(ScanState& st, const AlignP
     M[3] += prm.origin[0];
     M[7] += prm.origin[1];
     M[11] += prm.origin[2];
-    for (int k = 0; k < 16; k++) {
-        st.final_m[k] = M[k];
-        out->final_m[k] = M[k];
-    }
+    for (int k = 0; k < 16; k++) st.final_m[k] = M[k];
+    if (threadIdx.x % WAVE) return;
+    for (int k = 0; k < 16; k++) out->final_m[k] = M[k];
     out->score = st.score;
     out->iterations = st.iter;
     out->converged = converged;
@@ -2207,18 +2224,20 @@ __device__ __attribute__((noinline)) void ctl_finish(ScanState& st, const AlignP
  * score, gradient and Hessian, and its later passes are numbered (and chunked) as
  * those of a launch of its own. */
 __device__ inline void ctl_fallback(ScanState& st) {
+    const int lane = threadIdx.x % WAVE;
     st.fb_stage = FB_FALLBACK;
     st.used_alt = 0;
     st.iter = 0;
     st.converged = 0;
-    for (int k = 0; k < 6; k++) {
-        st.x_t[k] = st.alt[k];
-        st.p[k] = st.alt[k];
-    }
     st.score = st.probe_score;
-    for (int i = 0; i < 6; i++) st.grad[i] = st.probe_d[i];
-    for (int k = 0; k < 21; k++) st.hess[k] = st.probe_d[6 + k];
+    if (lane < 6) {
+        st.x_t[lane] = st.alt[lane];
+        st.p[lane] = st.alt[lane];
+        st.grad[lane] = st.probe_d[lane];
+    }
+    if (lane < 21) st.hess[lane] = st.probe_d[6 + lane];
     st.run_base = st.passes - 1;
+    wave_order();
 }
 
 /* The end of a run.  In a launch with refined starts, a run from the refined guess
@@ -2238,172 +2257,200 @@ __device__ inline int ctl_end(ScanState& st, const AlignParams& prm, int converg
     return 0;
 }
 
-__device__ __attribute__((noinline)) void ctl_newton_start(ScanState& __restrict__ st, const AlignParams& __restrict__ prm,
-                                                           ScanOut* __restrict__ out) {
+/* Starts a Newton iteration from the state, or ends the run: `end` >= 0 is a run that has
+ * just ended, with that for `converged`. */
+__device__ inline void ctl_newton_start(ScanState& st, const AlignParams& prm, int end, ScanOut* out) {
     const double mu = 1.e-4;
-    for (;;) {
-        if (st.iter >= prm.max_iterations) {
-            if (ctl_end(st, prm, 0, out)) continue;
-            return;
-        }
-        double H[36], ng[6], delta[6];
-        for (int i = 0; i < 6; i++) {
-            ng[i] = -st.grad[i];
-            for (int j = 0; j < 6; j++) H[i * 6 + j] = st.hess[i <= j ? tri_index(i, j) : tri_index(j, i)];
-        }
-        solve6_pivot(delta, H, ng);
-        double norm = sqrt(delta[0] * delta[0] + delta[1] * delta[1] + delta[2] * delta[2] + delta[3] * delta[3] +
-                           delta[4] * delta[4] + delta[5] * delta[5]);
-        if (norm == 0 || norm != norm) {
-            if (ctl_end(st, prm, norm == norm, out)) continue;
-            return;
-        }
-        for (int i = 0; i < 6; i++) st.dir[i] = delta[i] / norm;
-        st.phi_0 = -st.score;
-        st.d_phi_0 = -dot6(st.grad, st.dir);
-        if (st.d_phi_0 >= 0) {
-            if (st.d_phi_0 == 0) {
-                /* no descent direction: zero step */
-                st.iter++;
-                if (st.iter > 1 && 0.0 < prm.trans_eps) {
-                    if (ctl_end(st, prm, 1, out)) continue;
-                    return;
+    const int lane = threadIdx.x % WAVE;
+#pragma unroll 1
+    for (;; end = -1) {
+        if (end < 0 && st.iter >= prm.max_iterations) end = 0;
+        double norm = 0.0, dir = 0.0, d_phi_0 = 0.0;
+        if (end < 0) {
+            double x[6];
+            wave_solve6(x, st.hess, st.grad);
+            norm = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3] + x[4] * x[4] + x[5] * x[5]);
+            double delta = x[5];
+#pragma unroll
+            for (int k = 0; k < 5; k++) delta = lane == k ? x[k] : delta;
+            if (norm == 0 || norm != norm) {
+                end = norm == norm;
+            } else {
+                dir = delta / norm;
+                d_phi_0 = -sum_lanes6((lane < 6 ? st.grad[lane] : 0.0) * dir);
+                if (d_phi_0 == 0) {
+                    /* no descent direction: zero step */
+                    const int iter = st.iter + 1;
+                    st.iter = iter;
+                    if (!(iter > 1 && 0.0 < prm.trans_eps)) continue;
+                    end = 1;
                 }
-                continue;
             }
-            st.d_phi_0 *= -1;
-            for (int i = 0; i < 6; i++) st.dir[i] *= -1;
         }
-        st.a_l = 0;
-        st.a_u = 0;
-        st.f_l = psi_mt(st.a_l, st.phi_0, st.phi_0, st.d_phi_0, mu);
-        st.g_l = dpsi_mt(st.d_phi_0, st.d_phi_0, mu);
-        st.f_u = psi_mt(st.a_u, st.phi_0, st.phi_0, st.d_phi_0, mu);
-        st.g_u = dpsi_mt(st.d_phi_0, st.d_phi_0, mu);
-        st.interval_converged = 0;
-        st.open_interval = 1;
-        st.step_iterations = 0;
+        if (end >= 0) {
+            if (ctl_end(st, prm, end, out)) continue;
+            return;
+        }
+        if (d_phi_0 >= 0) {
+            d_phi_0 *= -1;
+            dir *= -1;
+        }
+        const double phi_0 = -st.score;
         double a_t = norm;
         a_t = dmin_std(a_t, prm.step_size);
         a_t = dmax_std(a_t, prm.trans_eps / 2);
+        if (lane < 6) {
+            st.dir[lane] = dir;
+            st.x_t[lane] = st.p[lane] + dir * a_t;
+        }
+        st.phi_0 = phi_0;
+        st.d_phi_0 = d_phi_0;
+        st.a_l = 0;
+        st.a_u = 0;
+        const double f = psi_mt(0.0, phi_0, phi_0, d_phi_0, mu), g = dpsi_mt(d_phi_0, d_phi_0, mu);
+        st.f_l = f;
+        st.g_l = g;
+        st.f_u = f;
+        st.g_u = g;
+        st.interval_converged = 0;
+        st.open_interval = 1;
+        st.step_iterations = 0;
         st.a_t = a_t;
-        for (int i = 0; i < 6; i++) st.x_t[i] = st.p[i] + st.dir[i] * a_t;
         st.phase = PH_MT_FIRST;
+        wave_order();
         return;
     }
 }
 
-/* accepts the line search's step x_t = p + a_t dir, whose score, gradient and
- * Hessian are in the state, and starts the next Newton iteration */
-__device__ inline void ctl_accept(ScanState& st, const AlignParams& prm, ScanOut* out) {
-    for (int i = 0; i < 6; i++) st.p[i] = st.p[i] + st.dir[i] * st.a_t;
-    st.iter++;
-    if (st.iter > 1 && fabs(st.a_t) < prm.trans_eps) {
-        if (!ctl_end(st, prm, 1, out)) return;
-    }
-    ctl_newton_start(st, prm, out);
-}
-
+/* One step of the controller; all lanes of the wave call it. */
 __device__ __attribute__((noinline)) void ctl_step(ScanState& __restrict__ st, const double* __restrict__ red,
                                                    const AlignParams& __restrict__ prm, ScanOut* __restrict__ out) {
     const double mu = 1.e-4, nu = 0.9;
-    st.passes++;
-    st.pairs += red[NACC];
-    if (st.phase == PH_PROBE) {
+    const int lane = threadIdx.x % WAVE;
+    const int phase = st.phase;
+    const int passes = st.passes + 1;
+    const double pairs = st.pairs + red[NACC];
+    wave_order();
+    st.passes = passes;
+    st.pairs = pairs;
+    if (phase == PH_PROBE) {
         /* the given guess's score and derivatives; the run starts at the refined
          * guess */
         st.probe_score = red[0];
-        for (int k = 0; k < 27; k++) st.probe_d[k] = red[1 + k];
-        for (int k = 0; k < 6; k++) {
-            const double given = st.x_t[k];
-            st.x_t[k] = st.alt[k];
-            st.p[k] = st.alt[k];
-            st.alt[k] = given;
+        if (lane < 27) st.probe_d[lane] = red[1 + lane];
+        if (lane < 6) {
+            const double given = st.x_t[lane], refined = st.alt[lane];
+            st.x_t[lane] = refined;
+            st.p[lane] = refined;
+            st.alt[lane] = given;
         }
         st.fb_stage = FB_REFINED;
         st.phase = PH_INIT;
-        st.run_base = st.passes;
+        st.run_base = passes;
+        wave_order();
         return;
     }
-    if (st.phase == PH_MT_HESS) {
+    /* the pass's score and gradient (and Hessian) become the state's, at x_t */
+    bool accept = true, take = true;
+    if (phase == PH_MT_HESS) {
         /* the Hessian at the accepted step of a line search whose loop ran
          * (computeHessian, kernel.cpp:1141-1142); score and gradient are the last
          * trial's */
-        for (int k = 0; k < 21; k++) st.hess[k] = red[7 + k];
-        ctl_accept(st, prm, out);
-        return;
-    }
-    if (st.phase == PH_INIT) {
+        take = false;
+    } else if (phase == PH_INIT) {
+        accept = false;
         if (st.fb_stage == FB_REFINED && red[0] < st.probe_score) {
             /* NDT scores the refined guess below the given one: the scan runs from
              * the given guess instead */
             ctl_fallback(st);
-            ctl_newton_start(st, prm, out);
+            ctl_newton_start(st, prm, -1, out);
             return;
         }
-        st.score = red[0];
-        for (int i = 0; i < 6; i++) st.grad[i] = red[1 + i];
-        for (int k = 0; k < 21; k++) st.hess[k] = red[7 + k];
-        for (int i = 0; i < 6; i++) st.p[i] = st.x_t[i];
-        ctl_newton_start(st, prm, out);
-        return;
-    }
-    /* a line-search evaluation at x_t = p + a_t dir */
-    const bool red_has_hess = !(prm.hess_at_accept && st.phase == PH_MT_LOOP);
-    double g_t[6];
-    for (int i = 0; i < 6; i++) g_t[i] = red[1 + i];
-    const double phi_t = -red[0];
-    const double d_phi_t = -dot6(g_t, st.dir);
-    const double psi_t = psi_mt(st.a_t, phi_t, st.phi_0, st.d_phi_0, mu);
-    const double d_psi_t = dpsi_mt(d_phi_t, st.d_phi_0, mu);
-    /* A trial at the step of the trial before it (the trial value clamped to the
-     * same bound again) is at the same pose, whose pass would reproduce `red` bit
-     * for bit: the search takes `red` again without a pass, for as long as it
-     * repeats the step. */
-    for (;;) {
-        if (st.phase == PH_MT_LOOP) {
-            if (st.open_interval && (psi_t <= 0 && d_psi_t >= 0)) {
-                st.open_interval = 0;
-                st.f_l = st.f_l + st.phi_0 - mu * st.d_phi_0 * st.a_l;
-                st.g_l = st.g_l + mu * st.d_phi_0;
-                st.f_u = st.f_u + st.phi_0 - mu * st.d_phi_0 * st.a_u;
-                st.g_u = st.g_u + mu * st.d_phi_0;
+        if (lane < 6) st.p[lane] = st.x_t[lane];
+    } else {
+        /* a line-search evaluation at x_t = p + a_t dir */
+        const bool red_has_hess = !(prm.hess_at_accept && phase == PH_MT_LOOP);
+        const double phi_t = -red[0];
+        const double d_phi_t = -sum_lanes6(lane < 6 ? red[1 + lane] * st.dir[lane] : 0.0);
+        const double phi_0 = st.phi_0, d_phi_0 = st.d_phi_0;
+        const double psi_t = psi_mt(st.a_t, phi_t, phi_0, d_phi_0, mu);
+        const double d_psi_t = dpsi_mt(d_phi_t, d_phi_0, mu);
+        /* A trial at the step of the trial before it (the trial value clamped to the
+         * same bound again) is at the same pose, whose pass would reproduce `red` bit
+         * for bit: the search takes `red` again without a pass, for as long as it
+         * repeats the step. */
+        double a_l = st.a_l, f_l = st.f_l, g_l = st.g_l, a_u = st.a_u, f_u = st.f_u, g_u = st.g_u;
+        const double a_t = st.a_t;
+        int open = st.open_interval, converged = st.interval_converged, steps = st.step_iterations;
+        bool loop = phase == PH_MT_LOOP;
+        double a_next = a_t;
+#pragma unroll 1
+        for (;;) {
+            if (loop) {
+                if (open && (psi_t <= 0 && d_psi_t >= 0)) {
+                    open = 0;
+                    f_l = f_l + phi_0 - mu * d_phi_0 * a_l;
+                    g_l = g_l + mu * d_phi_0;
+                    f_u = f_u + phi_0 - mu * d_phi_0 * a_u;
+                    g_u = g_u + mu * d_phi_0;
+                }
+                converged = mt_update_interval(a_l, f_l, g_l, a_u, f_u, g_u, a_t, open ? psi_t : phi_t,
+                                               open ? d_psi_t : d_phi_t);
+                steps++;
             }
-            if (st.open_interval)
-                st.interval_converged =
-                    mt_update_interval(st.a_l, st.f_l, st.g_l, st.a_u, st.f_u, st.g_u, st.a_t, psi_t, d_psi_t);
-            else
-                st.interval_converged =
-                    mt_update_interval(st.a_l, st.f_l, st.g_l, st.a_u, st.f_u, st.g_u, st.a_t, phi_t, d_phi_t);
-            st.step_iterations++;
+            if (converged || steps >= 10 || (psi_t <= 0 && d_phi_t <= -nu * d_phi_0)) break;
+            a_next = mt_trial_value(a_l, f_l, g_l, a_u, f_u, g_u, a_t, open ? psi_t : phi_t, open ? d_psi_t : d_phi_t);
+            a_next = dmin_std(a_next, prm.step_size);
+            a_next = dmax_std(a_next, prm.trans_eps / 2);
+            loop = true;
+            accept = a_next == a_t; /* otherwise another trial */
+            if (!accept) break;
         }
-        if (st.interval_converged || st.step_iterations >= 10 || (psi_t <= 0 && d_phi_t <= -nu * st.d_phi_0))
-            break;
-        double a_t;
-        if (st.open_interval)
-            a_t = mt_trial_value(st.a_l, st.f_l, st.g_l, st.a_u, st.f_u, st.g_u, st.a_t, psi_t, d_psi_t);
-        else
-            a_t = mt_trial_value(st.a_l, st.f_l, st.g_l, st.a_u, st.f_u, st.g_u, st.a_t, phi_t, d_phi_t);
-        a_t = dmin_std(a_t, prm.step_size);
-        a_t = dmax_std(a_t, prm.trans_eps / 2);
-        const bool repeat = a_t == st.a_t;
-        st.phase = PH_MT_LOOP;
-        if (repeat) continue;
-        st.a_t = a_t;
-        for (int i = 0; i < 6; i++) st.x_t[i] = st.p[i] + st.dir[i] * a_t;
-        return;
+        wave_order();
+        st.a_l = a_l;
+        st.f_l = f_l;
+        st.g_l = g_l;
+        st.a_u = a_u;
+        st.f_u = f_u;
+        st.g_u = g_u;
+        st.open_interval = open;
+        st.interval_converged = converged;
+        st.step_iterations = steps;
+        if (loop) st.phase = PH_MT_LOOP;
+        if (!accept) {
+            st.a_t = a_next;
+            if (lane < 6) st.x_t[lane] = st.p[lane] + st.dir[lane] * a_next;
+            wave_order();
+            return;
+        }
+        /* accept x_t: its pass supplies score and gradient, and the Hessian unless the
+         * loop's passes skipped it (then one more pass at x_t computes it, unless the
+         * pass in `red`, at the same pose, did) */
+        if (prm.hess_at_accept && loop && !red_has_hess) {
+            st.score = red[0];
+            if (lane < 6) st.grad[lane] = red[1 + lane];
+            st.phase = PH_MT_HESS;
+            wave_order();
+            return;
+        }
     }
-    /* accept x_t: its pass supplies score and gradient, and the Hessian unless the
-     * loop's passes skipped it (then one more pass at x_t computes it, unless the
-     * pass in `red`, at the same pose, did) */
-    st.score = red[0];
-    for (int i = 0; i < 6; i++) st.grad[i] = g_t[i];
-    if (prm.hess_at_accept && st.phase == PH_MT_LOOP && !red_has_hess) {
-        st.phase = PH_MT_HESS;
-        return;
+    if (take) {
+        st.score = red[0];
+        if (lane < 6) st.grad[lane] = red[1 + lane];
     }
-    for (int k = 0; k < 21; k++) st.hess[k] = red[7 + k];
-    ctl_accept(st, prm, out);
+    if (lane < 21) st.hess[lane] = red[7 + lane];
+    int end = -1;
+    if (accept) {
+        /* the line search's step; then the next Newton iteration */
+        const double a_t = st.a_t;
+        if (lane < 6) st.p[lane] = st.p[lane] + st.dir[lane] * a_t;
+        const int iter = st.iter + 1;
+        wave_order();
+        st.iter = iter;
+        if (iter > 1 && fabs(a_t) < prm.trans_eps) end = 1;
+    }
+    wave_order();
+    ctl_newton_start(st, prm, end, out);
 }
 
 /* pose parameters (x, y, z, roll, pitch, yaw) of a row-major world pose in the
@@ -2589,6 +2636,7 @@ __global__ __launch_bounds__(BLOCK, (sizeof(T) == 8 || SUM == NDT_SUM_FP64) ? AL
     __shared__ uint32_t s_prefix[MAX_BATCH + 1];
     __shared__ uint32_t lw[BLOCK / WAVE];
     __shared__ int s_nactive, s_pp_scan, s_flag, s_grad_only;
+    __shared__ AlignParams s_prm; /* the controller's copy */
     const int tid = threadIdx.x;
     const int wg = blockIdx.x;
     const int nwg = gridDim.x;
@@ -2596,6 +2644,7 @@ __global__ __launch_bounds__(BLOCK, (sizeof(T) == 8 || SUM == NDT_SUM_FP64) ? AL
     double prof[4] = {0, 0, 0, 0};
     bool ok = true;
     if (tid == 0) s_pp_scan = -1;
+    if (tid == 0) s_prm = prm;
     for (;;) {
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         /* active scans and their chunk counts, identical in every workgroup */
@@ -2677,9 +2726,9 @@ __global__ __launch_bounds__(BLOCK, (sizeof(T) == 8 || SUM == NDT_SUM_FP64) ? AL
             for (int q = tid; q < STATE_WORDS; q += BLOCK) sstate[q] = ld_agent_u64((const uint64_t*)(states + s) + q);
             __syncthreads();
             reduce_slots(partials, sd.chunk_base, pass_nchunks(sd, run_pass(*(ScanState*)sstate)), gred, red);
-            if (tid == 0) ctl_step(*(ScanState*)sstate, red, prm, out + s);
+            if (tid < WAVE) ctl_step(*(ScanState*)sstate, red, s_prm, out + s);
             __syncthreads();
-            if (tid < WAVE && !((ScanState*)sstate)->done) wave_pass_params(*(ScanState*)sstate, prm, s_trig);
+            if (tid < WAVE && !((ScanState*)sstate)->done) wave_pass_params(*(ScanState*)sstate, s_prm, s_trig);
             __syncthreads();
             for (int q = tid; q < STATE_WORDS; q += BLOCK) st_agent_u64((uint64_t*)(states + s) + q, sstate[q]);
             __syncthreads();
@@ -2817,10 +2866,12 @@ __global__ __launch_bounds__(BLOCK, (sizeof(T) == 8 || SUM == NDT_SUM_FP64) ? AL
     __shared__ uint32_t s_base;
     __shared__ int s_last, s_done, s_grad_only;
     __shared__ uint32_t s_run_base, s_next_rel;
+    __shared__ AlignParams s_prm; /* the controller's copy */
     const int tid = threadIdx.x;
     double prof[3] = {0, 0, 0};
     int ok = 1;
     if (tid == 0) s_ppkey = ~0ull;
+    if (tid == 0) s_prm = prm;
     for (;;) {
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         if (tid == 0) {
@@ -2893,30 +2944,37 @@ __global__ __launch_bounds__(BLOCK, (sizeof(T) == 8 || SUM == NDT_SUM_FP64) ? AL
         if (s_last) {
             /* every chunk of this pass is in: reduce in chunk order, G interleaved groups */
             if (tid == 0) __hip_atomic_store(&done_cnt[s], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            for (int w = tid; w < STATE_WORDS; w += BLOCK) sstate[w] = ld_agent_u64((const uint64_t*)(states + s) + w);
+            /* the state by the threads that do not load slots, in the same round trip */
+            constexpr int IDLE = BLOCK > SLOT_GROUPS * 32 ? SLOT_GROUPS * 32 : 0;
+            if (tid >= IDLE)
+                for (int w = tid - IDLE; w < STATE_WORDS; w += BLOCK - IDLE)
+                    sstate[w] = ld_agent_u64((const uint64_t*)(states + s) + w);
             reduce_slots(partials, sd.chunk_base, nck, gred, red);
-            if (tid == 0) {
+            if (tid < WAVE) {
                 ScanState& st = *(ScanState*)sstate;
-                ctl_step(st, red, prm, out + s);
+                ctl_step(st, red, s_prm, out + s);
                 if (!st.done && (uint64_t)pass + 1 >= (1ull << ITEM_PASS_BITS)) {
                     st.status = NDT_ERR_UNSUPPORTED;
-                    ctl_finish(st, prm, 0, out + s);
+                    ctl_finish(st, s_prm, 0, out + s);
                 }
                 s_done = st.done;
                 s_next_rel = run_pass(st);
             }
             __syncthreads();
-            if (tid < WAVE && !s_done) wave_pass_params(*(ScanState*)sstate, prm, s_trig);
+            if (!s_done) {
+                /* the queue positions of the next pass's chunks while its parameters are made
+                 * (a workgroup that claims one waits until its item is written) */
+                if (tid < WAVE) wave_pass_params(*(ScanState*)sstate, s_prm, s_trig);
+                else if (tid == WAVE)
+                    s_base = __hip_atomic_fetch_add(&q->tail, (uint32_t)pass_nchunks(sd, s_next_rel), __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+            }
             __syncthreads();
             for (int w = tid; w < STATE_WORDS; w += BLOCK) st_agent_u64((uint64_t*)(states + s) + w, sstate[w]);
             stores_complete();
             __syncthreads();
             if (!s_done) {
                 const int32_t nnext = pass_nchunks(sd, s_next_rel);
-                if (tid == 0)
-                    s_base = __hip_atomic_fetch_add(&q->tail, (uint32_t)nnext, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-                __syncthreads();
                 const uint64_t base = s_base;
                 if (base + (uint64_t)nnext > cap) {
                     if (tid == 0) __hip_atomic_store(&q->abort, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
