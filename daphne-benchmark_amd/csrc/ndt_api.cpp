@@ -278,26 +278,17 @@ static int pinned_stage(ndt_ctx* c, size_t bytes, char** p) {
     return 0;
 }
 
-/* Host-to-device copies (one or two) through the pinned staging buffer: a pageable
- * hipMemcpyAsync is staged by the runtime through buffers shared by every stream,
- * which serialises contexts that upload concurrently. */
-static int upload_staged2(ndt_ctx* c, void* d1, const void* s1, size_t b1, void* d2, const void* s2, size_t b2) {
-    const size_t off2 = (b1 + 255) & ~(size_t)255;
-    char* p = nullptr;
-    int e = pinned_stage(c, off2 + b2, &p);
-    if (e) return e;
-    std::memcpy(p, s1, b1);
-    c->pin_pending = true;
-    HIP_TRY(hipMemcpyAsync(d1, p, b1, hipMemcpyHostToDevice, c->stream));
-    if (b2) {
-        std::memcpy(p + off2, s2, b2);
-        HIP_TRY(hipMemcpyAsync(d2, p + off2, b2, hipMemcpyHostToDevice, c->stream));
-    }
-    return 0;
-}
-
+/* A host-to-device copy through the pinned staging buffer: a pageable hipMemcpyAsync is
+ * staged by the runtime through buffers shared by every stream, which serialises contexts
+ * that upload concurrently. */
 static int upload_staged(ndt_ctx* c, void* dst, const void* src, size_t bytes) {
-    return upload_staged2(c, dst, src, bytes, nullptr, nullptr, 0);
+    char* p = nullptr;
+    const int e = pinned_stage(c, bytes, &p);
+    if (e) return e;
+    std::memcpy(p, src, bytes);
+    c->pin_pending = true;
+    HIP_TRY(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, c->stream));
+    return 0;
 }
 
 /* Points of the concatenated arrays [p0, p1) to the staging buffer; false if `finite` is
@@ -811,20 +802,6 @@ static int results_from_out(const ScanOut* out, const int64_t* counts, int32_t S
     return 0;
 }
 
-/* Fills results from the device outputs of S scans in the context's buffers. */
-static int collect_results(ndt_ctx* c, const int64_t* counts, int32_t S, int aborted, ndt_result* results,
-                           int32_t* used_alt = nullptr) {
-    /* read back through the pinned staging buffer (stream order puts this copy
-     * after the uploads from it) */
-    const size_t bytes = sizeof(ScanOut) * (size_t)S;
-    int e = pinned_reserve(c, bytes);
-    if (e) return e;
-    HIP_TRY(hipMemcpyAsync(c->pin, c->out.p, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    c->pin_pending = false;
-    return results_from_out((const ScanOut*)c->pin, counts, S, aborted, c, results, used_alt);
-}
-
 /* Chunk descriptors of a batch: chunk size, count and first partial slot per scan. */
 static void make_descs(const int64_t* offsets, const int64_t* counts, int32_t S, const ndt_params* p,
                        std::vector<ScanDesc>& desc, int64_t* slots_out, int64_t* max_chunks_out,
@@ -890,24 +867,28 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     else LAUNCH_TRY(align_kernel_max_blocks(block, prm.point_fp64, prm.sum_mode, &bpc));
     if (bpc <= 0) return fail(NDT_ERR_UNSUPPORTED, "align kernel does not fit on a compute unit");
     const int32_t nwg = bpc * c->cus;
-    BUF_TRY(c->guesses, sizeof(double) * 16 * S * (alt ? 2 : 1));
+    /* descriptors, guesses and refined starts in one buffer, results and phase times in
+     * another: one copy each way */
+    const size_t desc_bytes = sizeof(ScanDesc) * (size_t)S, guess_bytes = sizeof(double) * 16 * (size_t)S;
+    const size_t out_bytes = sizeof(ScanOut) * (size_t)S;
+    BUF_TRY(c->desc, desc_bytes + guess_bytes * (alt ? 2 : 1));
     BUF_TRY(c->states, sizeof(ScanState) * S);
-    BUF_TRY(c->sync, sizeof(RoundSync) * ((S + MAX_BATCH_SCANS - 1) / MAX_BATCH_SCANS));
-    BUF_TRY(c->out, sizeof(ScanOut) * S);
-    BUF_TRY(c->desc, sizeof(ScanDesc) * S);
+    BUF_TRY(c->out, out_bytes + 8 * sizeof(double));
     BUF_TRY(c->partials, sizeof(double) * 32 * slots);
-    BUF_TRY(c->small, 64 * sizeof(double));
-    HIP_TRY(hipMemsetAsync(c->out.p, 0, sizeof(ScanOut) * S, c->stream));
     {
-        const int eu = upload_staged2(c, c->guesses.p, guesses, sizeof(double) * 16 * S, c->desc.p, desc.data(),
-                                      sizeof(ScanDesc) * S);
+        char* stage = nullptr;
+        const size_t bytes = desc_bytes + guess_bytes * (alt ? 2 : 1);
+        const int eu = pinned_stage(c, bytes, &stage);
         if (eu) return eu;
-        if (alt) {
-            const int ea = upload_staged(c, c->guesses.as<double>() + 16 * (size_t)S, alt, sizeof(double) * 16 * S);
-            if (ea) return ea;
-        }
+        std::memcpy(stage, desc.data(), desc_bytes);
+        std::memcpy(stage + desc_bytes, guesses, guess_bytes);
+        if (alt) std::memcpy(stage + desc_bytes + guess_bytes, alt, guess_bytes);
+        c->pin_pending = true;
+        HIP_TRY(hipMemcpyAsync(c->desc.p, stage, bytes, hipMemcpyHostToDevice, c->stream));
     }
-    const double* d_alt = alt ? c->guesses.as<double>() + 16 * (size_t)S : nullptr;
+    const double* d_guess = (const double*)(c->desc.as<char>() + desc_bytes);
+    const double* d_alt = alt ? d_guess + 16 * (size_t)S : nullptr;
+    double* d_prof = (double*)(c->out.as<char>() + out_bytes);
     int32_t launches = 0;
     double prof_sum[4] = {0, 0, 0, 0};
     int aborted = 0;
@@ -916,38 +897,32 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
         BUF_TRY(c->queue, sizeof(WorkQueue));
         BUF_TRY(c->items, sizeof(uint64_t) * cap);
         BUF_TRY(c->done, sizeof(uint32_t) * S);
-        HIP_TRY(hipMemsetAsync(c->items.p, 0, sizeof(uint64_t) * cap, c->stream));
-        LAUNCH_TRY(launch_init_states(c->guesses.as<double>(), d_alt, S, prm, c->states.as<ScanState>(),
-                                      c->sync.as<RoundSync>(), c->stream));
-        LAUNCH_TRY(launch_init_queue(c->desc.as<ScanDesc>(), S, (uint64_t)first_pass, c->queue.as<WorkQueue>(),
-                                     c->items.as<uint64_t>(), c->done.as<uint32_t>(), c->stream));
+        LAUNCH_TRY(launch_init_wq(d_guess, d_alt, c->desc.as<ScanDesc>(), S, prm, (uint64_t)first_pass, cap,
+                                  c->states.as<ScanState>(), c->queue.as<WorkQueue>(), c->items.as<uint64_t>(),
+                                  c->done.as<uint32_t>(), c->out.as<ScanOut>(), d_prof, c->stream));
         HIP_TRY(hipEventRecord(c->ev0, c->stream));
         LAUNCH_TRY(launch_align_wq(g->dev, pts, c->desc.as<ScanDesc>(), nwg, block, prm,
                                    c->states.as<ScanState>(), c->queue.as<WorkQueue>(), c->items.as<uint64_t>(), cap,
-                                   c->done.as<uint32_t>(), c->partials.as<double>(), c->out.as<ScanOut>(),
-                                   c->small.as<double>(), 1, c->stream));
+                                   c->done.as<uint32_t>(), c->partials.as<double>(), c->out.as<ScanOut>(), d_prof, 1,
+                                   c->stream));
         HIP_TRY(hipEventRecord(c->ev1, c->stream));
-        double prof[5];
-        HIP_TRY(hipMemcpyAsync(prof, c->small.p, sizeof(prof), hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        HIP_TRY(hipEventElapsedTime(&ms_total, c->ev0, c->ev1));
-        for (int k = 0; k < 4; k++) prof_sum[k] = prof[k];
-        aborted = prof[4] != 0.0;
         launches = 1;
     } else {
+        BUF_TRY(c->sync, sizeof(RoundSync) * ((S + MAX_BATCH_SCANS - 1) / MAX_BATCH_SCANS));
+        HIP_TRY(hipMemsetAsync(c->out.p, 0, out_bytes, c->stream));
         for (int32_t s0 = 0; s0 < S; s0 += MAX_BATCH_SCANS) {
             const int32_t n = std::min<int32_t>(MAX_BATCH_SCANS, S - s0);
             RoundSync* rs = c->sync.as<RoundSync>() + s0 / MAX_BATCH_SCANS;
-            LAUNCH_TRY(launch_init_states(c->guesses.as<double>() + 16 * (size_t)s0,
+            LAUNCH_TRY(launch_init_states(d_guess + 16 * (size_t)s0,
                                           d_alt ? d_alt + 16 * (size_t)s0 : nullptr, n, prm,
                                           c->states.as<ScanState>() + s0, rs, c->stream));
             HIP_TRY(hipEventRecord(c->ev0, c->stream));
             LAUNCH_TRY(launch_align(g->dev, pts, c->desc.as<ScanDesc>() + s0, n, nwg, block, prm,
                                     c->states.as<ScanState>() + s0, rs, c->partials.as<double>(),
-                                    c->out.as<ScanOut>() + s0, c->small.as<double>(), c->stream));
+                                    c->out.as<ScanOut>() + s0, d_prof, c->stream));
             HIP_TRY(hipEventRecord(c->ev1, c->stream));
             double prof[5];
-            HIP_TRY(hipMemcpyAsync(prof, c->small.p, sizeof(prof), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipMemcpyAsync(prof, d_prof, sizeof(prof), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
             float ms = 0;
             HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
@@ -957,11 +932,25 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
             launches++;
         }
     }
+    /* read back through the pinned staging buffer (stream order puts this copy
+     * after the uploads from it) */
+    const size_t back = out_bytes + (queue ? 5 * sizeof(double) : 0);
+    const int er = pinned_reserve(c, back);
+    if (er) return er;
+    HIP_TRY(hipMemcpyAsync(c->pin, c->out.p, back, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    c->pin_pending = false;
+    if (queue) {
+        const double* prof = (const double*)((const char*)c->pin + out_bytes);
+        HIP_TRY(hipEventElapsedTime(&ms_total, c->ev0, c->ev1));
+        for (int k = 0; k < 4; k++) prof_sum[k] = prof[k];
+        aborted = prof[4] != 0.0;
+    }
     c->last_ms = ms_total;
     c->last_step_ms = c->last_ms;
     c->last_launches = launches;
     for (int k = 0; k < 4; k++) c->last_profile[k] = prof_sum[k];
-    return collect_results(c, counts, S, aborted, results, used_alt);
+    return results_from_out((const ScanOut*)c->pin, counts, S, aborted, c, results, used_alt);
 }
 
 /* Copies scans into one device buffer, each scan's points reordered along a Morton
@@ -1132,7 +1121,7 @@ extern "C" int ndt_align_scans_noalloc(ndt_ctx* c, const ndt_grid* g, const ndt_
     const uint64_t o_desc = take(sizeof(ScanDesc) * (uint64_t)S);
     const uint64_t o_guess = take(sizeof(double) * 16 * (uint64_t)S);
     const uint64_t o_states = take(sizeof(ScanState) * (uint64_t)S);
-    const uint64_t o_sync = take(sizeof(RoundSync));
+    (void)take(256); /* part of the layout that the size limit is stated for */
     const uint64_t o_out = take(sizeof(ScanOut) * (uint64_t)S);
     const uint64_t o_part = take(sizeof(double) * 32 * (uint64_t)slots);
     const uint64_t o_queue = take(sizeof(WorkQueue));
@@ -1155,7 +1144,6 @@ extern "C" int ndt_align_scans_noalloc(ndt_ctx* c, const ndt_grid* g, const ndt_
     ScanDesc* d_desc = (ScanDesc*)(ws + o_desc);
     double* d_guess = (double*)(ws + o_guess);
     ScanState* d_states = (ScanState*)(ws + o_states);
-    RoundSync* d_sync = (RoundSync*)(ws + o_sync);
     ScanOut* d_out = (ScanOut*)(ws + o_out);
     double* d_part = (double*)(ws + o_part);
     WorkQueue* d_queue = (WorkQueue*)(ws + o_queue);
@@ -1167,11 +1155,8 @@ extern "C" int ndt_align_scans_noalloc(ndt_ctx* c, const ndt_grid* g, const ndt_
                            c->stream));
     HIP_TRY(hipMemcpyAsync(d_guess, guesses, sizeof(double) * 16 * (size_t)S, hipMemcpyHostToDevice, c->stream));
     LAUNCH_TRY(launch_make_descs(d_counts, S, chunk, fine_pass_of(p), d_desc, c->stream));
-    LAUNCH_TRY(launch_zero_u32(d_out, (int64_t)(sizeof(ScanOut) * (size_t)S / 4), c->stream));
-    LAUNCH_TRY(launch_zero_u32(d_items, (int64_t)(2 * cap), c->stream));
-    LAUNCH_TRY(launch_zero_u32(d_prof, 16, c->stream));
-    LAUNCH_TRY(launch_init_states(d_guess, nullptr, S, prm, d_states, d_sync, c->stream));
-    LAUNCH_TRY(launch_init_queue(d_desc, S, (uint64_t)first_pass, d_queue, d_items, d_done, c->stream));
+    LAUNCH_TRY(launch_init_wq(d_guess, nullptr, d_desc, S, prm, (uint64_t)first_pass, cap, d_states, d_queue, d_items,
+                              d_done, d_out, d_prof, c->stream));
     HIP_TRY(hipEventRecord(c->ev0, c->stream));
     LAUNCH_TRY(launch_align_wq(g->dev, sc->pts.as<float4>(), d_desc, nwg, block, prm, d_states, d_queue, d_items, cap,
                                d_done, d_part, d_out, d_prof, 0, c->stream));
@@ -1217,7 +1202,6 @@ int ndt::align_sub_prepare(ndt_ctx* c, const ndt_grid* g, const ndt_scans* sc, c
     a.fallback = fallback;
     BUF_TRY(a.desc, sizeof(ScanDesc) * S);
     BUF_TRY(a.states, sizeof(ScanState) * S);
-    BUF_TRY(a.sync, sizeof(RoundSync));
     BUF_TRY(a.out, sizeof(ScanOut) * S);
     BUF_TRY(a.partials, sizeof(double) * 32 * slots);
     BUF_TRY(a.queue, sizeof(WorkQueue));
@@ -1235,13 +1219,10 @@ int ndt::align_sub_prepare(ndt_ctx* c, const ndt_grid* g, const ndt_scans* sc, c
 int ndt::align_sub_enqueue(ndt_ctx* c, const ndt_grid* g, const ndt_scans* sc, AlignSub& a, const double* d_guesses,
                            const double* d_alt) {
     const int32_t S = a.S;
-    LAUNCH_TRY(launch_zero_u32(a.out.p, (int64_t)(sizeof(ScanOut) * S / 4), c->stream));
-    LAUNCH_TRY(launch_zero_u32(a.items.p, (int64_t)(2 * a.cap), c->stream));
-    LAUNCH_TRY(launch_zero_u32(a.prof.p, 16, c->stream));
-    LAUNCH_TRY(launch_init_states(d_guesses, a.fallback ? d_alt : nullptr, S, a.prm, a.states.as<ScanState>(),
-                                  a.sync.as<RoundSync>(), c->stream));
-    LAUNCH_TRY(launch_init_queue(a.desc.as<ScanDesc>(), S, (uint64_t)a.first_pass, a.queue.as<WorkQueue>(),
-                                 a.items.as<uint64_t>(), a.done.as<uint32_t>(), c->stream));
+    LAUNCH_TRY(launch_init_wq(d_guesses, a.fallback ? d_alt : nullptr, a.desc.as<ScanDesc>(), S, a.prm,
+                              (uint64_t)a.first_pass, a.cap, a.states.as<ScanState>(), a.queue.as<WorkQueue>(),
+                              a.items.as<uint64_t>(), a.done.as<uint32_t>(), a.out.as<ScanOut>(), a.prof.as<double>(),
+                              c->stream));
     LAUNCH_TRY(launch_align_wq(g->dev, sc->pts.as<float4>(), a.desc.as<ScanDesc>(), a.nwg, a.block, a.prm,
                                a.states.as<ScanState>(), a.queue.as<WorkQueue>(), a.items.as<uint64_t>(), a.cap,
                                a.done.as<uint32_t>(), a.partials.as<double>(), a.out.as<ScanOut>(),
@@ -1277,12 +1258,9 @@ static int capture_body(ndt_ctx* c, const ndt_grid* g, ndt_scans* sc, GraphPlan&
                         int64_t first_pass, uint64_t cap, int32_t nwg, int block) {
     const int32_t S = sc->S;
     HIP_TRY(hipMemcpyAsync(gp.guesses.p, gp.h_guess, sizeof(double) * 16 * S, hipMemcpyHostToDevice, c->stream));
-    LAUNCH_TRY(launch_zero_u32(gp.out.p, (int64_t)(sizeof(ScanOut) * S / 4), c->stream));
-    LAUNCH_TRY(launch_zero_u32(gp.items.p, (int64_t)(2 * cap), c->stream));
-    LAUNCH_TRY(launch_init_states(gp.guesses.as<double>(), nullptr, S, prm, gp.states.as<ScanState>(),
-                                  gp.sync.as<RoundSync>(), c->stream));
-    LAUNCH_TRY(launch_init_queue(gp.desc.as<ScanDesc>(), S, (uint64_t)first_pass, gp.queue.as<WorkQueue>(),
-                                 gp.items.as<uint64_t>(), gp.done.as<uint32_t>(), c->stream));
+    LAUNCH_TRY(launch_init_wq(gp.guesses.as<double>(), nullptr, gp.desc.as<ScanDesc>(), S, prm, (uint64_t)first_pass, cap,
+                              gp.states.as<ScanState>(), gp.queue.as<WorkQueue>(), gp.items.as<uint64_t>(),
+                              gp.done.as<uint32_t>(), gp.out.as<ScanOut>(), gp.prof.as<double>(), c->stream));
     LAUNCH_TRY(launch_align_wq(g->dev, sc->pts.as<float4>(), gp.desc.as<ScanDesc>(), nwg, block, prm,
                                gp.states.as<ScanState>(), gp.queue.as<WorkQueue>(), gp.items.as<uint64_t>(), cap,
                                gp.done.as<uint32_t>(), gp.partials.as<double>(), gp.out.as<ScanOut>(),
@@ -1318,7 +1296,6 @@ static int graph_prepare(ndt_ctx* c, const ndt_grid* g, ndt_scans* sc, const ndt
     const int32_t nwg = bpc * c->cus;
     BUF_TRY(gp.desc, sizeof(ScanDesc) * S);
     BUF_TRY(gp.states, sizeof(ScanState) * S);
-    BUF_TRY(gp.sync, sizeof(RoundSync));
     BUF_TRY(gp.out, sizeof(ScanOut) * S);
     BUF_TRY(gp.partials, sizeof(double) * 32 * slots);
     BUF_TRY(gp.queue, sizeof(WorkQueue));

@@ -181,7 +181,7 @@ struct ndt_ctx {
     char name[256] = {0};
     /* workspaces */
     DevBuf raw, order; /* scans as uploaded, and the work space of ordering them */
-    DevBuf pts, desc, states, sync, partials, out, guesses, small, partials2, queue, items, done;
+    DevBuf pts, desc, states, sync, partials, out, small, partials2, queue, items, done;
     /* grid-build temporaries, and the compat callback's grid and scan, kept for
      * reuse: freeing device memory synchronises the device, which would serialise
      * contexts that work concurrently (one per host thread) */
@@ -243,7 +243,7 @@ struct GraphPlan {
     ndt_params params{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    DevBuf desc, states, sync, out, partials, queue, items, done, guesses, prof;
+    DevBuf desc, states, out, partials, queue, items, done, guesses, prof;
     double* h_guess = nullptr;
     void* h_out = nullptr;
     double* h_prof = nullptr;
@@ -269,7 +269,7 @@ namespace ndt {
  * workspace, the chunk descriptors (uploaded by align_sub_prepare) and pinned
  * host memory for the results. */
 struct AlignSub {
-    DevBuf desc, states, sync, out, partials, queue, items, done, prof;
+    DevBuf desc, states, out, partials, queue, items, done, prof;
     void* h_out = nullptr;
     double* h_prof = nullptr;
     AlignParams prm{};

@@ -201,13 +201,17 @@ NDT_HD void pose_matrix(const double* p, double* M) {
     pose_matrix_cs(p, c, s, M);
 }
 
-/* inverse of pose_matrix for |pitch| < pi/2 */
-NDT_HD void pose_euler(const double* M, double* out) {
+NDT_HD double pose_euler_pitch(const double* M) {
     double s = M[2];
     if (s > 1.0) s = 1.0;
     if (s < -1.0) s = -1.0;
+    return asin(s);
+}
+
+/* inverse of pose_matrix for |pitch| < pi/2 */
+NDT_HD void pose_euler(const double* M, double* out) {
     out[0] = atan2(-M[6], M[10]);
-    out[1] = asin(s);
+    out[1] = pose_euler_pitch(M);
     out[2] = atan2(-M[1], M[0]);
 }
 
@@ -522,13 +526,15 @@ int launch_fit_rows(const uint64_t* vkey, const uint32_t* starts, int64_t nvox, 
                     const int32_t* dims, uint32_t* begin, hipStream_t stream);
 int launch_fitness(FitGridDev fg, const float4* pts, const int64_t* offsets, const int32_t* counts, int32_t S,
                    const double* poses, double max_d2, int shells, int nblk, double* partials, hipStream_t stream);
-int launch_init_queue(const ScanDesc* scans, int32_t S, uint64_t total_chunks, WorkQueue* q, uint64_t* items,
-                      uint32_t* done_cnt, hipStream_t stream);
+/* sets up a work-queue launch: states at the guesses (alt as for launch_init_states), the
+ * first pass's total_chunks items and the rest of the queue's cap items empty, counters,
+ * cleared results and prof (8 doubles).  One kernel, so that graphs can hold it. */
+int launch_init_wq(const double* guesses, const double* alt, const ScanDesc* scans, int32_t S, AlignParams prm,
+                   uint64_t total_chunks, uint64_t cap, ScanState* states, WorkQueue* q, uint64_t* items,
+                   uint32_t* done_cnt, ScanOut* out, double* prof, hipStream_t stream);
 int launch_align_wq(NdtGridDev g, const float4* pts, const ScanDesc* scans, int32_t nwg, int block_size,
                     AlignParams prm, ScanState* states, WorkQueue* q, uint64_t* items, uint64_t cap, uint32_t* done_cnt,
                     double* partials, ScanOut* out, double* prof, int cooperative, hipStream_t stream);
-/* writes n zero words (32-bit) from dst: a kernel, so that graphs can hold it */
-int launch_zero_u32(void* dst, int64_t n, hipStream_t stream);
 int align_wq_max_blocks(int block_size, int point_fp64, int sum_mode, int* blocks_per_cu);
 /* alt (optional, S x 16): refined starts; then every scan opens with a probe pass at
  * its given guess, runs from the refined guess and falls back to the given guess */

@@ -2829,14 +2829,63 @@ __device__ inline void stores_complete() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-__global__ void k_init_queue(const ScanDesc* __restrict__ scans, int32_t S, uint64_t total, WorkQueue* q,
-                             uint64_t* __restrict__ items, uint32_t* __restrict__ done_cnt) {
-    const int s = blockIdx.x;
-    if (s >= S) return;
-    const ScanDesc sd = scans[s];
-    for (int k = threadIdx.x; k < sd.nchunks; k += blockDim.x) items[sd.qbase + k] = make_item(0, s, k);
-    if (threadIdx.x == 0) done_cnt[s] = 0u;
-    if (s == 0 && threadIdx.x == 0) {
+/* Everything a work-queue launch starts from, in one launch: the states at the given
+ * guesses (and refined starts), the first pass's items, the rest of the queue empty, the
+ * counters, cleared results.  Workgroup s sets up scan s, all of them clear the queue.
+ * (Clearing results and queue, the states and the queue's head were four or five launches
+ * of 4 to 7 us and the gaps between them, and a lane took a state's angles and their
+ * cosines and sines one after the other.  With one copy each way around the launch, a lone
+ * scan's call went from 287 to 232 us at 2 k points, from 548 to 488 us at 20 k.) */
+__global__ __launch_bounds__(256) void k_init_wq(const double* __restrict__ guesses, const double* __restrict__ alt,
+                                                 const ScanDesc* __restrict__ scans, int32_t S, AlignParams prm,
+                                                 uint64_t total, uint64_t cap, ScanState* __restrict__ states,
+                                                 WorkQueue* __restrict__ q, uint64_t* __restrict__ items,
+                                                 uint32_t* __restrict__ done_cnt, ScanOut* __restrict__ out,
+                                                 double* __restrict__ prof) {
+    __shared__ uint64_t sstate[STATE_WORDS];
+    __shared__ double trig[6];
+    const int tid = threadIdx.x, s = blockIdx.x;
+    if (s < S) {
+        const ScanDesc sd = scans[s];
+        for (int k = tid; k < sd.nchunks; k += 256) items[sd.qbase + k] = make_item(0, s, k);
+        for (int w = tid; w < (int)(sizeof(ScanOut) / 8); w += 256) ((uint64_t*)(out + s))[w] = 0;
+        if (tid == 0) done_cnt[s] = 0u;
+        for (int w = tid; w < STATE_WORDS; w += 256) sstate[w] = 0;
+        __syncthreads();
+        ScanState& st = *(ScanState*)sstate;
+        if (tid < WAVE) {
+            /* lanes 0-5: position and angles of the guess; 8-13: of the refined start */
+            const double* G = (tid & 8) && alt ? alt + 16 * (int64_t)s : guesses + 16 * (int64_t)s;
+            const int k = tid & 7;
+            if (tid < 16 && k < 6) {
+                double v;
+                if (k < 3) {
+                    v = G[4 * k + 3] - prm.origin[k];
+                } else if (k == 4) {
+                    v = pose_euler_pitch(G);
+                } else {
+                    v = atan2(k == 3 ? -G[6] : -G[1], k == 3 ? G[10] : G[0]);
+                }
+                if (tid < 8) {
+                    st.x_t[k] = v;
+                    st.p[k] = v;
+                } else if (alt) {
+                    st.alt[k] = v;
+                }
+            }
+            wave_order();
+            wave_pass_params(st, prm, trig);
+            if (tid == 0) {
+                st.phase = alt ? PH_PROBE : PH_INIT;
+                if (alt) st.fb_stage = FB_PROBE;
+            }
+        }
+        __syncthreads();
+        for (int w = tid; w < STATE_WORDS; w += 256) ((uint64_t*)(states + s))[w] = sstate[w];
+    }
+    for (uint64_t i = total + blockIdx.x * 256ull + tid; i < cap; i += gridDim.x * 256ull) items[i] = 0;
+    if (s == 0 && tid < 8) prof[tid] = 0.0;
+    if (s == 0 && tid == 0) {
         q->head = 0u;
         q->tail = (uint32_t)total;
         q->remaining = (uint32_t)S;
@@ -2844,9 +2893,13 @@ __global__ void k_init_queue(const ScanDesc* __restrict__ scans, int32_t S, uint
     }
 }
 
-int launch_init_queue(const ScanDesc* scans, int32_t S, uint64_t total_chunks, WorkQueue* q, uint64_t* items,
-                      uint32_t* done_cnt, hipStream_t stream) {
-    hipLaunchKernelGGL(k_init_queue, dim3(S), dim3(256), 0, stream, scans, S, total_chunks, q, items, done_cnt);
+int launch_init_wq(const double* guesses, const double* alt, const ScanDesc* scans, int32_t S, AlignParams prm,
+                   uint64_t total_chunks, uint64_t cap, ScanState* states, WorkQueue* q, uint64_t* items,
+                   uint32_t* done_cnt, ScanOut* out, double* prof, hipStream_t stream) {
+    /* enough workgroups for the clearing (8 items per thread), at most 4096 */
+    const uint64_t want = std::min<uint64_t>(4096, (cap - total_chunks + 2047) / 2048);
+    hipLaunchKernelGGL(k_init_wq, dim3((unsigned)std::max<uint64_t>((uint64_t)S, want)), dim3(256), 0, stream, guesses, alt,
+                       scans, S, prm, total_chunks, cap, states, q, items, done_cnt, out, prof);
     return (int)hipGetLastError();
 }
 
@@ -3025,19 +3078,6 @@ static int launch_align_wq_t(NdtGridDev g, const float4* pts, const ScanDesc* sc
     const void* kern = prm.hess_at_accept ? (const void*)k_align_wq<T, SUM, BLOCK, true>
                                           : (const void*)k_align_wq<T, SUM, BLOCK, false>;
     return (int)hipLaunchCooperativeKernel(kern, dim3(nwg), dim3(BLOCK), args, 0, stream);
-}
-
-__global__ void k_zero_u32(uint32_t* __restrict__ dst, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = 0u;
-}
-
-int launch_zero_u32(void* dst, int64_t n, hipStream_t stream) {
-    if (n <= 0) return 0;
-    const int64_t want = (n + 255) / 256;
-    const int blocks = (int)(want < 4096 ? want : 4096);
-    hipLaunchKernelGGL(k_zero_u32, dim3(blocks), dim3(256), 0, stream, (uint32_t*)dst, n);
-    return (int)hipGetLastError();
 }
 
 template <typename T, int SUM, int BLOCK>
