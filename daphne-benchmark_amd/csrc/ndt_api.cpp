@@ -225,8 +225,8 @@ static int sorted_runs(ndt_ctx* c, const uint64_t* keys, int64_t n, int shift, u
                        DevBuf& scratch, int64_t* nruns, int64_t* below) {
     BUF_TRY(starts, sizeof(uint32_t) * (n + 1));
     BUF_TRY(scratch, runs_scratch_bytes(n));
-    LAUNCH_TRY(launch_runs(keys, n, shift, limit, starts.as<uint32_t>(), scratch.as<uint32_t>(), c->stream));
-    HIP_TRY(hipMemcpyAsync(c->hsmall, scratch.p, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+    LAUNCH_TRY(launch_runs(keys, n, shift, limit, starts.as<uint32_t>(), scratch.as<uint32_t>(), (uint32_t*)c->hsmall,
+                           c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     *nruns = ((const uint32_t*)c->hsmall)[0];
     *below = ((const uint32_t*)c->hsmall)[1];
@@ -475,11 +475,9 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)ncells);
         BUF_TRY(c->bk_vid, sizeof(uint32_t) * (size_t)ncells);
         BUF_TRY(scratch, cells_scratch_bytes(ncells));
-        uint64_t* totals = nullptr;
         LAUNCH_TRY(launch_cells_index(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), nvox, g->bits, tiles, ncells,
                                       c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_vid.as<uint32_t>(),
-                                      scratch.p, &totals, c->stream));
-        HIP_TRY(hipMemcpyAsync(c->hsmall, totals, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, c->stream));
+                                      scratch.p, (uint64_t*)c->hsmall, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         const uint64_t* h = (const uint64_t*)c->hsmall;
         nv = (int64_t)(h[0] >> 32);
@@ -867,19 +865,21 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     else LAUNCH_TRY(align_kernel_max_blocks(block, prm.point_fp64, prm.sum_mode, &bpc));
     if (bpc <= 0) return fail(NDT_ERR_UNSUPPORTED, "align kernel does not fit on a compute unit");
     const int32_t nwg = bpc * c->cus;
-    /* descriptors, guesses and refined starts in one buffer, results and phase times in
-     * another: one copy each way */
+    /* descriptors, guesses and refined starts go up in one copy; results and phase times
+     * are written to the pinned buffer by the kernel (a few stores per scan at its end) */
     const size_t desc_bytes = sizeof(ScanDesc) * (size_t)S, guess_bytes = sizeof(double) * 16 * (size_t)S;
     const size_t out_bytes = sizeof(ScanOut) * (size_t)S;
     BUF_TRY(c->desc, desc_bytes + guess_bytes * (alt ? 2 : 1));
     BUF_TRY(c->states, sizeof(ScanState) * S);
-    BUF_TRY(c->out, out_bytes + 8 * sizeof(double));
     BUF_TRY(c->partials, sizeof(double) * 32 * slots);
+    char* back = nullptr;
     {
-        char* stage = nullptr;
         const size_t bytes = desc_bytes + guess_bytes * (alt ? 2 : 1);
-        const int eu = pinned_stage(c, bytes, &stage);
+        const size_t up = (bytes + 255) & ~(size_t)255;
+        char* stage = nullptr;
+        const int eu = pinned_stage(c, up + out_bytes + 8 * sizeof(double), &stage);
         if (eu) return eu;
+        back = stage + up;
         std::memcpy(stage, desc.data(), desc_bytes);
         std::memcpy(stage + desc_bytes, guesses, guess_bytes);
         if (alt) std::memcpy(stage + desc_bytes + guess_bytes, alt, guess_bytes);
@@ -888,7 +888,8 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     }
     const double* d_guess = (const double*)(c->desc.as<char>() + desc_bytes);
     const double* d_alt = alt ? d_guess + 16 * (size_t)S : nullptr;
-    double* d_prof = (double*)(c->out.as<char>() + out_bytes);
+    ScanOut* out = (ScanOut*)back;
+    double* prof = (double*)(back + out_bytes);
     int32_t launches = 0;
     double prof_sum[4] = {0, 0, 0, 0};
     int aborted = 0;
@@ -899,17 +900,16 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
         BUF_TRY(c->done, sizeof(uint32_t) * S);
         LAUNCH_TRY(launch_init_wq(d_guess, d_alt, c->desc.as<ScanDesc>(), S, prm, (uint64_t)first_pass, cap,
                                   c->states.as<ScanState>(), c->queue.as<WorkQueue>(), c->items.as<uint64_t>(),
-                                  c->done.as<uint32_t>(), c->out.as<ScanOut>(), d_prof, c->stream));
+                                  c->done.as<uint32_t>(), out, prof, c->stream));
         HIP_TRY(hipEventRecord(c->ev0, c->stream));
         LAUNCH_TRY(launch_align_wq(g->dev, pts, c->desc.as<ScanDesc>(), nwg, block, prm,
                                    c->states.as<ScanState>(), c->queue.as<WorkQueue>(), c->items.as<uint64_t>(), cap,
-                                   c->done.as<uint32_t>(), c->partials.as<double>(), c->out.as<ScanOut>(), d_prof, 1,
-                                   c->stream));
+                                   c->done.as<uint32_t>(), c->partials.as<double>(), out, prof, 1, c->stream));
         HIP_TRY(hipEventRecord(c->ev1, c->stream));
         launches = 1;
     } else {
         BUF_TRY(c->sync, sizeof(RoundSync) * ((S + MAX_BATCH_SCANS - 1) / MAX_BATCH_SCANS));
-        HIP_TRY(hipMemsetAsync(c->out.p, 0, out_bytes, c->stream));
+        std::memset(out, 0, out_bytes);
         for (int32_t s0 = 0; s0 < S; s0 += MAX_BATCH_SCANS) {
             const int32_t n = std::min<int32_t>(MAX_BATCH_SCANS, S - s0);
             RoundSync* rs = c->sync.as<RoundSync>() + s0 / MAX_BATCH_SCANS;
@@ -919,10 +919,8 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
             HIP_TRY(hipEventRecord(c->ev0, c->stream));
             LAUNCH_TRY(launch_align(g->dev, pts, c->desc.as<ScanDesc>() + s0, n, nwg, block, prm,
                                     c->states.as<ScanState>() + s0, rs, c->partials.as<double>(),
-                                    c->out.as<ScanOut>() + s0, d_prof, c->stream));
+                                    out + s0, prof, c->stream));
             HIP_TRY(hipEventRecord(c->ev1, c->stream));
-            double prof[5];
-            HIP_TRY(hipMemcpyAsync(prof, d_prof, sizeof(prof), hipMemcpyDeviceToHost, c->stream));
             HIP_TRY(hipStreamSynchronize(c->stream));
             float ms = 0;
             HIP_TRY(hipEventElapsedTime(&ms, c->ev0, c->ev1));
@@ -932,16 +930,9 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
             launches++;
         }
     }
-    /* read back through the pinned staging buffer (stream order puts this copy
-     * after the uploads from it) */
-    const size_t back = out_bytes + (queue ? 5 * sizeof(double) : 0);
-    const int er = pinned_reserve(c, back);
-    if (er) return er;
-    HIP_TRY(hipMemcpyAsync(c->pin, c->out.p, back, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     c->pin_pending = false;
     if (queue) {
-        const double* prof = (const double*)((const char*)c->pin + out_bytes);
         HIP_TRY(hipEventElapsedTime(&ms_total, c->ev0, c->ev1));
         for (int k = 0; k < 4; k++) prof_sum[k] = prof[k];
         aborted = prof[4] != 0.0;
@@ -950,7 +941,7 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     c->last_step_ms = c->last_ms;
     c->last_launches = launches;
     for (int k = 0; k < 4; k++) c->last_profile[k] = prof_sum[k];
-    return results_from_out((const ScanOut*)c->pin, counts, S, aborted, c, results, used_alt);
+    return results_from_out(out, counts, S, aborted, c, results, used_alt);
 }
 
 /* Copies scans into one device buffer, each scan's points reordered along a Morton
@@ -1537,7 +1528,11 @@ extern "C" int ndt_derivatives(ndt_ctx* c, const ndt_grid* g, const float* scan,
     if (params->mode != g->params.mode) return fail(NDT_ERR_INVALID, "params mode differs from the grid's");
     HIP_TRY(hipSetDevice(c->device));
     BUF_TRY(c->pts, sizeof(float4) * n);
-    HIP_TRY(hipMemcpyAsync(c->pts.p, scan, sizeof(float4) * n, hipMemcpyHostToDevice, c->stream));
+    {
+        const int64_t first = 0;
+        e = upload_points(c, c->pts.as<char>(), nullptr, 0, &scan, &first, 1, n, false);
+        if (e) return e;
+    }
     if (params->mode == NDT_MODE_COMPAT) {
         if (!compat_transform) return fail(NDT_ERR_INVALID, "compat mode needs the transform matrix");
         double d1, d2;
@@ -1555,15 +1550,14 @@ extern "C" int ndt_derivatives(ndt_ctx* c, const ndt_grid* g, const float* scan,
     }
     AlignParams prm = make_align_params(params, 1);
     const int nblocks = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    BUF_TRY(c->partials2, sizeof(double) * NRED * nblocks + 64 * sizeof(double));
-    BUF_TRY(c->small, 64 * sizeof(double));
-    HIP_TRY(hipMemcpyAsync(c->small.p, p, sizeof(double) * 6, hipMemcpyHostToDevice, c->stream));
-    double* red_dev = c->partials2.as<double>() + (size_t)NRED * nblocks;
-    LAUNCH_TRY(launch_deriv_ndt(g->dev, c->pts.as<float4>(), n, c->small.as<double>(), prm, c->partials2.as<double>(),
-                                nblocks, c->stream));
-    LAUNCH_TRY(launch_reduce_partials(c->partials2.as<double>(), nblocks, NRED, red_dev, c->stream));
-    double red[NRED];
-    HIP_TRY(hipMemcpyAsync(red, red_dev, sizeof(red), hipMemcpyDeviceToHost, c->stream));
+    BUF_TRY(c->partials2, sizeof(double) * NRED * nblocks);
+    /* the pose is read from, and the sums are written to, pinned host memory */
+    double *red = (double*)c->hsmall, *pose = red + NRED;
+    static_assert(sizeof(double) * (NRED + 6) <= HSMALL_BYTES, "pinned readback buffer too small");
+    std::memcpy(pose, p, sizeof(double) * 6);
+    LAUNCH_TRY(launch_deriv_ndt(g->dev, c->pts.as<float4>(), n, pose, prm, c->partials2.as<double>(), nblocks,
+                                c->stream));
+    LAUNCH_TRY(launch_reduce_partials(c->partials2.as<double>(), nblocks, NRED, red, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     if (score) *score = red[0];
     if (gradient)
@@ -1588,12 +1582,10 @@ static int compat_pass(ndt_ctx* c, const ndt_grid* g, const float4* scan, int64_
         for (int q = 0; q < 3; q++) jh[(8 + k) * 3 + q] = hd[k][q];
     /* sixteen threads per point (k_deriv_compat) */
     const int nblocks = (int)std::min<int64_t>(512, (16 * n + 255) / 256);
-    BUF_TRY(c->partials2, sizeof(double) * NRED_COMPAT * (nblocks + 1));
-    double* red_dev = c->partials2.as<double>() + (size_t)NRED_COMPAT * nblocks;
+    BUF_TRY(c->partials2, sizeof(double) * NRED_COMPAT * nblocks);
     LAUNCH_TRY(launch_deriv_compat(g->cdev, scan, n, M, jh, d1, d2, c->partials2.as<double>(), nblocks, c->stream));
-    LAUNCH_TRY(launch_reduce_partials(c->partials2.as<double>(), nblocks, NRED_COMPAT, red_dev, c->stream));
     static_assert(sizeof(double) * NRED_COMPAT <= HSMALL_BYTES, "pinned readback buffer too small");
-    HIP_TRY(hipMemcpyAsync(c->hsmall, red_dev, sizeof(double) * NRED_COMPAT, hipMemcpyDeviceToHost, c->stream));
+    LAUNCH_TRY(launch_reduce_partials(c->partials2.as<double>(), nblocks, NRED_COMPAT, (double*)c->hsmall, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     std::memcpy(red, c->hsmall, sizeof(double) * NRED_COMPAT);
     return 0;

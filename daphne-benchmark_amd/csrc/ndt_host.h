@@ -181,7 +181,7 @@ struct ndt_ctx {
     char name[256] = {0};
     /* workspaces */
     DevBuf raw, order; /* scans as uploaded, and the work space of ordering them */
-    DevBuf pts, desc, states, sync, partials, out, small, partials2, queue, items, done;
+    DevBuf pts, desc, states, sync, partials, partials2, queue, items, done;
     /* grid-build temporaries, and the compat callback's grid and scan, kept for
      * reuse: freeing device memory synchronises the device, which would serialise
      * contexts that work concurrently (one per host thread) */

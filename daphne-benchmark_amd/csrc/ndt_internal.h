@@ -483,10 +483,11 @@ size_t scan_scratch_bytes(int64_t n);
 int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total_dev, void* scratch,
                        hipStream_t stream);
 /* starts[r] = where run r of equal (key >> shift) starts among the n sorted keys, keys >=
- * limit left out; scratch[0] = number of runs, scratch[1] = number of keys below the limit */
+ * limit left out; host_counts (pinned host memory) receives the number of runs and the
+ * number of keys below the limit */
 size_t runs_scratch_bytes(int64_t n);
 int launch_runs(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* starts, uint32_t* scratch,
-                hipStream_t stream);
+                uint32_t* host_counts, hipStream_t stream);
 int launch_voxel_stats_ndt(const float4* pts, const uint64_t* sorted_keys, const uint32_t* seg_start, int64_t nseg,
                            int64_t nvalid_pts, int min_points, double min_eig_ratio, double* mean, double* icov,
                            int32_t* count, uint32_t* valid, uint64_t* vkey, hipStream_t stream);
@@ -510,12 +511,12 @@ int launch_voxel_stats_compat(const float4* pts, const uint32_t* sorted_idx, con
 /* ndt alignment: init states from guesses, then the cooperative persistent kernel */
 /* dense query-cell index of the nvox voxels (those with valid[v] take part): run starts
  * begin[0..ncells] and, where a cell holds a valid voxel, its number vid[cell]; mask,
- * begin and vid hold ncells entries (begin one more).  *totals is device memory in
- * scratch: candidates and, in the upper half, valid voxels; then query cells. */
+ * begin and vid hold ncells entries (begin one more).  host_totals (pinned host
+ * memory) receives candidates and, in the upper half, valid voxels; then query cells. */
 size_t cells_scratch_bytes(int64_t ncells);
 int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
                        int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
-                       uint64_t** totals, hipStream_t stream);
+                       uint64_t* host_totals, hipStream_t stream);
 /* the candidate entries and float64 statistics behind that index */
 int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double* mean, const double* icov, int64_t nvox,
                       const int* bits, const int64_t* origin_cell, double res, const int32_t* tiles, const uint32_t* mask,

@@ -753,8 +753,11 @@ __global__ __launch_bounds__(SC_BLOCK) void k_runs_count(const uint64_t* __restr
 
 __global__ __launch_bounds__(SC_BLOCK) void k_runs_write(const uint64_t* __restrict__ keys, int64_t n, int shift,
                                                          uint64_t limit, const uint32_t* __restrict__ bsum,
-                                                         uint32_t* __restrict__ starts) {
+                                                         uint32_t* __restrict__ starts,
+                                                         const uint32_t* __restrict__ counts,
+                                                         uint32_t* __restrict__ host_counts) {
     __shared__ uint32_t cnt[SC_BLOCK / WAVE];
+    if (blockIdx.x == 0 && threadIdx.x < 2) host_counts[threadIdx.x] = counts[threadIdx.x];
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int64_t base = (int64_t)blockIdx.x * RUN_TILE + wave * RUN_PART + lane;
     uint32_t c = 0, heads = 0; /* bit r: this lane's key of round r is a head */
@@ -783,13 +786,14 @@ size_t runs_scratch_bytes(int64_t n) {
 }
 
 int launch_runs(const uint64_t* keys, int64_t n, int shift, uint64_t limit, uint32_t* starts, uint32_t* scratch,
-                hipStream_t stream) {
+                uint32_t* host_counts, hipStream_t stream) {
     const int64_t nb = (n + RUN_TILE - 1) / RUN_TILE;
     uint32_t* bsum = scratch + 2;
     hipLaunchKernelGGL(k_runs_count, dim3((unsigned)nb), dim3(SC_BLOCK), 0, stream, keys, n, shift, limit, bsum,
                        scratch + 1);
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, bsum, nb, scratch);
-    hipLaunchKernelGGL(k_runs_write, dim3((unsigned)nb), dim3(SC_BLOCK), 0, stream, keys, n, shift, limit, bsum, starts);
+    hipLaunchKernelGGL(k_runs_write, dim3((unsigned)nb), dim3(SC_BLOCK), 0, stream, keys, n, shift, limit, bsum, starts,
+                       scratch, host_counts);
     return (int)hipGetLastError();
 }
 
@@ -1205,8 +1209,10 @@ __global__ __launch_bounds__(1024) void k_cells_top(uint64_t* __restrict__ bsum,
  * each cell that holds one */
 __global__ __launch_bounds__(256) void k_cells_down(const uint32_t* __restrict__ mask, int64_t ncells,
                                                     const uint64_t* __restrict__ bsum, uint32_t* __restrict__ begin,
-                                                    uint32_t* __restrict__ vid) {
+                                                    uint32_t* __restrict__ vid, const uint64_t* __restrict__ totals,
+                                                    uint64_t* __restrict__ host_totals) {
     __shared__ uint64_t lw[256 / WAVE];
+    if (blockIdx.x == 0 && threadIdx.x < 2) host_totals[threadIdx.x] = totals[threadIdx.x];
     uint32_t m[CELL_ITEMS];
     const int64_t base = blockIdx.x * (int64_t)CELL_TILE + threadIdx.x * CELL_ITEMS;
     load_masks(mask, ncells, base, m);
@@ -1273,7 +1279,7 @@ size_t cells_scratch_bytes(int64_t ncells) {
 
 int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
                        int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
-                       uint64_t** totals, hipStream_t stream) {
+                       uint64_t* host_totals, hipStream_t stream) {
     Bits3 B;
     for (int k = 0; k < 3; k++) B.b[k] = bits[k];
     const int64_t nb = (ncells + CELL_TILE - 1) / CELL_TILE;
@@ -1286,8 +1292,8 @@ int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox
                        tiles[1], mask);
     hipLaunchKernelGGL(k_cells_reduce, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, tot);
     hipLaunchKernelGGL(k_cells_top, dim3(1), dim3(1024), 0, stream, bsum, nb, tot);
-    hipLaunchKernelGGL(k_cells_down, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, begin, vid);
-    *totals = tot;
+    hipLaunchKernelGGL(k_cells_down, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, begin, vid,
+                       tot, host_totals);
     return (int)hipGetLastError();
 }
 
