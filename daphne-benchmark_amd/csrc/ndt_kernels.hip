@@ -1,13 +1,14 @@
 /*
  * ndt_kernels.hip - gfx950 kernels of the NDT scan-matching engine.
  *
- *  grid build   bbox reduce, voxel keys, stable LSD radix sort, run heads/starts,
+ *  uploads      a scan's points in the order of a Morton curve
+ *  grid build   bbox reduce, voxel keys, stable LSD radix sort, run starts,
  *               per-voxel float64 statistics (ndt: two-pass covariance, Jacobi
  *               eigenvalue clamp, inverse; compat: the reference's single-pass
- *               normalisation), neighbourhood dilation, hash build
- *  align        fused per-point kernel: transform, hashed cell lookup, candidate
- *               list scan, score / gradient / Hessian per pair, wave64 shuffle +
- *               LDS reductions; persistent cooperative kernel that keeps every
+ *               normalisation), dense (cell masks) or hashed index of candidates
+ *  align        fused per-point kernel: transform, cell lookup, candidate list
+ *               scan, score / gradient / Hessian per pair, sums within the wave on
+ *               the vector ALU, then in LDS; persistent kernels that keep every
  *               scan's Newton / More-Thuente state on the device
  *  compat       the reference's per-pair arithmetic in float64 on the GPU
  *

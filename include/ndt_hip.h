@@ -102,9 +102,9 @@ typedef struct ndt_grid_info {
     int64_t map_points;
     int64_t voxels;          /* occupied voxels */
     int64_t valid_voxels;    /* voxels used for matching (ndt) */
-    int64_t query_cells;     /* hashed lookup cells (ndt: occupied cells dilated by one) */
+    int64_t query_cells;     /* lookup cells (ndt: occupied cells dilated by one) */
     int64_t candidates;      /* candidate entries of the lookup lists */
-    int64_t hash_capacity;
+    int64_t hash_capacity;   /* slots of a hash of the lookup cells (held where the index is hashed) */
     int64_t dense_cells;     /* compat: cells of the reference's dense grid; ndt: cells of the
                                 dense query-cell index, 0 when the index is hashed */
     int32_t dims[3];         /* compat: dense grid dimensions */
