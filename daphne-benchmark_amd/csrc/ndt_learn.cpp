@@ -584,7 +584,8 @@ static int forward_dev(ndt_model* md, int B, bool train) {
     return 0;
 }
 
-/* Backward of the loss of the last training forward: gradients into md->g. */
+/* Backward of the loss of the last training forward: gradients into md->g, W1's
+ * only up to the operands of its product (grad_w1_dev, or adam_dev). */
 static int backward_dev(ndt_model* md, int B) {
     hipStream_t st = md->ctx->stream;
     const int f0 = md->f0, f1 = md->f1, f2 = md->f2;
@@ -599,27 +600,45 @@ static int backward_dev(ndt_model* md, int B) {
     /* dW2 [f2 x f1] = dZ2^T H1 */
     LAUNCH_TRY(launch_gemm_nt(md->dZ2T.as<uint16_t>(), B, md->H1T.as<uint16_t>(), B, md->g[NDT_W2].as<float>(), f1, f2,
                               f1, B, 1, st));
-    /* dW1 [f1 x f0] = dZ1^T X */
     LAUNCH_TRY(launch_transpose_u16(md->X.as<uint16_t>(), B, f0, md->XT.as<uint16_t>(), st));
-    LAUNCH_TRY(launch_gemm_nt(md->dZ1T.as<uint16_t>(), B, md->XT.as<uint16_t>(), B, md->g[NDT_W1].as<float>(), f0, f1,
-                              f0, B, 1, st));
     return 0;
 }
 
-static int adam_dev(ndt_model* md, float lr, float b1, float b2, float eps, float wd) {
+/* dW1 [f1 x f0] = dZ1^T X */
+static int grad_w1_dev(ndt_model* md, int B) {
+    LAUNCH_TRY(launch_gemm_nt(md->dZ1T.as<uint16_t>(), B, md->XT.as<uint16_t>(), B, md->g[NDT_W1].as<float>(), md->f0,
+                              md->f1, md->f0, B, 1, md->ctx->stream));
+    return 0;
+}
+
+/* One Adam step from the gradients in md->g.  With rows > 0, W1's gradient is made
+ * from the operands that backward_dev left for a batch of `rows`, in the launch that
+ * steps W1, and goes to md->g only if keep_g: a training run asks for that on its
+ * last step, whose gradients can be read afterwards. */
+static int adam_dev(ndt_model* md, float lr, float b1, float b2, float eps, float wd, int rows = 0,
+                    bool keep_g = false) {
     hipStream_t st = md->ctx->stream;
     md->step++;
     const float bc1 = (float)(1.0 - std::pow((double)b1, (double)md->step));
     const float bc2 = (float)(1.0 - std::pow((double)b2, (double)md->step));
+    AdamArgs q = {lr, b1, b2, eps, bc1, bc2, 0.0f};
+    AdamSegs segs{};
     for (int k = 0; k < 6; k++) {
         uint16_t* wb = k == NDT_W1 ? md->wb1.as<uint16_t>()
                        : k == NDT_W2 ? md->wb2.as<uint16_t>()
                        : k == NDT_W3 ? md->wb3.as<uint16_t>()
                                      : nullptr;
         const float wdk = (k == NDT_W1 || k == NDT_W2 || k == NDT_W3) ? wd : 0.0f;
-        LAUNCH_TRY(launch_adam(md->w[k].as<float>(), md->mom[k].as<float>(), md->vel[k].as<float>(),
-                               md->g[k].as<float>(), tensor_size(md, k), lr, b1, b2, eps, bc1, bc2, wdk, wb, st));
+        q.wd = wdk;
+        if (k == NDT_W1 && rows > 0)
+            LAUNCH_TRY(launch_gemm_adam(md->dZ1T.as<uint16_t>(), rows, md->XT.as<uint16_t>(), rows, md->f1, md->f0,
+                                        rows, md->w[k].as<float>(), md->mom[k].as<float>(), md->vel[k].as<float>(),
+                                        md->g[k].as<float>(), keep_g, q, wb, st));
+        else
+            segs.seg[segs.count++] = {md->w[k].as<float>(), md->mom[k].as<float>(), md->vel[k].as<float>(),
+                                      md->g[k].as<float>(), wb, tensor_size(md, k), 0, wdk};
     }
+    LAUNCH_TRY(launch_adam(segs, q, st));
     LAUNCH_TRY(launch_transpose_u16(md->wb2.as<uint16_t>(), md->f2, md->f1, md->wb2t.as<uint16_t>(), st));
     return 0;
 }
@@ -657,6 +676,7 @@ extern "C" int ndt_model_backward(ndt_ctx* c, ndt_model* md, const uint16_t* x, 
     HIP_TRY(hipMemcpyAsync(md->weights.p, w, sizeof(w), hipMemcpyHostToDevice, c->stream));
     if ((e = forward_dev(md, B, true))) return e;
     if ((e = backward_dev(md, B))) return e;
+    if ((e = grad_w1_dev(md, B))) return e;
     std::vector<float> lb((size_t)B);
     HIP_TRY(hipMemcpyAsync(lb.data(), md->lossb.p, 4 * (size_t)B, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -951,7 +971,7 @@ extern "C" int ndt_model_train(ndt_ctx* c, ndt_model* md, const ndt_dataset* dsc
                 lr = (float)(lo + (tp->lr - lo) * 0.5 * (1.0 + std::cos(3.141592653589793 * (double)step / (double)total_steps)));
             }
             step++;
-            if ((e = adam_dev(md, lr, tp->beta1, tp->beta2, tp->eps, tp->weight_decay))) return e;
+            if ((e = adam_dev(md, lr, tp->beta1, tp->beta2, tp->eps, tp->weight_decay, B, step == total_steps))) return e;
             LAUNCH_TRY(launch_sum_ordered(md->lossb.as<float>(), B, md->lossacc.as<float>(), st));
         }
         float acc = 0.f;

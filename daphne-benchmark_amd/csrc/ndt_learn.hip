@@ -843,18 +843,20 @@ int launch_transpose_u16(const uint16_t* src, int64_t rows, int64_t cols, uint16
  * multiplied.  Rows are padded by 8 elements (16 bytes). */
 constexpr int GPAD = 8;
 
-__global__ __launch_bounds__(256) void k_gemm_nt(const uint16_t* __restrict__ A, int64_t lda,
-                                                 const uint16_t* __restrict__ B, int64_t ldb, float* __restrict__ C,
-                                                 int64_t ldc, int64_t split_stride, int kps) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][GEMM_BM][GEMM_BK + GPAD];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][GEMM_BN][GEMM_BK + GPAD];
+struct GemmLds {
+    uint16_t a[2][GEMM_BM][GEMM_BK + GPAD];
+    uint16_t b[2][GEMM_BN][GEMM_BK + GPAD];
+};
+
+/* The 128 x 128 tile of A B^T whose first rows are Ab and Bb, over nk K steps.
+ * With ROWS the operands of each instruction change places, so that a lane
+ * receives D^T: four neighbouring columns of one row of C instead of four
+ * neighbouring rows of one column.  The products and their order are the same. */
+template <bool ROWS>
+__device__ __forceinline__ void gemm_tile(GemmLds& L, const uint16_t* __restrict__ Ab, int64_t lda,
+                                          const uint16_t* __restrict__ Bb, int64_t ldb, int nk, f32x4 (&acc)[4][4]) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wm = w >> 1, wn = w & 1;
-    const int64_t m0 = (int64_t)blockIdx.y * GEMM_BM, n0 = (int64_t)blockIdx.x * GEMM_BN;
-    const int64_t k0 = (int64_t)blockIdx.z * kps;
-    const int nk = kps / GEMM_BK;
-    const uint16_t* Ab = A + m0 * lda + k0;
-    const uint16_t* Bb = B + n0 * ldb + k0;
     uint4 ra[4], rb[4];
     /* tile chunk c = tid + 256 q (q = 0..3): row c / 8, columns 8 (c mod 8) .. +7 */
     const int lr = tid >> 3, lc = (tid & 7) * 8;
@@ -865,11 +867,10 @@ __global__ __launch_bounds__(256) void k_gemm_nt(const uint16_t* __restrict__ A,
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        *(uint4*)&As[0][lr + 32 * q][lc] = ra[q];
-        *(uint4*)&Bs[0][lr + 32 * q][lc] = rb[q];
+        *(uint4*)&L.a[0][lr + 32 * q][lc] = ra[q];
+        *(uint4*)&L.b[0][lr + 32 * q][lc] = rb[q];
     }
     __syncthreads();
-    f32x4 acc[4][4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -888,23 +889,36 @@ __global__ __launch_bounds__(256) void k_gemm_nt(const uint16_t* __restrict__ A,
         for (int kk = 0; kk < GEMM_BK; kk += 32) {
             bf16x8 a[4], bv[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = *(const bf16x8*)&As[buf][wm * 64 + i * 16 + fr][kk + fk];
+            for (int i = 0; i < 4; i++) a[i] = *(const bf16x8*)&L.a[buf][wm * 64 + i * 16 + fr][kk + fk];
 #pragma unroll
-            for (int j = 0; j < 4; j++) bv[j] = *(const bf16x8*)&Bs[buf][wn * 64 + j * 16 + fr][kk + fk];
+            for (int j = 0; j < 4; j++) bv[j] = *(const bf16x8*)&L.b[buf][wn * 64 + j * 16 + fr][kk + fk];
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bv[j], acc[i][j], 0, 0, 0);
+                    acc[i][j] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j], a[i], acc[i][j], 0, 0, 0)
+                                     : __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bv[j], acc[i][j], 0, 0, 0);
         }
         /* the other buffer was last read in the previous iteration, before its barrier */
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            *(uint4*)&As[buf ^ 1][lr + 32 * q][lc] = ra[q];
-            *(uint4*)&Bs[buf ^ 1][lr + 32 * q][lc] = rb[q];
+            *(uint4*)&L.a[buf ^ 1][lr + 32 * q][lc] = ra[q];
+            *(uint4*)&L.b[buf ^ 1][lr + 32 * q][lc] = rb[q];
         }
         __syncthreads();
     }
+}
+
+__global__ __launch_bounds__(256) void k_gemm_nt(const uint16_t* __restrict__ A, int64_t lda,
+                                                 const uint16_t* __restrict__ B, int64_t ldb, float* __restrict__ C,
+                                                 int64_t ldc, int64_t split_stride, int kps) {
+    __shared__ __attribute__((aligned(16))) GemmLds L;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int wm = w >> 1, wn = w & 1, fr = lane & 15;
+    const int64_t m0 = (int64_t)blockIdx.y * GEMM_BM, n0 = (int64_t)blockIdx.x * GEMM_BN;
+    const int64_t k0 = (int64_t)blockIdx.z * kps;
+    f32x4 acc[4][4];
+    gemm_tile<false>(L, A + m0 * lda + k0, lda, B + n0 * ldb + k0, ldb, kps / GEMM_BK, acc);
     float* Cz = C + (int64_t)blockIdx.z * split_stride;
 #pragma unroll
     for (int i = 0; i < 4; i++)
@@ -1156,27 +1170,126 @@ int launch_relu_bwd(const float* dH, const uint16_t* H, int B, int F, uint16_t* 
 }
 
 /* Adam (Kingma & Ba 2015) with decoupled weight decay wd (Loshchilov & Hutter
- * 2019) on float32 master weights; bc1 = 1 - beta1^t and bc2 = 1 - beta2^t; wb
- * (optional) receives the bf16 copy used by the GEMMs. */
-__global__ void k_adam(float* __restrict__ w, float* __restrict__ m, float* __restrict__ v, const float* __restrict__ g,
-                       int64_t n, float lr, float beta1, float beta2, float eps, float bc1, float bc2, float wd,
-                       uint16_t* __restrict__ wb) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
-    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * ((mi / bc1) / (sqrtf(vi / bc2) + eps) + wd * w[i]);
-    w[i] = wi;
-    if (wb) wb[i] = f2bf(wi);
+ * 2019) on float32 master weights; bc1 = 1 - beta1^t and bc2 = 1 - beta2^t. */
+__device__ __forceinline__ float adam_step(const AdamArgs& q, float w, float& m, float& v, float g) {
+    m = q.beta1 * m + (1.f - q.beta1) * g;
+    v = q.beta2 * v + (1.f - q.beta2) * g * g;
+    return w - q.lr * ((m / q.bc1) / (sqrtf(v / q.bc2) + q.eps) + q.wd * w);
 }
 
-int launch_adam(float* w, float* m, float* v, const float* g, int64_t n, float lr, float beta1, float beta2, float eps,
-                float bc1, float bc2, float wd, uint16_t* wb, hipStream_t stream) {
-    hipLaunchKernelGGL(k_adam, dim3(blocks_for(n, 256)), dim3(256), 0, stream, w, m, v, g, n, lr, beta1, beta2, eps, bc1,
-                       bc2, wd, wb);
+/* Up to six tensors in one launch, a segment of workgroups each: five of the
+ * model's are smaller than a launch is long (4.6 us each in a launch of its own).
+ * wb (optional) receives the bf16 copy used by the GEMMs. */
+__global__ __launch_bounds__(256) void k_adam(AdamSegs S, AdamArgs q) {
+    int k = 0;
+    while (k + 1 < S.count && (int64_t)blockIdx.x >= S.seg[k + 1].block0) k++;
+    const AdamSeg& t = S.seg[k];
+    const int64_t i = (blockIdx.x - t.block0) * 256 + threadIdx.x;
+    if (i >= t.n) return;
+    q.wd = t.wd;
+    float mi = t.m[i], vi = t.v[i];
+    const float wi = adam_step(q, t.w[i], mi, vi, t.g[i]);
+    t.m[i] = mi;
+    t.v[i] = vi;
+    t.w[i] = wi;
+    if (t.wb) t.wb[i] = f2bf(wi);
+}
+
+/* The gradient A B^T (as k_gemm_nt, no split) and Adam on its weights in one
+ * pass: the gradient of a tile goes from the accumulators into the step and is
+ * written only where KEEP asks for it.  The input layer's step is bound by
+ * memory: its 67 M weights take 12 bytes in and 14 out each, 1.7 GB; writing the
+ * gradient and reading it back added 0.54 GB, and a launch of its own kept the
+ * matrix cores idle.  The tile goes through LDS, so that half a wave moves 512
+ * neighbouring bytes of a row: rows lie a power of two (256 KB) apart, and sixteen
+ * rows of 64 bytes, as the accumulators hold them, meet in the same memory channels.
+ * A thread loads eight rows' vectors before the first is used.  Eight neighbouring
+ * workgroups, one per XCD, take eight column tiles, and each XCD runs through the
+ * row tiles of its own column tile, whose rows of B then stay in its L2.
+ * Batch 512, 65536 x 1024 weights: 415 us; the product and the step in two launches
+ * 134 + 345 us; without the way through LDS 502 us. */
+template <bool KEEP>
+__global__ __launch_bounds__(256, 2) void k_gemm_adam(const uint16_t* __restrict__ A, int64_t lda,
+                                                   const uint16_t* __restrict__ B, int64_t ldb, int mtiles, int nk,
+                                                   float* __restrict__ w, float* __restrict__ m, float* __restrict__ v,
+                                                   float* __restrict__ g, int64_t ldc, AdamArgs q,
+                                                   uint16_t* __restrict__ wb) {
+    union Lds {
+        GemmLds tiles;
+        float g[GEMM_BM][GEMM_BN + 4];
+    };
+    __shared__ __attribute__((aligned(16))) Lds L;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t group = blockIdx.x / (8 * mtiles), in = blockIdx.x % (8 * mtiles);
+    const int64_t m0 = in / 8 * GEMM_BM, n0 = (group * 8 + in % 8) * GEMM_BN;
+    f32x4 acc[4][4];
+    gemm_tile<true>(L.tiles, A + m0 * lda, lda, B + n0 * ldb, ldb, nk, acc); /* ends at a barrier */
+    const int lr = threadIdx.x >> 5, lc = (threadIdx.x & 31) * 4;
+    const int64_t at0 = (m0 + lr) * ldc + n0 + lc;
+    constexpr int NB = 8; /* rows a thread has in flight: 24 vectors */
+    f32x4 w4[NB], m4[NB], v4[NB];
+#pragma unroll
+    for (int h = 0; h < GEMM_BM / 8 / NB; h++) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int64_t at = at0 + (int64_t)(h * NB + j) * 8 * ldc;
+            w4[j] = *(const f32x4*)(w + at);
+            m4[j] = *(const f32x4*)(m + at);
+            v4[j] = *(const f32x4*)(v + at);
+        }
+        if (h == 0) { /* the tile to LDS while the first rows are on their way */
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    *(f32x4*)&L.g[(wv >> 1) * 64 + i * 16 + (lane & 15)][(wv & 1) * 64 + j * 16 + (lane >> 4) * 4] =
+                        acc[i][j];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int row = (h * NB + j) * 8;
+            const int64_t at = at0 + (int64_t)row * ldc;
+            const f32x4 g4 = *(const f32x4*)&L.g[row + lr][lc];
+            uint16_t b[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                float mr = m4[j][r], vr = v4[j][r];
+                const float wr = adam_step(q, w4[j][r], mr, vr, g4[r]);
+                w4[j][r] = wr;
+                m4[j][r] = mr;
+                v4[j][r] = vr;
+                b[r] = f2bf(wr);
+            }
+            *(f32x4*)(w + at) = w4[j];
+            *(f32x4*)(m + at) = m4[j];
+            *(f32x4*)(v + at) = v4[j];
+            if (KEEP) *(f32x4*)(g + at) = g4;
+            *(uint2*)(wb + at) =
+                make_uint2((uint32_t)b[0] | (uint32_t)b[1] << 16, (uint32_t)b[2] | (uint32_t)b[3] << 16);
+        }
+    }
+}
+
+int launch_gemm_adam(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, int M, int N, int K, float* w,
+                     float* m, float* v, float* g, bool keep_g, const AdamArgs& q, uint16_t* wb, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || M % GEMM_BM || N % (8 * GEMM_BN) || K % GEMM_BK || lda % 8 || ldb % 8 ||
+        lda < K || ldb < K || !wb)
+        return (int)hipErrorInvalidValue;
+    const int mtiles = M / GEMM_BM;
+    hipLaunchKernelGGL(keep_g ? k_gemm_adam<true> : k_gemm_adam<false>, dim3((unsigned)(mtiles * (N / GEMM_BN))),
+                       dim3(256), 0, stream, A, lda, B, ldb, mtiles, K / GEMM_BK, w, m, v, g, (int64_t)N, q, wb);
+    return (int)hipGetLastError();
+}
+
+int launch_adam(AdamSegs& S, const AdamArgs& q, hipStream_t stream) {
+    if (S.count <= 0 || S.count > 6) return (int)hipErrorInvalidValue;
+    int64_t blocks = 0;
+    for (int k = 0; k < S.count; k++) {
+        S.seg[k].block0 = blocks;
+        blocks += (S.seg[k].n + 255) / 256;
+    }
+    hipLaunchKernelGGL(k_adam, dim3((unsigned)blocks), dim3(256), 0, stream, S, q);
     return (int)hipGetLastError();
 }
 

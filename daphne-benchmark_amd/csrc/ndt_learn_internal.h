@@ -63,8 +63,27 @@ int launch_head_bwd(const float* dY, const uint16_t* H2, const uint16_t* W3, int
                     uint16_t* dZ2, uint16_t* dZ2T, float* db2, float* part, hipStream_t stream);
 int launch_relu_bwd(const float* dH, const uint16_t* H, int B, int F, uint16_t* dZT, float* db, float* part,
                     hipStream_t stream);
-int launch_adam(float* w, float* m, float* v, const float* g, int64_t n, float lr, float beta1, float beta2, float eps,
-                float bc1, float bc2, float wd, uint16_t* wb, hipStream_t stream);
+/* one Adam step's settings */
+struct AdamArgs {
+    float lr, beta1, beta2, eps, bc1, bc2, wd;
+};
+/* one tensor of a step over several: its arrays, its weight decay, its first workgroup */
+struct AdamSeg {
+    float *w, *m, *v;
+    const float* g;
+    uint16_t* wb;
+    int64_t n, block0;
+    float wd;
+};
+struct AdamSegs {
+    AdamSeg seg[6];
+    int count;
+};
+int launch_adam(AdamSegs& segs, const AdamArgs& q, hipStream_t stream);
+/* gradient A B^T [M x N] and Adam on w, m, v, wb of that shape in one launch; g
+ * receives the gradient if keep_g (M % 128 = 0, N % 1024 = 0, K % 64 = 0) */
+int launch_gemm_adam(const uint16_t* A, int64_t lda, const uint16_t* B, int64_t ldb, int M, int N, int K, float* w,
+                     float* m, float* v, float* g, bool keep_g, const AdamArgs& q, uint16_t* wb, hipStream_t stream);
 int launch_sum_ordered(const float* x, int n, float* out, hipStream_t stream);
 int launch_to_bf16(const float* x, int64_t n, uint16_t* out, hipStream_t stream);
 

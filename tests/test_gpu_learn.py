@@ -394,3 +394,45 @@ def test_registered_warm_start_saves_passes(A, trained):
     assert pl < 0.8 * pp, (pp, pl)
     assert np.mean([r["converged"] for r in res]) >= np.mean([r["converged"] for r in plain])
     assert _success(res, t["ev_gt"]).mean() >= _success(plain, t["ev_gt"]).mean()
+
+
+@pytest.mark.parametrize("dims", [(128, 128, 128), (1024, 256, 512)])
+def test_train_steps_the_input_layer_with_its_gradient(A, ctx, small_scene, dims):
+    """A run of one step against backward and Adam called one by one on the same rows:
+    the batch is the whole dataset, so both see the same samples, in another order.
+    W1's gradient of the step can be read after the run; it differs from the one of
+    the given order by float32 sums and bf16 roundings (the tolerance of the gradients
+    above), and the weights are Adam's of it: a dozen operations of half an ulp each on
+    a step of at most lr, and the half ulp of the sum."""
+    f1, f2, B = dims
+    w = small_scene
+    r = np.random.default_rng(f1)
+    idx = (np.arange(B) % len(w.scans)).astype(np.int32)
+    gt = np.asarray(w.gt)[idx]
+    guesses = A.perturb_poses(gt, r)
+    sc, bm = A.Scans(ctx, w.scans), A.BevMap(ctx, w.map_xyzw)
+    m = A.Model(ctx, f1=f1, f2=f2, seed=2)
+    ref = A.Model(ctx, f1=f1, f2=f2, seed=2)
+    w0 = m.get(0)
+    lr = 1e-3
+    m.train(A.Dataset(ctx, bm, sc, idx, guesses, gt), A.train_params(epochs=1, batch=B, lr=lr, cosine=0))
+    g, w1 = m.grad(0), m.get(0).astype(np.float64)
+    scale = np.array([3.0, 3.0, 1.0, 0.05, 0.05, 0.2])  # of the model's outputs
+    target = np.array([L.correction_params(a, b) / scale for a, b in zip(guesses, gt)], np.float32)
+    ref.backward(bm.features(sc, idx, guesses), target)
+    gr = ref.grad(0).astype(np.float64)
+    assert np.linalg.norm(g - gr) < 2e-2 * np.linalg.norm(gr)
+    we, _, _ = L.adam_step(w0.astype(np.float64), 0.0, 0.0, g.astype(np.float64), 1, lr)
+    assert np.abs(w1 - we).max() <= 2.0 ** -24 * (np.abs(w0).max() + lr) + 1e-5 * lr
+    # the weights the forward pass multiplies are the stepped ones, to bf16
+    m2 = A.Model(ctx, f1=f1, f2=f2, seed=2)
+    for k in range(6):
+        m2.set(k, m.get(k))
+    xb = bm.features(sc, idx[:128], guesses[:128])
+    assert np.array_equal(m.forward(xb), m2.forward(xb))
+    # two steps, one per epoch: only the last one's gradient is kept, and it is the last one's
+    m3 = A.Model(ctx, f1=f1, f2=f2, seed=2)
+    m3.train(A.Dataset(ctx, bm, sc, idx, guesses, gt), A.train_params(epochs=2, batch=B, lr=lr, cosine=0))
+    m.train(A.Dataset(ctx, bm, sc, idx, guesses, gt), A.train_params(epochs=1, batch=B, lr=lr, cosine=0, seed=7))
+    a, b = m3.grad(0).astype(np.float64), m.grad(0).astype(np.float64)
+    assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(a)
