@@ -839,9 +839,22 @@ int launch_transpose_u16(const uint16_t* src, int64_t rows, int64_t cols, uint16
  * D[4 (l / 16) + r][l mod 16], r = 0..3.  A and B take their K values from the
  * same positions, so the product is independent of how the hardware orders the
  * K values inside one lane's 8.  K steps of 64 are staged through two LDS
- * buffers: the next step's global loads are in flight while the current one is
- * multiplied.  Rows are padded by 8 elements (16 bytes). */
+ * buffers and two register sets: a step's global loads are issued two products
+ * before it is stored, as one product (about 2 us with two workgroups on a CU) does
+ * not cover the memory's latency under load.  Rows are padded by 8 elements (16
+ * bytes).
+ *
+ * Workgroups go round the 8 XCDs in launch order.  Where the splits are a multiple
+ * of 8, an XCD takes all tiles of a split, so that its L2 fetches every operand once;
+ * in launch order each XCD would hold one column of tiles and fetch all of A.  Fewer
+ * splits (many tiles, or a short K) leave too few for that and keep the launch order.
+ *
+ * 512 x 1024 x 65536 in 16 splits, bound by the latency of the operands' loads:
+ * 131 us with loads one product ahead, 124 us two ahead, 118 us with the splits on
+ * XCDs as well (580 TFLOP/s); the splits on XCDs alone gave 130 us. */
 constexpr int GPAD = 8;
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct GemmLds {
     uint16_t a[2][GEMM_BM][GEMM_BK + GPAD];
@@ -857,34 +870,36 @@ __device__ __forceinline__ void gemm_tile(GemmLds& L, const uint16_t* __restrict
                                           const uint16_t* __restrict__ Bb, int64_t ldb, int nk, f32x4 (&acc)[4][4]) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int wm = w >> 1, wn = w & 1;
-    uint4 ra[4], rb[4];
+    /* two register sets, a K step each: loads are two products ahead of their use */
+    u32x4 a0[4], b0[4], a1[4], b1[4];
     /* tile chunk c = tid + 256 q (q = 0..3): row c / 8, columns 8 (c mod 8) .. +7 */
     const int lr = tid >> 3, lc = (tid & 7) * 8;
+    const uint16_t *pa = Ab + (int64_t)lr * lda + lc, *pb = Bb + (int64_t)lr * ldb + lc;
+    /* K step kt (steps past the last reload it: in bounds, unused) */
+    auto load = [&](u32x4(&ra)[4], u32x4(&rb)[4], int kt) __attribute__((always_inline)) {
+        int64_t ko = (int64_t)(kt < nk ? kt : nk - 1) * GEMM_BK, sa = 32 * lda, sb = 32 * ldb;
+        /* hides the strides, so that addresses are made from two pointers each time: kept
+         * over the loop they take 64 registers, which spill */
+        asm volatile("" : "+s"(sa), "+s"(sb));
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        ra[q] = *(const uint4*)(Ab + (int64_t)(lr + 32 * q) * lda + lc);
-        rb[q] = *(const uint4*)(Bb + (int64_t)(lr + 32 * q) * ldb + lc);
-    }
+        for (int q = 0; q < 4; q++) {
+            ra[q] = *(const u32x4*)(pa + (ko + q * sa));
+            rb[q] = *(const u32x4*)(pb + (ko + q * sb));
+        }
+    };
+    auto store = [&](int s, const u32x4(&ra)[4], const u32x4(&rb)[4]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        *(uint4*)&L.a[0][lr + 32 * q][lc] = ra[q];
-        *(uint4*)&L.b[0][lr + 32 * q][lc] = rb[q];
-    }
-    __syncthreads();
+        for (int q = 0; q < 4; q++) {
+            *(u32x4*)&L.a[s][lr + 32 * q][lc] = ra[q];
+            *(u32x4*)&L.b[s][lr + 32 * q][lc] = rb[q];
+        }
+    };
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     const int fr = lane & 15, fk = (lane >> 4) * 8;
-    for (int kt = 0; kt < nk; kt++) {
-        const int buf = kt & 1;
-        /* next K step (the last iteration reloads its own step: in bounds, unused) */
-        const int64_t ko = (int64_t)(kt + 1 < nk ? kt + 1 : kt) * GEMM_BK;
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            ra[q] = *(const uint4*)(Ab + (int64_t)(lr + 32 * q) * lda + ko + lc);
-            rb[q] = *(const uint4*)(Bb + (int64_t)(lr + 32 * q) * ldb + ko + lc);
-        }
+    auto multiply = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int kk = 0; kk < GEMM_BK; kk += 32) {
             bf16x8 a[4], bv[4];
@@ -899,27 +914,46 @@ __device__ __forceinline__ void gemm_tile(GemmLds& L, const uint16_t* __restrict
                     acc[i][j] = ROWS ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv[j], a[i], acc[i][j], 0, 0, 0)
                                      : __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], bv[j], acc[i][j], 0, 0, 0);
         }
-        /* the other buffer was last read in the previous iteration, before its barrier */
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            *(uint4*)&L.a[buf ^ 1][lr + 32 * q][lc] = ra[q];
-            *(uint4*)&L.b[buf ^ 1][lr + 32 * q][lc] = rb[q];
-        }
+    };
+    load(a0, b0, 0);
+    load(a1, b1, 1);
+    store(0, a0, b0);
+    load(a0, b0, 2);
+    __syncthreads();
+    for (int kt = 0;; kt += 2) {
+        multiply(0);
+        store(1, a1, b1); /* step kt + 1: that buffer was last read before the last barrier */
+        load(a1, b1, kt + 3);
         __syncthreads();
+        if (kt + 1 >= nk) break;
+        multiply(1);
+        store(0, a0, b0);
+        load(a0, b0, kt + 4);
+        __syncthreads();
+        if (kt + 2 >= nk) break;
     }
 }
 
-__global__ __launch_bounds__(256) void k_gemm_nt(const uint16_t* __restrict__ A, int64_t lda,
+__global__ __launch_bounds__(256, 2) void k_gemm_nt(const uint16_t* __restrict__ A, int64_t lda,
                                                  const uint16_t* __restrict__ B, int64_t ldb, float* __restrict__ C,
                                                  int64_t ldc, int64_t split_stride, int kps) {
     __shared__ __attribute__((aligned(16))) GemmLds L;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int wm = w >> 1, wn = w & 1, fr = lane & 15;
-    const int64_t m0 = (int64_t)blockIdx.y * GEMM_BM, n0 = (int64_t)blockIdx.x * GEMM_BN;
-    const int64_t k0 = (int64_t)blockIdx.z * kps;
+    int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
+    if (gridDim.z % 8 == 0) {
+        const int tiles = gridDim.x * gridDim.y;
+        const int id = bx + gridDim.x * by + tiles * bz;
+        const int tile = (id >> 3) % tiles;
+        bz = (id >> 3) / tiles * 8 + (id & 7);
+        bx = tile % gridDim.x;
+        by = tile / gridDim.x;
+    }
+    const int64_t m0 = (int64_t)by * GEMM_BM, n0 = (int64_t)bx * GEMM_BN;
+    const int64_t k0 = (int64_t)bz * kps;
     f32x4 acc[4][4];
     gemm_tile<false>(L, A + m0 * lda + k0, lda, B + n0 * ldb + k0, ldb, kps / GEMM_BK, acc);
-    float* Cz = C + (int64_t)blockIdx.z * split_stride;
+    float* Cz = C + (int64_t)bz * split_stride;
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -1206,7 +1240,7 @@ __global__ __launch_bounds__(256) void k_adam(AdamSegs S, AdamArgs q) {
  * A thread loads eight rows' vectors before the first is used.  Eight neighbouring
  * workgroups, one per XCD, take eight column tiles, and each XCD runs through the
  * row tiles of its own column tile, whose rows of B then stay in its L2.
- * Batch 512, 65536 x 1024 weights: 415 us; the product and the step in two launches
+ * Batch 512, 65536 x 1024 weights: 402 us; the product and the step in two launches
  * 134 + 345 us; without the way through LDS 502 us. */
 template <bool KEEP>
 __global__ __launch_bounds__(256, 2) void k_gemm_adam(const uint16_t* __restrict__ A, int64_t lda,
