@@ -15,7 +15,6 @@
 #include <new>
 #include <atomic>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "ndt_hip.h"
@@ -329,33 +328,50 @@ static bool gather_points(float* dst, const float* const* arrays, const int64_t*
 constexpr size_t UPLOAD_PIECE = (size_t)2 << 20;
 constexpr int UPLOAD_RING = 6;
 
-/* `head_bytes` (a multiple of 256) and the t points of S arrays behind them to dst.  With
- * `finite`, NDT_ERR_INVALID if a point's x, y or z is not finite (parts of the upload may
- * have been made).  The arrays are free when this returns. */
-static int upload_points(ndt_ctx* c, char* dst, const void* head, size_t head_bytes, const float* const* arrays,
-                         const int64_t* offsets, int32_t S, int64_t t, bool finite) {
-    const size_t bytes = sizeof(float4) * (size_t)t;
-    const int64_t step = (int64_t)(UPLOAD_PIECE / sizeof(float4));
-    const int64_t pieces = (t + step - 1) / step, half = UPLOAD_RING / 2;
+/* `head_bytes` (a multiple of 256) to dst and the points of S arrays behind them, in groups
+ * of the points before ends[0], ends[1], ...: each group's points go to the same place, and
+ * done(g) enqueues what reads them before the next group's overwrite them (more than one
+ * group: more points than the ring holds).  With `finite`, NDT_ERR_INVALID if a point's x, y
+ * or z is not finite (parts of the upload may have been made).  The arrays are free when
+ * this returns. */
+template <class Done>
+static int upload_groups(ndt_ctx* c, char* dst, const void* head, size_t head_bytes, const float* const* arrays,
+                         const int64_t* offsets, int32_t S, const int64_t* ends, int32_t ngroups, bool finite,
+                         const Done& done) {
+    const size_t bytes = sizeof(float4) * (size_t)ends[ngroups - 1];
+    const int64_t step = (int64_t)(UPLOAD_PIECE / sizeof(float4)), half = UPLOAD_RING / 2;
+    const bool wraps = bytes > UPLOAD_RING * UPLOAD_PIECE;
     char* stage = nullptr;
     int err = pinned_stage(c, head_bytes + std::min(bytes, UPLOAD_RING * UPLOAD_PIECE), &stage);
     if (err) return err;
     if (head_bytes) std::memcpy(stage, head, head_bytes);
-    for (int64_t k = 0; k < pieces; k++) {
-        const int64_t p0 = k * step, p1 = std::min(t, p0 + step);
-        /* the ring's halves are filled again once the copies from them have completed */
-        if (k >= UPLOAD_RING && k % half == 0) HIP_TRY(hipEventSynchronize(c->ev_stage[k / half & 1]));
-        char* d = stage + head_bytes + UPLOAD_PIECE * (size_t)(k % UPLOAD_RING);
-        if (!gather_points((float*)d, arrays, offsets, S, p0, p1, finite))
-            return fail(NDT_ERR_INVALID, "compat mode needs finite map points");
-        const size_t lead = k == 0 ? head_bytes : 0;
-        c->pin_pending = true;
-        HIP_TRY(hipMemcpyAsync(dst + head_bytes - lead + sizeof(float4) * (size_t)p0, d - lead,
-                               lead + sizeof(float4) * (size_t)(p1 - p0), hipMemcpyHostToDevice, c->stream));
-        if (pieces > UPLOAD_RING && (k + 1) % half == 0)
-            HIP_TRY(hipEventRecord(c->ev_stage[k / half & 1], c->stream));
+    int64_t k = 0, p0 = 0;
+    for (int32_t g = 0; g < ngroups; g++) {
+        const int64_t first = p0;
+        for (; p0 < ends[g]; k++) {
+            const int64_t p1 = std::min(ends[g], p0 + step);
+            /* the ring's halves are filled again once the copies from them have completed */
+            if (k >= UPLOAD_RING && k % half == 0) HIP_TRY(hipEventSynchronize(c->ev_stage[k / half & 1]));
+            char* d = stage + head_bytes + UPLOAD_PIECE * (size_t)(k % UPLOAD_RING);
+            if (!gather_points((float*)d, arrays, offsets, S, p0, p1, finite))
+                return fail(NDT_ERR_INVALID, "compat mode needs finite map points");
+            const size_t lead = k == 0 ? head_bytes : 0;
+            c->pin_pending = true;
+            HIP_TRY(hipMemcpyAsync(dst + head_bytes - lead + sizeof(float4) * (size_t)(p0 - first), d - lead,
+                                   lead + sizeof(float4) * (size_t)(p1 - p0), hipMemcpyHostToDevice, c->stream));
+            if (wraps && (k + 1) % half == 0) HIP_TRY(hipEventRecord(c->ev_stage[k / half & 1], c->stream));
+            p0 = p1;
+        }
+        err = done(g);
+        if (err) return err;
     }
     return 0;
+}
+
+/* n points to dst, as above */
+static int upload_points(ndt_ctx* c, DevBuf& dst, const float* points, int64_t n, bool finite) {
+    const int64_t first = 0;
+    return upload_groups(c, dst.as<char>(), nullptr, 0, &points, &first, 1, &n, 1, finite, [](int32_t) { return 0; });
 }
 
 /* bounding box of the m points in c->pts, as ordered words (minima, maxima) */
@@ -376,11 +392,8 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     const double res = (double)g->params.resolution;
     int e = 0;
     BUF_TRY(c->pts, sizeof(float4) * m);
-    {
-        const int64_t first = 0;
-        e = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, false);
-        if (e) return e;
-    }
+    e = upload_points(c, c->pts, map, m, false);
+    if (e) return e;
     uint32_t h_mm[6];
     e = map_bounds(c, m, h_mm);
     if (e) return e;
@@ -587,8 +600,7 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
     /* initCompute, src/CPU/ndt_mapping/kernel.cpp:1302-1373 */
     const float res = g->params.resolution;
     BUF_TRY(c->pts, sizeof(float4) * m);
-    const int64_t first = 0;
-    int e = upload_points(c, c->pts.as<char>(), nullptr, 0, &map, &first, 1, m, true);
+    int e = upload_points(c, c->pts, map, m, true);
     if (e) return e;
     uint32_t h_mm[6];
     e = map_bounds(c, m, h_mm);
@@ -944,64 +956,137 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     return results_from_out(out, counts, S, aborted, c, results, used_alt);
 }
 
+/* The scans ordered on the host, for want of device memory to order them there. */
+static int pack_scans_host(ndt_ctx* c, DevBuf& dst, const float* const* scans, const int64_t* counts, int32_t S,
+                           const std::vector<int64_t>& offsets, int64_t t) {
+    try {
+        std::vector<float> points((size_t)(4 * t));
+        std::vector<uint64_t> key; /* place on the curve, then place in the scan */
+        for (int32_t s = 0; s < S; s++) {
+            key.resize((size_t)counts[s]);
+            for (size_t i = 0; i < key.size(); i++) {
+                const float* p = scans[s] + 4 * i;
+                key[i] = ((uint64_t)curve_key(p[0], p[1], p[2]) << 32) | i;
+            }
+            std::sort(key.begin(), key.end());
+            float* d = points.data() + 4 * offsets[s];
+            for (size_t i = 0; i < key.size(); i++) std::memcpy(d + 4 * i, scans[s] + 4 * (key[i] & 0xffffffffu), 16);
+        }
+        return upload_points(c, dst, points.data(), t, false);
+    } catch (const std::bad_alloc&) {
+        return fail(NDT_ERR_NOMEM, "host allocation failed");
+    }
+}
+
 /* Copies scans into one device buffer, each scan's points reordered along a Morton
  * curve of 1 m cells of its own (sensor-frame) coordinates: consecutive points,
  * and so the points of one workgroup, then look up neighbouring voxels and hit the
  * same cache lines.  A rigid transform keeps that locality.  The alignment does not
  * depend on the point order beyond floating-point rounding of the sums.  The points go
- * to the device as they are and are ordered there; the work is enqueued on the context's
- * stream, and the callers' buffers are free when this returns. */
+ * to the device as they are and are ordered there, a group at a time; the work is
+ * enqueued on the context's stream, and the callers' buffers are free when this returns.
+ * Ordering takes 25 bytes a point of a group beside the 16 of the points' place (raw
+ * points, a key and an index, tile counts), about 105 MB at most, which the context keeps;
+ * for a scan larger than a group it is given back.  Where the device has no room for it, the
+ * points are ordered on the host. */
 static int pack_scans(ndt_ctx* c, DevBuf& dst, const float* const* scans, const int64_t* counts, int32_t S,
                       std::vector<int64_t>& offsets, int64_t* total) {
+    struct Group {
+        int32_t seg0, nsmall, nlarge; /* its scans' segments: small ones, then larger ones */
+        int64_t tile0, ntiles;
+    };
+    std::vector<Group> groups;
+    std::vector<int64_t> ends;
     offsets.assign(S, 0);
-    int64_t t = 0, ntiles = 0;
-    int32_t nsmall = 0;
+    int64_t t = 0, ntiles = 0, most = 0, most_order = 0;
     for (int32_t s = 0; s < S; s++) {
         if (!scans[s] || counts[s] <= 0) return fail(NDT_ERR_INVALID, "empty or null scan");
         if (counts[s] > 0x7fffffffll) return fail(NDT_ERR_UNSUPPORTED, "scan larger than 2^31 points");
+        const int64_t begin = ends.size() > 1 ? ends[ends.size() - 2] : 0;
+        if (ends.empty() || t + counts[s] - begin > ORDER_GROUP) {
+            groups.push_back({s, 0, 0, ntiles, 0});
+            ends.push_back(t);
+        }
         offsets[s] = t;
         t += counts[s];
-        if (counts[s] <= ORDER_SMALL) nsmall++;
-        else ntiles += (counts[s] + ORDER_TILE - 1) / ORDER_TILE;
+        Group& g = groups.back();
+        if (counts[s] <= ORDER_SMALL) {
+            g.nsmall++;
+        } else {
+            g.nlarge++;
+            g.ntiles += (counts[s] + ORDER_TILE - 1) / ORDER_TILE;
+            ntiles += (counts[s] + ORDER_TILE - 1) / ORDER_TILE;
+        }
+        ends.back() = t;
     }
-    if (ntiles > 0x7fffffffll) return fail(NDT_ERR_UNSUPPORTED, "scans larger than 2^43 points together");
-    /* the small scans' segments, the larger ones', then their tiles */
+    const int32_t ngroups = (int32_t)groups.size();
+    for (int32_t k = 0; k < ngroups; k++) {
+        const int64_t n = ends[k] - (k ? ends[k - 1] : 0);
+        most = std::max(most, n);
+        if (groups[k].ntiles)
+            most_order = std::max<int64_t>(most_order, sizeof(uint32_t) * (2 * n + ORDER_HIST_WORDS * groups[k].ntiles));
+    }
+    /* the groups' segments, then their tiles */
     const size_t seg_bytes = sizeof(OrderSeg) * (size_t)S;
     const size_t head_bytes = (seg_bytes + sizeof(OrderTile) * (size_t)ntiles + 255) & ~(size_t)255;
-    const size_t words = sizeof(uint32_t) * (size_t)t;
     BUF_TRY(dst, sizeof(float4) * t);
-    BUF_TRY(c->raw, head_bytes + sizeof(float4) * (size_t)t);
-    if (ntiles > 0) BUF_TRY(c->order, 2 * words + sizeof(uint32_t) * ORDER_HIST_WORDS * (size_t)ntiles);
+    *total = t;
+    int e = c->raw.ensure(head_bytes + sizeof(float4) * (size_t)most);
+    if (!e && most_order) e = c->order.ensure((size_t)most_order);
+    if (e == NDT_ERR_NOMEM) {
+        c->raw.release();
+        c->order.release();
+        return pack_scans_host(c, dst, scans, counts, S, offsets, t);
+    }
+    if (e) return e;
     std::vector<char> head(head_bytes);
     OrderSeg* segs = (OrderSeg*)head.data();
     OrderTile* tiles = (OrderTile*)(head.data() + seg_bytes);
-    int32_t small = 0, large = nsmall, tile = 0;
-    for (int32_t s = 0; s < S; s++) {
-        OrderSeg sg{offsets[s], (int32_t)counts[s], 0, 0, 0};
-        if (counts[s] <= ORDER_SMALL) {
-            segs[small++] = sg;
-            continue;
+    for (int32_t k = 0, s = 0; k < ngroups; k++) {
+        const Group& g = groups[k];
+        const int64_t begin = k ? ends[k - 1] : 0;
+        OrderSeg *small = segs + g.seg0, *large = small + g.nsmall;
+        OrderTile* tile = tiles + g.tile0;
+        int32_t nlarge = 0, done = 0;
+        for (const int32_t last = s + g.nsmall + g.nlarge; s < last; s++) {
+            OrderSeg sg{offsets[s] - begin, (int32_t)counts[s], 0, 0, 0};
+            if (counts[s] <= ORDER_SMALL) {
+                *small++ = sg;
+                continue;
+            }
+            sg.tile0 = done;
+            for (int64_t p = 0; p < counts[s]; p += ORDER_TILE)
+                tile[done++] = {sg.offset + p, (int32_t)std::min<int64_t>(ORDER_TILE, counts[s] - p), nlarge};
+            sg.ntiles = done - sg.tile0;
+            large[nlarge++] = sg;
         }
-        sg.tile0 = tile;
-        for (int64_t p = 0; p < counts[s]; p += ORDER_TILE)
-            tiles[tile++] = {offsets[s] + p, (int32_t)std::min<int64_t>(ORDER_TILE, counts[s] - p), large - nsmall};
-        sg.ntiles = tile - sg.tile0;
-        segs[large++] = sg;
     }
-    int e = upload_points(c, c->raw.as<char>(), head.data(), head_bytes, scans, offsets.data(), S, t, false);
-    if (e) return e;
     const OrderSeg* d_segs = c->raw.as<OrderSeg>();
     const OrderTile* d_tiles = (const OrderTile*)(c->raw.as<char>() + seg_bytes);
     const float4* raw = (const float4*)(c->raw.as<char>() + head_bytes);
-    if (ntiles > 0) {
-        /* the passes' second key and index arrays lie in dst: the last pass, which
-         * writes the points there, reads the first ones */
-        uint32_t *w = c->order.as<uint32_t>(), *w2 = dst.as<uint32_t>();
-        LAUNCH_TRY(launch_order_large(raw, d_segs + nsmall, S - nsmall, d_tiles, (int)ntiles, w, w2, w + t, w2 + t,
-                                      w + 2 * t, dst.as<float4>(), c->stream));
+    const auto order = [&](int32_t k) -> int {
+        const Group& g = groups[k];
+        const int64_t begin = k ? ends[k - 1] : 0, n = ends[k] - begin;
+        float4* to = dst.as<float4>() + begin;
+        if (g.nlarge > 0) {
+            /* the passes' second key and index arrays lie in dst: the last pass, which
+             * writes the points there, reads the first ones */
+            uint32_t *w = c->order.as<uint32_t>(), *w2 = (uint32_t*)to;
+            LAUNCH_TRY(launch_order_large(raw, d_segs + g.seg0 + g.nsmall, g.nlarge, d_tiles + g.tile0, (int)g.ntiles, w,
+                                          w2, w + n, w2 + n, w + 2 * n, to, c->stream));
+        }
+        if (g.nsmall > 0) LAUNCH_TRY(launch_order_small(raw, d_segs + g.seg0, g.nsmall, to, c->stream));
+        return 0;
+    };
+    e = upload_groups(c, c->raw.as<char>(), head.data(), head_bytes, scans, offsets.data(), S, ends.data(), ngroups, false,
+                      order);
+    if (e) return e;
+    if (most > ORDER_GROUP) {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        c->pin_pending = false;
+        c->raw.release();
+        c->order.release();
     }
-    if (nsmall > 0) LAUNCH_TRY(launch_order_small(raw, d_segs, nsmall, dst.as<float4>(), c->stream));
-    *total = t;
     return 0;
 }
 
@@ -1528,11 +1613,8 @@ extern "C" int ndt_derivatives(ndt_ctx* c, const ndt_grid* g, const float* scan,
     if (params->mode != g->params.mode) return fail(NDT_ERR_INVALID, "params mode differs from the grid's");
     HIP_TRY(hipSetDevice(c->device));
     BUF_TRY(c->pts, sizeof(float4) * n);
-    {
-        const int64_t first = 0;
-        e = upload_points(c, c->pts.as<char>(), nullptr, 0, &scan, &first, 1, n, false);
-        if (e) return e;
-    }
+    e = upload_points(c, c->pts, scan, n, false);
+    if (e) return e;
     if (params->mode == NDT_MODE_COMPAT) {
         if (!compat_transform) return fail(NDT_ERR_INVALID, "compat mode needs the transform matrix");
         double d1, d2;

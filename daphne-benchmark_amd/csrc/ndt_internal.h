@@ -448,19 +448,44 @@ struct ScanOut {
  * ORDER_SMALL points one workgroup each, larger ones in tiles of ORDER_TILE points. */
 constexpr int ORDER_SMALL = 8192, ORDER_TILE = 4096;
 constexpr int ORDER_HIST_WORDS = 1024; /* histogram words per tile */
+/* A batch is ordered in groups of whole scans of at most this many points together (a
+ * larger scan is a group of its own), which bounds the work space on the device. */
+constexpr int64_t ORDER_GROUP = (int64_t)1 << 22;
+
+/* spreads the bits of a 10-bit value to every third bit */
+NDT_HD uint32_t spread3(uint32_t v) {
+    v &= 0x3ff;
+    v = (v | (v << 16)) & 0x030000FF;
+    v = (v | (v << 8)) & 0x0300F00F;
+    v = (v | (v << 4)) & 0x030C30C3;
+    v = (v | (v << 2)) & 0x09249249;
+    return v;
+}
+
+/* A point's place on the curve: cells -512 .. 511 m per axis, clamped; a coordinate that
+ * is not finite (v - v is then NaN) counts as the first cell. */
+NDT_HD uint32_t curve_key(float x, float y, float z) {
+    const float v[3] = {x, y, z};
+    uint32_t q[3];
+    for (int k = 0; k < 3; k++) {
+        const double cell = v[k] - v[k] == 0.0f ? floor((double)v[k]) + 512.0 : 0.0;
+        q[k] = (uint32_t)fmin(1023.0, fmax(0.0, cell));
+    }
+    return spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
+}
 struct OrderSeg {
-    int64_t offset; /* first point of the scan */
+    int64_t offset; /* first point of the scan in its group */
     int32_t n;
-    int32_t tile0, ntiles; /* larger scans: its tiles */
+    int32_t tile0, ntiles; /* larger scans: its tiles of the group's */
     int32_t pad;
 };
 struct OrderTile {
-    int64_t start; /* first point */
+    int64_t start; /* first point in the group */
     int32_t n;
-    int32_t seg; /* index of the scan among the larger ones */
+    int32_t seg; /* index of the scan among the group's larger ones */
 };
 int launch_order_small(const float4* raw, const OrderSeg* segs, int nsegs, float4* out, hipStream_t stream);
-/* key_a/b, idx_a/b: a word per point of the batch each; hist: ORDER_HIST_WORDS per tile */
+/* key_a/b, idx_a/b: a word per point of the group each; hist: ORDER_HIST_WORDS per tile */
 int launch_order_large(const float4* raw, const OrderSeg* segs, int nsegs, const OrderTile* tiles, int ntiles,
                        uint32_t* key_a, uint32_t* key_b, uint32_t* idx_a, uint32_t* idx_b, uint32_t* hist, float4* out,
                        hipStream_t stream);

@@ -543,28 +543,6 @@ int radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_tmp, uint32_
  * alignment took 6.2 to 7.9 ms per call; now 3.6, of it 2.4 in the passes. */
 constexpr int ORDER_BITS = 10, ORDER_DIGITS = 1 << ORDER_BITS, ORDER_PASSES = 3;
 
-/* spreads the bits of a 10-bit value to every third bit */
-__device__ inline uint32_t spread3(uint32_t v) {
-    v &= 0x3ff;
-    v = (v | (v << 16)) & 0x030000FF;
-    v = (v | (v << 8)) & 0x0300F00F;
-    v = (v | (v << 4)) & 0x030C30C3;
-    v = (v | (v << 2)) & 0x09249249;
-    return v;
-}
-
-/* cells -512 .. 511 m per axis, clamped; a coordinate that is not finite counts as the
- * first cell */
-__device__ inline uint32_t curve_key(const float4 p) {
-    const float v[3] = {p.x, p.y, p.z};
-    uint32_t q[3];
-    for (int k = 0; k < 3; k++) {
-        const double cell = isfinite(v[k]) ? floor((double)v[k]) + 512.0 : 0.0;
-        q[k] = (uint32_t)fmin(1023.0, fmax(0.0, cell));
-    }
-    return spread3(q[0]) | (spread3(q[1]) << 1) | (spread3(q[2]) << 2);
-}
-
 constexpr int ORDER_SMALL_WAVES = 16;
 __global__ __launch_bounds__(1024) void k_order_small(const float4* __restrict__ raw, const OrderSeg* __restrict__ segs,
                                                       float4* __restrict__ out) {
@@ -577,7 +555,8 @@ __global__ __launch_bounds__(1024) void k_order_small(const float4* __restrict__
     raw += sg.offset;
     out += sg.offset;
     for (int i = tid; i < n; i += 1024) {
-        key[i] = curve_key(raw[i]);
+        const float4 p = raw[i];
+        key[i] = curve_key(p.x, p.y, p.z);
         idx[0][i] = (uint16_t)i;
     }
     /* the wave's points: whole rounds of 64, in order over the waves */
@@ -622,7 +601,8 @@ __global__ __launch_bounds__(256) void k_order_hist(const float4* __restrict__ r
     for (int i = threadIdx.x; i < tl.n; i += 256) {
         uint32_t k;
         if (pass == 0) {
-            k = curve_key(raw[tl.start + i]);
+            const float4 p = raw[tl.start + i];
+            k = curve_key(p.x, p.y, p.z);
             key[tl.start + i] = k;
         } else {
             k = key[tl.start + i];

@@ -1,0 +1,86 @@
+"""What calls take of the device's memory, and what they keep of it."""
+import gc
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LIMIT = "NDT_DEVICE_MEMORY_LIMIT"
+
+
+@pytest.fixture()
+def fresh(A, monkeypatch):
+    """A context of its own, which holds no workspace from other tests."""
+    c = A.Context(0)
+    yield c
+    monkeypatch.delenv(LIMIT, raising=False)
+    c.close()
+
+
+def _held(A, ctx, monkeypatch):
+    """Device bytes that the process's buffers hold: the least limit under which one more
+    point (16 bytes) still finds room, less those (the context has ordered a point before)."""
+    point = np.ones((1, 4), np.float32)
+    A.Scans(ctx, [point]).close()
+    gc.collect()
+    lo, hi = 0, 1 << 38
+    while lo < hi:
+        mid = (lo + hi) // 2
+        monkeypatch.setenv(LIMIT, str(mid))
+        try:
+            A.Scans(ctx, [point]).close()
+            hi = mid
+        except A.NdtError as e:
+            assert e.code == 3
+            lo = mid + 1
+    monkeypatch.delenv(LIMIT)
+    return lo - 16
+
+
+def _scans(A, counts, seed):
+    """Scans of a 100 m scene with repeated, far-off and non-finite points; their guesses."""
+    scene = A.scene_cfg(3, extent=100.0)
+    mp = A.make_map(scene, 100_000)
+    rng = np.random.default_rng(seed)
+    scans, guesses = [], []
+    for k, n in enumerate(counts):
+        scan, _, guess = A.make_scan(scene, mp, A.scan_cfg(min(n, 20000)), 60 + k)
+        scan = np.resize(scan, (n, 4))
+        scan[n // 2:, :3] += rng.uniform(-0.01, 0.01, (n - n // 2, 3)).astype(np.float32)
+        scan[rng.integers(n), 0] = np.nan
+        scan[rng.integers(n), 1] = -900.0
+        scans.append(scan)
+        guesses.append(guess)
+    return mp, scans, guesses
+
+
+@pytest.mark.parametrize("counts", [(1, 700, 8192, 8193, 20481), (3_000_000, 700, 1_500_000, 20_000, 4_400_000, 9_000)])
+def test_upload_fits_where_its_points_do(A, fresh, monkeypatch, counts):
+    """A batch uploads where the device has room for its points and nothing else (they are
+    then ordered on the host), and gives the bits of one ordered on the device, of which
+    the second runs through several groups with one larger than a group's limit."""
+    mp, scans, guesses = _scans(A, counts, 1)
+    grid = A.Grid(fresh, mp, A.params(A.NDT_MODE_NDT))
+    prm = A.params(A.NDT_MODE_NDT, max_iterations=2)
+    held = _held(A, fresh, monkeypatch)
+    monkeypatch.setenv(LIMIT, str(held + 16 * sum(counts) + 1024))
+    tight = A.Scans(fresh, scans)
+    monkeypatch.delenv(LIMIT)
+    roomy = A.Scans(fresh, scans)
+    for a, b in zip(tight.align(grid, guesses, prm), roomy.align(grid, guesses, prm)):
+        assert a["status"] == 0 and a["passes"] == b["passes"] and a["score"] == b["score"]
+        assert np.array_equal(a["final_f64"], b["final_f64"])
+
+
+@pytest.mark.parametrize("counts", [(12_000_000,), (1_000_000,) * 12])
+def test_upload_keeps_a_bounded_workspace(A, fresh, monkeypatch, counts):
+    """Ordering scans leaves the context at most 26 bytes a point of 2^22 points, whatever
+    was uploaded: 16 of raw points, 8 of keys and indices, less than 2 of tile counts and
+    segments."""
+    points = np.random.default_rng(2).uniform(-50, 50, (max(counts), 4)).astype(np.float32)
+    before = _held(A, fresh, monkeypatch)
+    sc = A.Scans(fresh, [points[:n] for n in counts])
+    kept = _held(A, fresh, monkeypatch) - before - 16 * sum(counts)
+    sc.close()
+    assert kept <= 26 << 22
