@@ -176,9 +176,9 @@ int ndt_align_batch(ndt_ctx* ctx, const ndt_grid* grid, const float* const* scan
  * grid and parameters: a scans handle must not be used by two threads at once, even
  * through the const pointer (each thread uploads its own batch).
  * A batch holds 16 bytes of device memory a point.  An upload (and ndt_align,
- * ndt_align_batch) also orders the points, in up to about 105 MB that the context keeps,
- * 25 bytes a point while a scan above 4 M points is ordered, or on the host where the
- * device has no room for that. */
+ * ndt_align_batch) also orders the points: in about 105 MB of device memory, for a scan
+ * above 4 M points in 25 bytes a point, of which the context keeps up to 256 MB; on the
+ * host where the device has no room for that. */
 int ndt_scans_upload(ndt_ctx* ctx, const float* const* scans, const int64_t* counts, int32_t S,
                      ndt_scans** out);
 int ndt_scans_destroy(ndt_scans* scans);
