@@ -318,8 +318,9 @@ static bool gather_points(float* dst, const float* const* arrays, const int64_t*
     return true;
 }
 
-/* Work space of an upload's ordering that a context keeps for the next one; more is given
- * back (allocating and freeing 187 MB takes 0.5 ms of a 6 ms upload of 7.5 M points). */
+/* Work space of an upload's ordering, and of a dense index's build, that a context keeps for
+ * the next one, each; more is given back (allocating and freeing 139 MB takes 0.25 ms, of a
+ * 1.6 ms build of a map of 1 M points in a box of 34 M cells). */
 constexpr size_t WORK_KEEP = (size_t)256 << 20;
 
 /* Uploads of points go through the staging buffer in pieces, at most UPLOAD_RING of them
@@ -392,48 +393,22 @@ static int map_bounds(ndt_ctx* c, int64_t m, uint32_t mm[6]) {
     return 0;
 }
 
-static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) {
+/* cells of the map's box */
+static double cells_of(const ndt_grid* g) {
+    return (double)g->dims[0] * (double)g->dims[1] * (double)g->dims[2];
+}
+
+/* Statistics and indices of the map in c->pts, whose nvalid_pts points with a cell are
+ * sorted by it (c->bk_keys, c->bk_vals, runs at c->bk_starts), with the dense or the
+ * hashed index of query cells. */
+static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pts, bool dense, ndt_grid* g) {
     const double res = (double)g->params.resolution;
-    int e = 0;
-    BUF_TRY(c->pts, sizeof(float4) * m);
-    e = upload_points(c, c->pts, map, m, false);
-    if (e) return e;
-    uint32_t h_mm[6];
-    e = map_bounds(c, m, h_mm);
-    if (e) return e;
-    if (h_mm[0] == 0xFFFFFFFFu) return fail(NDT_ERR_INVALID, "map has no finite points");
-    int64_t lo_cell[3], hi_cell[3];
-    for (int k = 0; k < 3; k++) {
-        lo_cell[k] = (int64_t)std::floor((double)ord2f(h_mm[k]) / res);
-        hi_cell[k] = (int64_t)std::floor((double)ord2f(h_mm[3 + k]) / res);
-        g->origin_cell[k] = lo_cell[k] - 1;
-        g->bits[k] = std::max(1, ceil_log2(hi_cell[k] - lo_cell[k] + 3));
-        g->dims[k] = (int32_t)std::min<int64_t>(hi_cell[k] - lo_cell[k] + 3, 0x7fffffff);
-    }
     const int B = g->bits[0] + g->bits[1] + g->bits[2];
-    if (B + 5 > 62) return fail(NDT_ERR_UNSUPPORTED, "map extent too large for the cell key");
+    const double box = cells_of(g);
     DevBuf &keys = c->bk_keys, &vals = c->bk_vals, &keys_t = c->bk_keys_t, &vals_t = c->bk_vals_t;
     DevBuf &scratch = c->bk_scratch, &starts = c->bk_starts, &sc2 = c->bk_sc2;
-    BUF_TRY(keys, sizeof(uint64_t) * m);
-    BUF_TRY(vals, sizeof(uint32_t) * m);
-    BUF_TRY(keys_t, sizeof(uint64_t) * m);
-    BUF_TRY(vals_t, sizeof(uint32_t) * m);
-    BUF_TRY(scratch, radix_sort_scratch_bytes(m));
-    const uint64_t limit = (1ull << B) - 1; /* the key of points without a cell */
-    LAUNCH_TRY(launch_keys_ndt(c->pts.as<float4>(), m, res, g->origin_cell, g->bits,
-                               (radix_sort_from_tmp(B) ? keys_t : keys).as<uint64_t>(), c->stream));
-    LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
-                                B, true, scratch.p, c->stream));
-    int64_t nvox = 0, nvalid_pts = 0;
-    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, starts, sc2, &nvox, &nvalid_pts);
-    if (e) return e;
-    if (nvox == 0) return fail(NDT_ERR_INVALID, "map has no finite points");
-    /* dense query-cell index when the map's cell box is at most 2^28 cells; the
-     * environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
-     * index, so that tests run that path on maps of every size */
-    const double box = (double)g->dims[0] * (double)g->dims[1] * (double)g->dims[2];
-    const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
-    const bool dense = box <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
+    int e = 0;
+    g->dense.p = g->slots.p = g->fit_begin.p = g->fit_slots.p = nullptr;
     int32_t tiles[2] = {0, 0};
     int64_t ncells = 0;
     if (dense) {
@@ -442,7 +417,7 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
     }
     /* nearest-point queries: the first point of every cell of the box where that takes no
-     * more memory than the hash of the occupied voxels (32 to 64 bytes each) */
+     * more than 64 bytes per occupied voxel, as much as their hash (32 to 64) at its emptiest */
     const bool rows = dense && box <= 16.0 * (double)nvox;
     const int flog2 = std::max(4, ceil_log2(2 * nvox));
     {
@@ -489,18 +464,17 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     g->info.voxels = nvox;
     int64_t nv = 0, ne = 0, nq = 0;
     if (dense) {
-        BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)ncells);
-        BUF_TRY(c->bk_vid, sizeof(uint32_t) * (size_t)ncells);
+        BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)(ncells + ncells / 32));
         BUF_TRY(scratch, cells_scratch_bytes(ncells));
         LAUNCH_TRY(launch_cells_index(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), nvox, g->bits, tiles, ncells,
-                                      c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_vid.as<uint32_t>(),
+                                      c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_mask.as<uint32_t>() + ncells,
                                       scratch.p, (uint64_t*)c->hsmall, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         const uint64_t* h = (const uint64_t*)c->hsmall;
         nv = (int64_t)(h[0] >> 32);
         ne = 27 * nv;
         nq = (int64_t)h[1];
-        if (ne > 0xfffffffell) return fail(NDT_ERR_NOMEM, "more candidates than the index numbers");
+        if (ne > 0xfffffffell) return fail(NDT_ERR_UNSUPPORTED, "more candidates than the index numbers");
     }
     DevBuf vkey_c;
     if (!dense) {
@@ -514,6 +488,7 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         HIP_TRY(hipMemcpyAsync(&h_nvalid, vtotal, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         nv = h_nvalid;
+        if (27 * nv > 0xfffffffell) return fail(NDT_ERR_UNSUPPORTED, "more candidates than the index numbers");
         BUF_TRY(g->mean_c, sizeof(double) * 3 * (nv + 1));
         BUF_TRY(g->icov_c, sizeof(double) * 6 * (nv + 1));
         BUF_TRY(vkey_c, sizeof(uint64_t) * (nv + 1));
@@ -553,7 +528,7 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     if (dense) {
         LAUNCH_TRY(launch_cells_fill(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), g->all_mean.as<double>(),
                                      g->all_icov.as<double>(), nvox, g->bits, g->origin_cell, res, tiles,
-                                     c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_vid.as<uint32_t>(),
+                                     c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_mask.as<uint32_t>() + ncells,
                                      g->cand_head.as<float4>(), g->cand_s32.as<float4>(), g->vs64.as<double2>(),
                                      c->stream));
     } else {
@@ -568,6 +543,7 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
         }
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
+    if (c->bk_mask.bytes > WORK_KEEP) c->bk_mask.release();
     g->info.query_cells = nq;
     g->info.candidates = ne;
     g->info.hash_capacity = cap;
@@ -593,6 +569,58 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     d.res_pow2 = std::frexp(res, &ex) == 0.5 ? 1 : 0;
     d.inv_resolution_d = 1.0 / res;
     return 0;
+}
+
+static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) {
+    const double res = (double)g->params.resolution;
+    int e = 0;
+    BUF_TRY(c->pts, sizeof(float4) * m);
+    e = upload_points(c, c->pts, map, m, false);
+    if (e) return e;
+    uint32_t h_mm[6];
+    e = map_bounds(c, m, h_mm);
+    if (e) return e;
+    if (h_mm[0] == 0xFFFFFFFFu) return fail(NDT_ERR_INVALID, "map has no finite points");
+    int64_t lo_cell[3], hi_cell[3];
+    for (int k = 0; k < 3; k++) {
+        lo_cell[k] = (int64_t)std::floor((double)ord2f(h_mm[k]) / res);
+        hi_cell[k] = (int64_t)std::floor((double)ord2f(h_mm[3 + k]) / res);
+        g->origin_cell[k] = lo_cell[k] - 1;
+        g->bits[k] = std::max(1, ceil_log2(hi_cell[k] - lo_cell[k] + 3));
+        g->dims[k] = (int32_t)std::min<int64_t>(hi_cell[k] - lo_cell[k] + 3, 0x7fffffff);
+    }
+    const int B = g->bits[0] + g->bits[1] + g->bits[2];
+    if (B + 5 > 62) return fail(NDT_ERR_UNSUPPORTED, "map extent too large for the cell key");
+    DevBuf &keys = c->bk_keys, &vals = c->bk_vals, &keys_t = c->bk_keys_t, &vals_t = c->bk_vals_t;
+    DevBuf &scratch = c->bk_scratch, &starts = c->bk_starts, &sc2 = c->bk_sc2;
+    BUF_TRY(keys, sizeof(uint64_t) * m);
+    BUF_TRY(vals, sizeof(uint32_t) * m);
+    BUF_TRY(keys_t, sizeof(uint64_t) * m);
+    BUF_TRY(vals_t, sizeof(uint32_t) * m);
+    BUF_TRY(scratch, radix_sort_scratch_bytes(m));
+    const uint64_t limit = (1ull << B) - 1; /* the key of points without a cell */
+    LAUNCH_TRY(launch_keys_ndt(c->pts.as<float4>(), m, res, g->origin_cell, g->bits,
+                               (radix_sort_from_tmp(B) ? keys_t : keys).as<uint64_t>(), c->stream));
+    LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
+                                B, true, scratch.p, c->stream));
+    int64_t nvox = 0, nvalid_pts = 0;
+    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, starts, sc2, &nvox, &nvalid_pts);
+    if (e) return e;
+    if (nvox == 0) return fail(NDT_ERR_INVALID, "map has no finite points");
+    /* dense query-cell index when the map's cell box is at most 2^28 cells: 4 bytes for
+     * each cell of the box, in whole tiles of 4 x 4 x 2, and 4.1 more while it is built
+     * (2.2 GB for a cube at the limit), or the hashed one where the device has no room for
+     * that; the environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
+     * index, so that tests run that path on maps of every size */
+    const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
+    const bool dense = cells_of(g) <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
+    e = grid_index_ndt(c, m, nvox, nvalid_pts, dense, g);
+    if (dense && e == NDT_ERR_NOMEM) {
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        for (DevBuf* b : {&g->voxel_mem, &g->cand_mem, &c->bk_mask}) b->release();
+        e = grid_index_ndt(c, m, nvox, nvalid_pts, false, g);
+    }
+    return e;
 }
 
 static uint64_t next_grid_serial() {

@@ -185,7 +185,7 @@ struct ndt_ctx {
     /* grid-build temporaries, and the compat callback's grid and scan, kept for
      * reuse: freeing device memory synchronises the device, which would serialise
      * contexts that work concurrently (one per host thread) */
-    DevBuf bk_keys, bk_vals, bk_keys_t, bk_vals_t, bk_scratch, bk_starts, bk_sc2, bk_mm, bk_mask, bk_vid;
+    DevBuf bk_keys, bk_vals, bk_keys_t, bk_vals_t, bk_scratch, bk_starts, bk_sc2, bk_mm, bk_mask;
     DevBuf compat_scan;
     ndt_grid* compat_grid = nullptr;
     /* pinned staging buffer for host-to-device uploads; pin_pending while a copy

@@ -535,17 +535,18 @@ int launch_voxel_stats_compat(const float4* pts, const uint32_t* sorted_idx, con
 
 /* ndt alignment: init states from guesses, then the cooperative persistent kernel */
 /* dense query-cell index of the nvox voxels (those with valid[v] take part): run starts
- * begin[0..ncells] and, where a cell holds a valid voxel, its number vid[cell]; mask,
- * begin and vid hold ncells entries (begin one more).  host_totals (pinned host
- * memory) receives candidates and, in the upper half, valid voxels; then query cells. */
+ * begin[0..ncells], and for the entries' making, freed with them, the cells' masks (ncells
+ * words) and the tiles' first voxel numbers tile_vid (a word per 32 cells).  host_totals
+ * (pinned host memory) receives candidates and, in the upper half, valid voxels; then
+ * query cells. */
 size_t cells_scratch_bytes(int64_t ncells);
 int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
-                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
+                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* tile_vid, void* scratch,
                        uint64_t* host_totals, hipStream_t stream);
 /* the candidate entries and float64 statistics behind that index */
 int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double* mean, const double* icov, int64_t nvox,
                       const int* bits, const int64_t* origin_cell, double res, const int32_t* tiles, const uint32_t* mask,
-                      const uint32_t* begin, const uint32_t* vid, float4* head, float4* s32, double2* vs64,
+                      const uint32_t* begin, const uint32_t* tile_vid, float4* head, float4* s32, double2* vs64,
                       hipStream_t stream);
 int launch_gather_points(const float4* pts, const uint32_t* idx, int64_t n, float4* out, hipStream_t stream);
 int launch_fit_rows(const uint64_t* vkey, const uint32_t* starts, int64_t nvox, int64_t npts, const int* bits,

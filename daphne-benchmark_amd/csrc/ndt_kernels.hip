@@ -1186,11 +1186,13 @@ __global__ __launch_bounds__(1024) void k_cells_top(uint64_t* __restrict__ bsum,
     if (threadIdx.x == 0) totals[0] = tot;
 }
 
-/* begin[cell] (begin[ncells] = all candidates), and the number of the valid voxel in
- * each cell that holds one */
-__global__ __launch_bounds__(256) void k_cells_down(const uint32_t* __restrict__ mask, int64_t ncells,
+/* begin[cell] (begin[ncells] = all candidates), the number of the first valid voxel in or
+ * behind each tile (32 cells, two threads), and in a cell that holds one, in the mask's
+ * upper five bits, how many of its tile come before it.  (A word per cell for the numbers
+ * themselves held half as much memory again during the build.) */
+__global__ __launch_bounds__(256) void k_cells_down(uint32_t* __restrict__ mask, int64_t ncells,
                                                     const uint64_t* __restrict__ bsum, uint32_t* __restrict__ begin,
-                                                    uint32_t* __restrict__ vid, const uint64_t* __restrict__ totals,
+                                                    uint32_t* __restrict__ tile_vid, const uint64_t* __restrict__ totals,
                                                     uint64_t* __restrict__ host_totals) {
     __shared__ uint64_t lw[256 / WAVE];
     if (blockIdx.x == 0 && threadIdx.x < 2) host_totals[threadIdx.x] = totals[threadIdx.x];
@@ -1202,13 +1204,16 @@ __global__ __launch_bounds__(256) void k_cells_down(const uint32_t* __restrict__
     for (int k = 0; k < CELL_ITEMS; k++) s += cell_sum(m[k]);
     block_exclusive_scan64(s, &run, lw);
     run += bsum[blockIdx.x];
+    const uint32_t own = (uint32_t)(run >> 32), before = __shfl_up(own, 1, WAVE);
+    const uint32_t first = threadIdx.x & 1 ? before : own;
+    if (!(threadIdx.x & 1) && base < ncells) tile_vid[base / 32] = first;
 #pragma unroll
     for (int k = 0; k < CELL_ITEMS; k += 4) {
         uint32_t at[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             at[j] = (uint32_t)run;
-            if ((m[k + j] >> 13) & 1u) vid[base + k + j] = (uint32_t)(run >> 32);
+            if ((m[k + j] >> 13) & 1u) mask[base + k + j] = m[k + j] | (((uint32_t)(run >> 32) - first) << 27);
             run += cell_sum(m[k + j]);
         }
         if (base + k < ncells) *(uint4*)(begin + base + k) = make_uint4(at[0], at[1], at[2], at[3]);
@@ -1225,7 +1230,7 @@ __global__ void k_cells_fill(const uint64_t* __restrict__ vkey, const uint32_t* 
                              const double* __restrict__ mean, const double* __restrict__ icov, int64_t nvox, Bits3 B,
                              int64_t o0, int64_t o1, int64_t o2, double res, int32_t tx, int32_t ty,
                              const uint32_t* __restrict__ mask, const uint32_t* __restrict__ begin,
-                             const uint32_t* __restrict__ vid, float4* __restrict__ head, float4* __restrict__ s32,
+                             const uint32_t* __restrict__ tile_vid, float4* __restrict__ head, float4* __restrict__ s32,
                              double2* __restrict__ vs64) {
     const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t v = i / 27;
@@ -1233,7 +1238,8 @@ __global__ void k_cells_fill(const uint64_t* __restrict__ vkey, const uint32_t* 
     const int o = (int)(i - 27 * v);
     int32_t c[3];
     cell_of_key(vkey[v], B, c);
-    const uint32_t id = vid[cell_index(c[0], c[1], c[2], tx, ty)];
+    const int32_t ci = cell_index(c[0], c[1], c[2], tx, ty);
+    const uint32_t id = tile_vid[ci >> 5] + (mask[ci] >> 27);
     const int32_t q0 = c[0] - (o % 3 - 1), q1 = c[1] - (o / 3 % 3 - 1), q2 = c[2] - (o / 9 - 1);
     const int32_t qi = cell_index(q0, q1, q2, tx, ty);
     const uint32_t at = begin[qi] + (uint32_t)__popc(mask[qi] & ((1u << o) - 1u));
@@ -1259,7 +1265,7 @@ size_t cells_scratch_bytes(int64_t ncells) {
 }
 
 int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox, const int* bits, const int32_t* tiles,
-                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* vid, void* scratch,
+                       int64_t ncells, uint32_t* mask, uint32_t* begin, uint32_t* tile_vid, void* scratch,
                        uint64_t* host_totals, hipStream_t stream) {
     Bits3 B;
     for (int k = 0; k < 3; k++) B.b[k] = bits[k];
@@ -1273,19 +1279,19 @@ int launch_cells_index(const uint64_t* vkey, const uint32_t* valid, int64_t nvox
                        tiles[1], mask);
     hipLaunchKernelGGL(k_cells_reduce, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, tot);
     hipLaunchKernelGGL(k_cells_top, dim3(1), dim3(1024), 0, stream, bsum, nb, tot);
-    hipLaunchKernelGGL(k_cells_down, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, begin, vid,
-                       tot, host_totals);
+    hipLaunchKernelGGL(k_cells_down, dim3((unsigned)nb), dim3(256), 0, stream, mask, ncells, bsum, begin,
+                       tile_vid, tot, host_totals);
     return (int)hipGetLastError();
 }
 
 int launch_cells_fill(const uint64_t* vkey, const uint32_t* valid, const double* mean, const double* icov, int64_t nvox,
                       const int* bits, const int64_t* origin_cell, double res, const int32_t* tiles, const uint32_t* mask,
-                      const uint32_t* begin, const uint32_t* vid, float4* head, float4* s32, double2* vs64,
+                      const uint32_t* begin, const uint32_t* tile_vid, float4* head, float4* s32, double2* vs64,
                       hipStream_t stream) {
     Bits3 B;
     for (int k = 0; k < 3; k++) B.b[k] = bits[k];
     hipLaunchKernelGGL(k_cells_fill, dim3(grid_for(27 * nvox, 256)), dim3(256), 0, stream, vkey, valid, mean, icov, nvox, B,
-                       origin_cell[0], origin_cell[1], origin_cell[2], res, tiles[0], tiles[1], mask, begin, vid, head,
+                       origin_cell[0], origin_cell[1], origin_cell[2], res, tiles[0], tiles[1], mask, begin, tile_vid, head,
                        s32, vs64);
     return (int)hipGetLastError();
 }

@@ -83,3 +83,42 @@ def test_upload_keeps_a_bounded_workspace(A, fresh, monkeypatch, counts):
     kept = _held(A, fresh, monkeypatch) - before - 16 * sum(counts)
     sc.close()
     assert kept <= 256 << 20
+
+
+def _sparse_map(dims, seed):
+    """A map of up to 1,500 voxels of 9 points in a box of `dims` cells, which counts a
+    margin of a cell around the map; its first and last cells are occupied."""
+    rng = np.random.default_rng(seed)
+    size = np.array(dims) - 2
+    cells = np.r_[[[0, 0, 0], size - 1], rng.integers(0, size, (1498, 3))]
+    pts = (np.unique(cells, axis=0)[:, None, :] + rng.uniform(0.1, 0.9, (1, 9, 3))).reshape(-1, 3)
+    return np.c_[pts, np.ones(len(pts))].astype(np.float32)
+
+
+@pytest.mark.parametrize("dims,room,dense", [((640, 640, 640), 8.25, True), ((640, 640, 640), 2.0, False),
+                                             ((5, 5, 1_000_000), 8.0, False)])
+def test_map_in_little_memory(A, fresh, monkeypatch, dims, room, dense):
+    """A map of a large, nearly empty box: its dense index is built in 8.25 bytes a cell (the
+    points' and voxels' arrays aside, less than 16 MB here), of which no more than 256 MB
+    remain once the grid is gone; where the device has no room for it, the map gets the
+    hashed index, and a pass has the same bits."""
+    box = int(np.prod(dims))
+    mp = _sparse_map(dims, 3)
+    prm = A.params(A.NDT_MODE_NDT)
+    before = _held(A, fresh, monkeypatch)
+    monkeypatch.setenv(LIMIT, str(int(before + room * box) + (16 << 20)))
+    tight = A.Grid(fresh, mp, prm)
+    monkeypatch.delenv(LIMIT)
+    assert tight.info()["dense_cells"] == (box if dense else 0)
+    roomy = A.Grid(fresh, mp, prm)
+    assert roomy.info()["dense_cells"] == box
+    for k in ("voxels", "valid_voxels", "query_cells", "candidates", "hash_capacity"):
+        assert tight.info()[k] == roomy.info()[k]
+    scan = mp[::2] + np.float32([0.05, -0.04, 0.03, 0])
+    p = np.array([0.03, -0.02, 0.01, 0.0, 0.0, 0.0])
+    x, y = tight.derivatives(scan, p), roomy.derivatives(scan, p)
+    assert x[3] == y[3] and x[3] > 0
+    assert x[0] == y[0] and np.array_equal(x[1], y[1]) and np.array_equal(x[2], y[2])
+    tight.close()
+    roomy.close()
+    assert _held(A, fresh, monkeypatch) - before <= (256 << 20) + (16 << 20)
