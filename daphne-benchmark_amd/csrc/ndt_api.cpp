@@ -664,7 +664,7 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
     BUF_TRY(vals_t, sizeof(uint32_t) * m);
     BUF_TRY(scratch, radix_sort_scratch_bytes(m));
     const int nbits = std::max(1, ceil_log2(ncells + 1));
-    LAUNCH_TRY(launch_keys_compat(c->pts.as<float4>(), m, d.minv, d.dims, res,
+    LAUNCH_TRY(launch_keys_compat(c->pts.as<float4>(), m, d.minv, d.dims, res, ncells,
                                   (radix_sort_from_tmp(nbits) ? keys_t : keys).as<uint64_t>(), c->stream));
     LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
                                 nbits, true, scratch.p, c->stream));

@@ -494,7 +494,7 @@ int launch_bbox(const float4* pts, int64_t n, uint32_t* minmax_bits /* 6 */, hip
 int launch_keys_ndt(const float4* pts, int64_t n, double resolution, const int64_t* origin_cell,
                     const int* bits, uint64_t* keys, hipStream_t stream);
 int launch_keys_compat(const float4* pts, int64_t n, const float* minv, const int* dims, float resolution,
-                       uint64_t* keys, hipStream_t stream);
+                       int64_t ncells, uint64_t* keys, hipStream_t stream);
 /* stable LSD radix sort of (key, value) pairs on the low `nbits` bits.  The pairs are in
  * (keys_tmp, vals_tmp) where radix_sort_from_tmp(nbits), otherwise in (keys, vals), and
  * end in (keys, vals); with iota the values are the keys' indices and not read.  The tmp

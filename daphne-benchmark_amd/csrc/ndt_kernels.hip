@@ -229,22 +229,25 @@ __device__ inline int compat_linearize(const float* minv, const int* dims, float
     return ix + dims[0] * (iy + dims[1] * iz);
 }
 
-__global__ void k_keys_compat(const float4* __restrict__ pts, int64_t n, CompatLayout L, uint64_t* __restrict__ keys) {
+/* ncells for all points outside the grid (a box of more than 2^24 cells on an axis may end a
+ * cell short, as its size is rounded to float): the sort takes no more bits than that */
+__global__ void k_keys_compat(const float4* __restrict__ pts, int64_t n, CompatLayout L, uint32_t ncells,
+                              uint64_t* __restrict__ keys) {
     int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (i >= n) return;
     float4 p = pts[i];
-    keys[i] = (uint64_t)(uint32_t)compat_linearize(L.minv, L.dims, L.res, p.x, p.y, p.z);
+    keys[i] = min((uint32_t)compat_linearize(L.minv, L.dims, L.res, p.x, p.y, p.z), ncells);
 }
 
 int launch_keys_compat(const float4* pts, int64_t n, const float* minv, const int* dims, float resolution,
-                       uint64_t* keys, hipStream_t stream) {
+                       int64_t ncells, uint64_t* keys, hipStream_t stream) {
     CompatLayout L;
     for (int k = 0; k < 3; k++) {
         L.minv[k] = minv[k];
         L.dims[k] = dims[k];
     }
     L.res = resolution;
-    hipLaunchKernelGGL(k_keys_compat, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, L, keys);
+    hipLaunchKernelGGL(k_keys_compat, dim3(grid_for(n, 256)), dim3(256), 0, stream, pts, n, L, (uint32_t)ncells, keys);
     return (int)hipGetLastError();
 }
 

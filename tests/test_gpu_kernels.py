@@ -173,3 +173,12 @@ def test_fitness_rows_match_hashed(A, orc, ctx, box, res):
         if limit:
             want, n = orc.fitness_score(mp, finite, poses[0], limit)
             assert na[0] == n and (n == 0 or abs(a[0] - want) <= 1e-12 * want)
+
+
+def test_compat_cells_beside_a_point_past_the_grid(A, ctx):
+    """The reference sizes a grid in float arithmetic, which leaves a box of 5 x 5 cells and
+    42,949,672 m one layer short of its highest point (the point's index is 2^30, whose low
+    30 bits are those of cell 0): cell 0 is one voxel of its three points all the same."""
+    pts = np.array([[0, 0, 0], [4, 4, 42949672], [0.3, 0.2, 0.1], [2, 2, 5], [0.1, 0.1, 0.1]], np.float32)
+    v = A.Grid(ctx, np.c_[pts, np.ones(5, np.float32)], A.params(A.NDT_MODE_COMPAT)).voxels()
+    assert v["key"][:, 0].tolist() == [0, 2 + 5 * (2 + 5 * 5)] and v["n"][0] == 3
