@@ -182,3 +182,50 @@ def test_compat_cells_beside_a_point_past_the_grid(A, ctx):
     pts = np.array([[0, 0, 0], [4, 4, 42949672], [0.3, 0.2, 0.1], [2, 2, 5], [0.1, 0.1, 0.1]], np.float32)
     v = A.Grid(ctx, np.c_[pts, np.ones(5, np.float32)], A.params(A.NDT_MODE_COMPAT)).voxels()
     assert v["key"][:, 0].tolist() == [0, 2 + 5 * (2 + 5 * 5)] and v["n"][0] == 3
+
+
+@pytest.mark.parametrize("n,extent,passes", [(5000, 1.0, 1), (5000, 60.0, 2), (70001, 2000.0, 3), (300001, 2000.0, 3),
+                                             (70001, 1e5, 4), (70001, 2e6, 5)])
+def test_map_sort_passes(A, ctx, n, extent, passes):
+    """Keys of one to five digits (up to 11 bits each), an odd and an even number of passes:
+    every voxel's cell and count as numpy has them."""
+    rng = np.random.default_rng(passes)
+    pts = rng.uniform(0, extent, (n, 3)).astype(np.float32)
+    pts[:, 2] = rng.uniform(-1, 1, n) * min(extent, 3.0)
+    cell = np.floor(pts.astype(np.float64)).astype(np.int64)
+    dims = cell.max(0) - cell.min(0) + 3  # a margin of a cell on each side
+    bits = sum(int(d - 1).bit_length() for d in dims)
+    assert -(-bits // 11) == passes
+    v = A.Grid(ctx, np.c_[pts, np.ones(n, np.float32)], A.params(A.NDT_MODE_NDT)).voxels()
+    keys, cnt = np.unique(cell[:, ::-1], axis=0, return_counts=True)
+    assert np.array_equal(v["key"], keys[:, ::-1]) and np.array_equal(v["n"], cnt)
+
+
+@pytest.mark.parametrize("box,rows", [((2, 2, 2), True), ((3, 3, 3), True), ((1, 1, 1), False)])
+def test_fitness_of_small_boxes(A, orc, ctx, box, rows):
+    """The smallest boxes that have runs of cells (at most 16 cells a voxel, a margin of one
+    around the map counted), and one that has the hash in both grids."""
+    mp = (np.stack(np.meshgrid(*[np.arange(b) for b in box], indexing="ij"), -1).reshape(-1, 3) + 0.5).astype(np.float32)
+    info = A.Grid(ctx, np.c_[mp, np.ones(len(mp), np.float32)], A.params(A.NDT_MODE_NDT)).info()
+    assert (info["dense_cells"] <= 16 * info["voxels"]) == rows
+    test_fitness_rows_match_hashed(A, orc, ctx, box, 1.0)
+
+
+def test_compat_map_refused_in_every_part_of_its_upload(A, ctx, compat_cases):
+    """A non-finite point of a 1 M point map in the first piece of the upload (131,072
+    points), in pieces behind copies still in flight, and behind the sixth, whose place in
+    the staging buffer is the first one's: refused, and the next callback gives the bits of
+    the one before."""
+    c = compat_cases[0]
+    first = ctx.compat_callback(c["scan"], c["guess"], c["map"])
+    big = np.ascontiguousarray(np.resize(c["map"], (1_000_000, 4)))
+    whole = ctx.compat_callback(c["scan"], c["guess"], big)
+    for at, v in ((5, np.nan), (131_072, np.inf), (700_000, np.nan), (786_431, -np.inf), (786_432, np.nan), (999_999, np.inf)):
+        bad = big.copy()
+        bad[at, at % 3] = v
+        with pytest.raises(A.NdtError) as e:
+            ctx.compat_callback(c["scan"], c["guess"], bad)
+        assert e.value.code == 1 and "finite" in str(e.value), at
+        again = ctx.compat_callback(c["scan"], c["guess"], c["map"])
+        assert np.array_equal(first["final_f32"], again["final_f32"]) and first["iterations"] == again["iterations"], at
+    assert np.array_equal(whole["final_f32"], ctx.compat_callback(c["scan"], c["guess"], big)["final_f32"])

@@ -436,3 +436,10 @@ def test_train_steps_the_input_layer_with_its_gradient(A, ctx, small_scene, dims
     m.train(A.Dataset(ctx, bm, sc, idx, guesses, gt), A.train_params(epochs=1, batch=B, lr=lr, cosine=0, seed=7))
     a, b = m3.grad(0).astype(np.float64), m.grad(0).astype(np.float64)
     assert np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("dims", [(384, 128, 128, 128), (640, 384, 640, 384)])
+def test_products_of_odd_k_steps(A, ctx, dims):
+    """Products whose split leaves an odd number of K steps of 64 (three and five in the
+    input layer's forward product), which end in the other one of the two buffers."""
+    test_forward_backward_adam_match_oracle(A, ctx, dims)
