@@ -841,17 +841,22 @@ int launch_transpose_u16(const uint16_t* src, int64_t rows, int64_t cols, uint16
  * K values inside one lane's 8.  K steps of 64 are staged through two LDS
  * buffers and two register sets: a step's global loads are issued two products
  * before it is stored, as one product (about 2 us with two workgroups on a CU) does
- * not cover the memory's latency under load.  Rows are padded by 8 elements (16
- * bytes).
+ * not cover the memory's latency under load.  The loop ends before its last steps, which
+ * follow it without loads: loading past the end instead (in bounds, unused) kept registers
+ * alive that spilled, and made two of a two-step product's five loads.  Rows are padded by
+ * 8 elements (16 bytes).
  *
  * Workgroups go round the 8 XCDs in launch order.  Where the splits are a multiple
  * of 8, an XCD takes all tiles of a split, so that its L2 fetches every operand once;
  * in launch order each XCD would hold one column of tiles and fetch all of A.  Fewer
- * splits (many tiles, or a short K) leave too few for that and keep the launch order.
+ * splits (many tiles, or a short K) leave too few for that and keep the launch order, and
+ * so do splits of less than four K steps (256 x 512 in 64 splits of two steps: 16.0 us by
+ * XCD, 14.0 in launch order; of four steps 15.3 and 19.5).
  *
  * 512 x 1024 x 65536 in 16 splits, bound by the latency of the operands' loads:
  * 131 us with loads one product ahead, 124 us two ahead, 118 us with the splits on
- * XCDs as well (580 TFLOP/s); the splits on XCDs alone gave 130 us. */
+ * XCDs as well, 104 us without the spill (660 TFLOP/s); the splits on XCDs alone gave
+ * 130 us. */
 constexpr int GPAD = 8;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -920,18 +925,31 @@ __device__ __forceinline__ void gemm_tile(GemmLds& L, const uint16_t* __restrict
     store(0, a0, b0);
     load(a0, b0, 2);
     __syncthreads();
-    for (int kt = 0;; kt += 2) {
+    int kt = 0;
+    for (; kt + 3 < nk; kt += 2) {
         multiply(0);
         store(1, a1, b1); /* step kt + 1: that buffer was last read before the last barrier */
         load(a1, b1, kt + 3);
         __syncthreads();
-        if (kt + 1 >= nk) break;
         multiply(1);
         store(0, a0, b0);
         load(a0, b0, kt + 4);
         __syncthreads();
-        if (kt + 2 >= nk) break;
     }
+    /* the last one to three steps, all of them loaded */
+    const int left = nk - kt;
+    multiply(0);
+    if (left > 1) {
+        store(1, a1, b1);
+        __syncthreads();
+        multiply(1);
+    }
+    if (left > 2) {
+        store(0, a0, b0);
+        __syncthreads();
+        multiply(0);
+    }
+    __syncthreads();
 }
 
 __global__ __launch_bounds__(256, 2) void k_gemm_nt(const uint16_t* __restrict__ A, int64_t lda,
@@ -941,7 +959,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_nt(const uint16_t* __restrict__
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int wm = w >> 1, wn = w & 1, fr = lane & 15;
     int bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;
-    if (gridDim.z % 8 == 0) {
+    if (gridDim.z % 8 == 0 && kps >= 4 * GEMM_BK) {
         const int tiles = gridDim.x * gridDim.y;
         const int id = bx + gridDim.x * by + tiles * bz;
         const int tile = (id >> 3) % tiles;
