@@ -319,8 +319,8 @@ static bool gather_points(float* dst, const float* const* arrays, const int64_t*
 }
 
 /* Work space of an upload's ordering, and of a dense index's build, that a context keeps for
- * the next one, each; more is given back (allocating and freeing 139 MB takes 0.25 ms, of a
- * 1.6 ms build of a map of 1 M points in a box of 34 M cells). */
+ * the next one, each (allocating and freeing 139 MB takes 0.25 ms, of a 1.6 ms build of a map
+ * of 1 M points in a box of 34 M cells; 187 MB 0.5 ms, of a 6 ms upload of 7.5 M points). */
 constexpr size_t WORK_KEEP = (size_t)256 << 20;
 
 /* Uploads of points go through the staging buffer in pieces, at most UPLOAD_RING of them
@@ -416,6 +416,11 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
         tiles[1] = (g->dims[1] + 3) / 4;
         ncells = 32ll * tiles[0] * tiles[1] * ((g->dims[2] + 1) / 2);
     }
+    /* the cells' masks and the tiles' voxel numbers, for the dense index's build: in the
+     * context, large ones in the grid's own memory (allocating and freeing them by themselves
+     * took 0.4 ms, now and then some tens of ms) */
+    const size_t mask_bytes = sizeof(uint32_t) * (size_t)(ncells + ncells / 32);
+    DevView mask;
     /* nearest-point queries: the first point of every cell of the box where that takes no
      * more than 64 bytes per occupied voxel, as much as their hash (32 to 64) at its emptiest */
     const bool rows = dense && box <= 16.0 * (double)nvox;
@@ -431,8 +436,13 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
         if (rows) l.add(g->fit_begin, sizeof(uint32_t) * ((size_t)box + 1));
         else l.add(g->fit_slots, sizeof(HashSlot) << flog2);
         if (dense) l.add(g->dense, sizeof(uint32_t) * (size_t)(ncells + 1));
+        if (mask_bytes > WORK_KEEP) l.add(mask, mask_bytes);
         e = l.place(g->voxel_mem);
         if (e) return e;
+    }
+    if (mask_bytes && !mask.p) {
+        BUF_TRY(c->bk_mask, mask_bytes);
+        mask.p = c->bk_mask.p;
     }
     /* map points sorted by voxel: for the statistics, and with a hash of the occupied
      * voxels for nearest-point queries (fitness score) */
@@ -464,10 +474,9 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
     g->info.voxels = nvox;
     int64_t nv = 0, ne = 0, nq = 0;
     if (dense) {
-        BUF_TRY(c->bk_mask, sizeof(uint32_t) * (size_t)(ncells + ncells / 32));
         BUF_TRY(scratch, cells_scratch_bytes(ncells));
         LAUNCH_TRY(launch_cells_index(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), nvox, g->bits, tiles, ncells,
-                                      c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_mask.as<uint32_t>() + ncells,
+                                      mask.as<uint32_t>(), g->dense.as<uint32_t>(), mask.as<uint32_t>() + ncells,
                                       scratch.p, (uint64_t*)c->hsmall, c->stream));
         HIP_TRY(hipStreamSynchronize(c->stream));
         const uint64_t* h = (const uint64_t*)c->hsmall;
@@ -528,7 +537,7 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
     if (dense) {
         LAUNCH_TRY(launch_cells_fill(g->all_key.as<uint64_t>(), g->all_valid.as<uint32_t>(), g->all_mean.as<double>(),
                                      g->all_icov.as<double>(), nvox, g->bits, g->origin_cell, res, tiles,
-                                     c->bk_mask.as<uint32_t>(), g->dense.as<uint32_t>(), c->bk_mask.as<uint32_t>() + ncells,
+                                     mask.as<uint32_t>(), g->dense.as<uint32_t>(), mask.as<uint32_t>() + ncells,
                                      g->cand_head.as<float4>(), g->cand_s32.as<float4>(), g->vs64.as<double2>(),
                                      c->stream));
     } else {
@@ -543,7 +552,6 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
         }
     }
     HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->bk_mask.bytes > WORK_KEEP) c->bk_mask.release();
     g->info.query_cells = nq;
     g->info.candidates = ne;
     g->info.hash_capacity = cap;
@@ -607,11 +615,10 @@ static int grid_build_ndt(ndt_ctx* c, const float* map, int64_t m, ndt_grid* g) 
     e = sorted_runs(c, keys.as<uint64_t>(), m, 0, limit, starts, sc2, &nvox, &nvalid_pts);
     if (e) return e;
     if (nvox == 0) return fail(NDT_ERR_INVALID, "map has no finite points");
-    /* dense query-cell index when the map's cell box is at most 2^28 cells: 4 bytes for
-     * each cell of the box, in whole tiles of 4 x 4 x 2, and 4.1 more while it is built
-     * (2.2 GB for a cube at the limit), or the hashed one where the device has no room for
-     * that; the environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed
-     * index, so that tests run that path on maps of every size */
+    /* dense query-cell index when the map's cell box is at most 2^28 cells, or the hashed one
+     * where the device has no room for it (8.1 bytes a cell, 2.2 GB for a cube at the limit);
+     * the environment variable NDT_FORCE_HASHED_INDEX=1 makes any map use the hashed index, so
+     * that tests run that path on maps of every size */
     const char* force_hash = std::getenv("NDT_FORCE_HASHED_INDEX");
     const bool dense = cells_of(g) <= (double)(1 << 28) && !(force_hash && std::strcmp(force_hash, "1") == 0);
     e = grid_index_ndt(c, m, nvox, nvalid_pts, dense, g);

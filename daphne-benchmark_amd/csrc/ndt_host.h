@@ -9,6 +9,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
+#include <cassert>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -88,17 +89,19 @@ struct DevBuf {
     template <class T> T* as() const { return (T*)p; }
 };
 
-/* Parts of a DevBuf: up to eight arrays in one allocation, at multiples of 256 bytes. */
+/* Parts of a DevBuf: up to MAX arrays in one allocation, at multiples of 256 bytes. */
 struct DevView {
     void* p = nullptr;
     template <class T> T* as() const { return (T*)p; }
 };
 struct DevLayout {
-    DevView* views[8];
-    size_t offsets[8];
+    static constexpr int MAX = 12;
+    DevView* views[MAX];
+    size_t offsets[MAX];
     int n = 0;
     size_t bytes = 0;
     void add(DevView& v, size_t want) {
+        assert(n < MAX);
         views[n] = &v;
         offsets[n++] = bytes;
         bytes += (want + 255) & ~(size_t)255;

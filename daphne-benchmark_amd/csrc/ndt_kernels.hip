@@ -1201,12 +1201,15 @@ __global__ __launch_bounds__(256) void k_cells_down(uint32_t* __restrict__ mask,
     if (blockIdx.x == 0 && threadIdx.x < 2) host_totals[threadIdx.x] = totals[threadIdx.x];
     uint32_t m[CELL_ITEMS];
     const int64_t base = blockIdx.x * (int64_t)CELL_TILE + threadIdx.x * CELL_ITEMS;
-    load_masks(mask, ncells, base, m);
+    /* a workgroup without candidates (most, in a large and nearly empty box) reads no masks */
+    const uint64_t from = bsum[blockIdx.x];
+    const uint64_t to = blockIdx.x + 1 < gridDim.x ? bsum[blockIdx.x + 1] : totals[0];
+    load_masks(mask, from == to ? 0 : ncells, base, m);
     uint64_t s = 0, run;
 #pragma unroll
     for (int k = 0; k < CELL_ITEMS; k++) s += cell_sum(m[k]);
     block_exclusive_scan64(s, &run, lw);
-    run += bsum[blockIdx.x];
+    run += from;
     const uint32_t own = (uint32_t)(run >> 32), before = __shfl_up(own, 1, WAVE);
     const uint32_t first = threadIdx.x & 1 ? before : own;
     if (!(threadIdx.x & 1) && base < ncells) tile_vid[base / 32] = first;

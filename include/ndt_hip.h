@@ -146,8 +146,8 @@ int ndt_ctx_device_info(ndt_ctx* ctx, int32_t* compute_units, char* name, int32_
  * map-local coordinates (params->origin gives their world offset in ndt mode).
  * An ndt grid indexes its query cells densely where the box of the map's cells has at most
  * 2^28 of them, in 4 bytes a cell (the box padded to whole tiles of 4 x 4 x 2 cells) and
- * another 4.1 during the build, of which the context keeps up to 256 MB; by a hash above
- * that, or where the device has no room for it. */
+ * another 4.1 for the build, which the context keeps up to 256 MB and the grid holds above
+ * that (62 M cells); by a hash above 2^28, or where the device has no room for it. */
 int ndt_grid_build(ndt_ctx* ctx, const float* map_xyzw, int64_t m, const ndt_params* params,
                    ndt_grid** out);
 int ndt_grid_info_get(const ndt_grid* grid, ndt_grid_info* info);
