@@ -995,7 +995,12 @@ static int align_packed(ndt_ctx* c, const ndt_grid* g, const float4* pts, const 
     return results_from_out(out, counts, S, aborted, c, results, used_alt);
 }
 
-/* The scans ordered on the host, for want of device memory to order them there. */
+/* Batches of up to this many points are ordered on the host: an upload of 1 point takes 17 us
+ * there and 26 us with a launch, of 300 points 21 and 27, of 768 points 26 and 29. */
+constexpr int64_t HOST_ORDER = 768;
+
+/* The scans ordered on the host: few points, and others where the device has no memory to
+ * order them in. */
 static int pack_scans_host(ndt_ctx* c, DevBuf& dst, const float* const* scans, const int64_t* counts, int32_t S,
                            const std::vector<int64_t>& offsets, int64_t t) {
     try {
@@ -1026,7 +1031,8 @@ static int pack_scans_host(ndt_ctx* c, DevBuf& dst, const float* const* scans, c
  * enqueued on the context's stream, and the callers' buffers are free when this returns.
  * Ordering takes 25 bytes a point of a group beside the 16 of the points' place (raw
  * points, a key and an index, tile counts): about 105 MB, and more only for a scan larger
- * than a group.  Where the device has no room for it, the points are ordered on the host. */
+ * than a group.  Where the device has no room for it, and where they are few, the points
+ * are ordered on the host. */
 static int pack_scans(ndt_ctx* c, DevBuf& dst, const float* const* scans, const int64_t* counts, int32_t S,
                       std::vector<int64_t>& offsets, int64_t* total) {
     struct Group {
@@ -1069,6 +1075,7 @@ static int pack_scans(ndt_ctx* c, DevBuf& dst, const float* const* scans, const 
     const size_t head_bytes = (seg_bytes + sizeof(OrderTile) * (size_t)ntiles + 255) & ~(size_t)255;
     BUF_TRY(dst, sizeof(float4) * t);
     *total = t;
+    if (t <= HOST_ORDER) return pack_scans_host(c, dst, scans, counts, S, offsets, t);
     int e = c->raw.ensure(head_bytes + sizeof(float4) * (size_t)most);
     if (!e && most_order) e = c->order.ensure((size_t)most_order);
     if (e == NDT_ERR_NOMEM) {

@@ -229,3 +229,9 @@ def test_compat_map_refused_in_every_part_of_its_upload(A, ctx, compat_cases):
         again = ctx.compat_callback(c["scan"], c["guess"], c["map"])
         assert np.array_equal(first["final_f32"], again["final_f32"]) and first["iterations"] == again["iterations"], at
     assert np.array_equal(whole["final_f32"], ctx.compat_callback(c["scan"], c["guess"], big)["final_f32"])
+
+
+@pytest.mark.parametrize("counts", [(767,), (768,), (769,), (384, 384), (1, 768), (1,) * 60])
+def test_scan_order_on_either_side(A, ctx, scene, counts):
+    """Batches of up to 768 points in all are ordered on the host, larger ones on the device."""
+    test_scan_order(A, ctx, scene, counts)
