@@ -218,17 +218,17 @@ static inline float ord2f(uint32_t u) {
     return f;
 }
 
-/* runs of equal keys in a sorted array: their starts and number, and the number of keys
- * below the limit */
+/* runs of equal keys in a sorted array: their starts and number, and (optional) the number
+ * of keys below the limit */
 static int sorted_runs(ndt_ctx* c, const uint64_t* keys, int64_t n, int shift, uint64_t limit, DevBuf& starts,
-                       DevBuf& scratch, int64_t* nruns, int64_t* below) {
+                       DevBuf& scratch, int64_t* nruns, int64_t* below = nullptr) {
     BUF_TRY(starts, sizeof(uint32_t) * (n + 1));
     BUF_TRY(scratch, runs_scratch_bytes(n));
     LAUNCH_TRY(launch_runs(keys, n, shift, limit, starts.as<uint32_t>(), scratch.as<uint32_t>(), (uint32_t*)c->hsmall,
                            c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     *nruns = ((const uint32_t*)c->hsmall)[0];
-    *below = ((const uint32_t*)c->hsmall)[1];
+    if (below) *below = ((const uint32_t*)c->hsmall)[1];
     return 0;
 }
 
@@ -517,8 +517,7 @@ static int grid_index_ndt(ndt_ctx* c, int64_t m, int64_t nvox, int64_t nvalid_pt
                                           (from_tmp ? vals_t : vals).as<uint32_t>(), c->stream));
             LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(),
                                         vals_t.as<uint32_t>(), ne, B + 5, false, scratch.p, c->stream));
-            int64_t all = 0;
-            e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, starts, sc2, &nq, &all);
+            e = sorted_runs(c, keys.as<uint64_t>(), ne, 5, ~0ull, starts, sc2, &nq);
             if (e) return e;
         }
     }
@@ -675,8 +674,8 @@ static int grid_build_compat(ndt_ctx* c, const float* map, int64_t m, ndt_grid* 
                                   (radix_sort_from_tmp(nbits) ? keys_t : keys).as<uint64_t>(), c->stream));
     LAUNCH_TRY(radix_sort_pairs(keys.as<uint64_t>(), vals.as<uint32_t>(), keys_t.as<uint64_t>(), vals_t.as<uint32_t>(), m,
                                 nbits, true, scratch.p, c->stream));
-    int64_t nvox = 0, inside = 0;
-    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, (uint64_t)ncells, starts, sc2, &nvox, &inside);
+    int64_t nvox = 0;
+    e = sorted_runs(c, keys.as<uint64_t>(), m, 0, (uint64_t)ncells, starts, sc2, &nvox);
     if (e) return e;
     const int log2cap = std::max(4, ceil_log2(2 * std::max<int64_t>(nvox, 1)));
     const int64_t cap = 1ll << log2cap;
@@ -1200,8 +1199,8 @@ extern "C" int ndt_scans_destroy(ndt_scans* sc) {
  * address looked up when the context was created), the chunk descriptors made on
  * the device from the batch's point counts, and the results converted on the device
  * and copied straight into the caller's array.  Calls on one device share the
- * array, so calls that overlap on a device race; every region a launch reads
- * before writing is cleared by fill kernels first. */
+ * array, so calls that overlap on a device race; the set-up kernel writes every region
+ * that the alignment reads before writing. */
 extern "C" int ndt_align_scans_noalloc(ndt_ctx* c, const ndt_grid* g, const ndt_scans* sc, const double* guesses,
                                        const ndt_params* p, ndt_result* results) {
     if (!c || !g || !sc || !guesses || !results) return fail(NDT_ERR_INVALID, "null argument");
